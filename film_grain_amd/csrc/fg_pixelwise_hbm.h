@@ -222,8 +222,8 @@ hipError_t launch_lambda_check(const float *lambda, long long n, int *status, hi
 // LDS bytes the splat kernel needs beyond its static arrays for one tile.
 size_t splat_hbm_lds(int tile_w, int tile_h, int n_samples, int qbuckets);
 // Static LDS of the splat kernels per workgroup of `block` threads: per wave a
-// candidate queue and 64 grain records.
-inline size_t splat_hbm_static_lds(int block) { return (size_t)block / 64 * (kQueueCap * 4 + 64 * 16) + 64; }
+// candidate queue, 64 grain records and the walk's list-end bits.
+inline size_t splat_hbm_static_lds(int block) { return (size_t)block / 64 * (kQueueCap * 4 + 64 * 16 + 64) + 64; }
 hipError_t launch_splat_hbm(const PixelArgs &a, const PixGeom &g, const SampleTable &t, const uint32_t *bin_start,
                             const float4 *grains, int block, hipStream_t s);
 
