@@ -509,13 +509,16 @@ bool plane_geometry(const fg_plane_desc *d, const float4 &r, fg::PixGeom *g)
 //           ulp(C_out)/2 <= C_out * 2^-24; the box and the fraction query take
 //           fewer than ten such steps, and eps = C_out * 2^-20 + 2^-16 covers
 //           them with room to spare.
-//   safe_r  a grain that passes the f32 disk test of a point lies within
-//           r (1 + 2^-23) + ulp(C_in) of it, and its centre lies in
-//           [i delta, (i + 1) delta) up to ulp(C_in); with rm - r above
-//           sixteen ulp(C_in) >= C_in * 2^-19, the points whose disk test it
-//           passes have windows (f32 floor((x -+ rm) / delta), rounding
-//           included) that contain its cell.  C_in bounds every coordinate
-//           in input pixels.
+//   safe_r  a point at most safe_r from a grain's centre in both axes (as the
+//           kernel's f32 dx and dy have it) has the grain's cell (i, j) in
+//           its window.  With h = C_in * 2^-24 (half an ulp of C_in, which
+//           bounds every coordinate in input pixels), the centre lies in
+//           [i delta - 2h, (i + 1) delta + 2h] (its two roundings), dx is the
+//           true difference but for h, and the window's f32 bounds
+//           floor((x -+ rm) / delta) take two roundings of at most h each: i
+//           is in the window when |dx| <= rm - 6h.  A grain of radius r that
+//           passes the f32 disk test has |dx| <= r (1 + 2^-23), 2h more at
+//           most; safe_r = rm - 12h leaves room for both.
 void splat_bounds(const fg::PixelArgs &a, const fg::PixGeom &g, const float4 &r, float *eps, float *safe_r)
 {
     const double maxo = std::max(std::max(std::fabs((double)r.x), std::fabs((double)r.y)),
@@ -526,7 +529,7 @@ void splat_bounds(const fg::PixelArgs &a, const fg::PixGeom &g, const float4 &r,
     const double c_in = std::max(cells * (double)a.delta, pix) + (double)a.rm + maxo + 4.0;
     const double c_out = (c_in + maxo + (double)a.rm) * (double)a.zoom + 8.0;
     *eps = (float)(c_out * std::ldexp(1.0, -20) + std::ldexp(1.0, -16));
-    const double lim = (double)a.rm - c_in * std::ldexp(1.0, -19);
+    const double lim = (double)a.rm - 1.5 * c_in * std::ldexp(1.0, -21);
     float sr = (float)lim;
     if ((double)sr > lim) sr = std::nextafter(sr, -INFINITY);
     *safe_r = sr > 0.0f ? sr : -1.0f;

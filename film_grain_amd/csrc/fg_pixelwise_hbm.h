@@ -37,8 +37,9 @@ struct SampleTable {
     int n;                 // samples in the table
     int qbuckets;          // power of two
     float eps;             // widening of the fraction interval (covers f32 rounding of the box)
-    float safe_r;          // a grain of radius <= safe_r that passes the disk test of a point
-                           // lies in that point's cell window
+    float safe_r;          // a point at most safe_r from a grain's centre in both axes (as any
+                           // that passes the disk test of a radius <= safe_r) has the grain's
+                           // cell in its window
     // the splat's candidate lists over this order (launch_splat_lists), or
     // nullptr: (start, length) per (radius class, cell), the entries (sorted
     // position * 16) of each list in order of the scaled y offset, and per

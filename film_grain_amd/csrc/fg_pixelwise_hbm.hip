@@ -18,8 +18,8 @@
 //               grain's centre fractions): the samples whose box can hold a
 //               pixel column and row (splat_lists_kernel)
 //   splat       per output tile, every wave streams 64-grain chunks of the
-//               tile's bins on its own.  The chunk's listed grains (narrow,
-//               no cell window to check) walk their lists concatenated, 64
+//               tile's bins on its own.  The chunk's listed grains (the
+//               narrow ones) walk their lists concatenated, 64
 //               entries a step whatever the grains they belong to; each lane
 //               tests the pixel nearest its sample's target with the exact
 //               reference test.  Every other grain walks, on its own, the one
@@ -1073,10 +1073,12 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
     t.X1 = min(t.X0 + a.tile_w, a.out_w);
     t.Y1 = min(t.Y0 + a.tile_h, a.out_h);
     t.TW = a.tile_w;
-    t.fx0 = (float)t.X0;
-    t.fx1 = (float)(t.X1 - 1);
-    t.fy0 = (float)t.Y0;
-    t.fy1 = (float)(t.Y1 - 1);
+    // per-tile floats are held in SGPRs (this target has no scalar float ALU:
+    // left to the compiler they stay in VGPRs, and the walk spilled)
+    t.fx0 = uniform_f((float)t.X0);
+    t.fx1 = uniform_f((float)(t.X1 - 1));
+    t.fy0 = uniform_f((float)t.Y0);
+    t.fy1 = uniform_f((float)(t.Y1 - 1));
     t.I0 = geo.Ix0;  // grain cells are packed relative to the extended grid
     t.J0 = geo.Jy0;
     const float rm = a.rm, delta = a.delta, rd = a.rdelta, iz = a.inv_zoom, z = a.zoom;
@@ -1148,19 +1150,22 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
         const float4 r = srec[p];
         return make_uint2(__float_as_uint(r.z), __float_as_uint(r.w));
     };
-    const float4 ext = *st.ext;
-    const RowBuckets rbk = row_buckets(ext);
+    const float4 ext0 = *st.ext;
+    const float4 ext = make_float4(uniform_f(ext0.x), uniform_f(ext0.y), uniform_f(ext0.z), uniform_f(ext0.w));
+    RowBuckets rbk = row_buckets(ext0);
+    rbk.inv_w = uniform_f(rbk.inv_w);
+    rbk.y0 = ext.z;
     // the tile's 64-grain chunks go to its waves on demand (the first NW
     // statically), so that a wave that drew sparse chunks takes more
     __shared__ int s_next_chunk;
     if (tid == 0) s_next_chunk = NW;
     __syncthreads();
 
-    const float slack = 4e-3f + 2e-6f * (float)max(a.out_w, a.out_h);
-    const float eps = st.eps, safe_r = st.safe_r, Qf = (float)Q;
+    const float slack = uniform_f(4e-3f + 2e-6f * (float)max(a.out_w, a.out_h));
+    const float eps = st.eps, safe_r = st.safe_r, Qf = uniform_f((float)Q);
     // A pixel's point is (x + 0.5) * iz - O.  For integral x, x + 0.5 is exact,
     // so fma(x, iz, iz / 2) rounds the same exact product once: the same f32.
-    const float hiz = 0.5f * iz;
+    const float hiz = uniform_f(0.5f * iz);
     uint32_t *queue = s_queue[wid];
     int qcount = 0;
 
@@ -1169,6 +1174,33 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
     // and packed cell.
     float gcx = 0.0f, gcy = 0.0f, gr = 0.0f;
     uint32_t gcell = 0;
+
+    // The reference's window test: the grain's cell is one the point (xg, yg)
+    // visits (src/pixelwise.rs:56-60).
+    auto in_window = [&](uint32_t cell, float xg, float yg) {
+        const int gi = t.I0 + (int)(cell & 0xFFFFu), gj = t.J0 + (int)(cell >> 16);
+        return floor_div(xg - rm, delta, rd, fast) <= gi && gi <= floor_div(xg + rm, delta, rd, fast) &&
+               floor_div(yg - rm, delta, rd, fast) <= gj && gj <= floor_div(yg + rm, delta, rd, fast);
+    };
+
+    // The same test where every quotient takes floor_div's reciprocal
+    // sequence: floor(q) <= i is q < i + 1, floor(q) >= i is q >= i.  The
+    // sequence needs |xg -+ rm| in [2^-60, 2^60] or zero: a difference of two
+    // f32 values near rm is a multiple of rm * 2^-25, and none exceeds the
+    // grid's extent, hence the bounds on rm, delta and the grid; and i, i + 1
+    // exact in f32.  (Inlined in each step of the walk, the
+    // general form's divisions spilled.)
+    const bool win_fast = fast && rm >= 9.313225746154785e-10f && rm <= 1073741824.0f && delta <= 1073741824.0f &&
+                          abs(t.I0) < (1 << 22) && abs(t.J0) < (1 << 22);
+    auto in_window_fast = [&](uint32_t cell, float xg, float yg) {
+        const float gi = (float)(t.I0 + (int)(cell & 0xFFFFu)), gj = (float)(t.J0 + (int)(cell >> 16));
+        auto quot = [&](float v) {
+            const float q0 = v * rd;
+            return __builtin_fmaf(__builtin_fmaf(-q0, delta, v), rd, q0);
+        };
+        const bool in_x = quot(xg - rm) < gi + 1.0f && quot(xg + rm) >= gi;
+        return in_x && quot(yg - rm) < gj + 1.0f && quot(yg + rm) >= gj;
+    };
 
     // A queue entry is one (grain, sample, pixel) test: grain lane (6 bits) |
     // sorted sample position << 6 (11 bits) | tile column << 17 (7 bits) |
@@ -1192,10 +1224,7 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
         const float dx = xg - cx, dy = yg - cy;
         const float r = fabsf(rs);
         if (dx * dx + dy * dy <= r * r) {
-            const int gi = t.I0 + (int)(cell & 0xFFFFu), gj = t.J0 + (int)(cell >> 16);
-            if (rs > 0.0f ||
-                (floor_div(xg - rm, delta, rd, fast) <= gi && gi <= floor_div(xg + rm, delta, rd, fast) &&
-                 floor_div(yg - rm, delta, rd, fast) <= gj && gj <= floor_div(yg + rm, delta, rd, fast)))
+            if (rs > 0.0f || in_window(cell, xg, yg))
                 lds_or(mad_u24((uint32_t)ty, row_b, mad_u24((uint32_t)tx, w4, wm.x)), wm.y);
         }
     };
@@ -1226,14 +1255,16 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
     // the output's larger side), so the nearest pixel is the same whenever
     // one can pass.  The grain's values may differ between lanes.
     const int tw = t.X1 - t.X0, th = t.Y1 - t.Y0;
-    auto test = [&](bool ok, float4 r, float gcx_, float gcy_, float rs2) {
+    // win(dx, dy, xg, yg): the grain's cell lies in the passing point's
+    // window.
+    auto test = [&](bool ok, float4 r, float gcx_, float gcy_, float rs2, auto win) {
         const float px = rintf(__builtin_fmaf(r.x + gcx_, z, -0.5f)), py = rintf(__builtin_fmaf(r.y + gcy_, z, -0.5f));
         const int tx = (int)px - t.X0, ty = (int)py - t.Y0;
         if (ok & ((unsigned)tx < (unsigned)tw) & ((unsigned)ty < (unsigned)th)) {
             const float xg = __builtin_fmaf(px, iz, hiz) - r.x;
             const float yg = __builtin_fmaf(py, iz, hiz) - r.y;
             const float dx = xg - gcx_, dy = yg - gcy_;
-            if (dx * dx + dy * dy <= rs2)
+            if (dx * dx + dy * dy <= rs2 && win(dx, dy, xg, yg))
                 // tile coordinates and the bitset's bytes are far below 2^24:
                 // two 24-bit multiply-adds (full rate; the compiler otherwise
                 // forms the pixel index with a quarter-rate 64-bit mad)
@@ -1306,10 +1337,19 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
                 len = end - p0;
             }
         }
-        // a narrow grain that takes the direct test and has a radius class:
-        // its cell's candidate list replaces the run
+        // a narrow grain that has a radius class: its cell's candidate list
+        // replaces the run.  A radius above safe_r (a constant radius is the
+        // clamp radius itself, so all of them; under a lognormal law one in a
+        // thousand) needs its passing points' windows checked, which the walk
+        // does in a second form; a single such grain goes without the list.
+        // (Grains above safe_r used to queue every candidate of their x run:
+        // the splat of a 1080p constant-radius plane at N = 32 takes 0.80 ms
+        // with the lists and took 6.0 without, a 256x256 one 129 and 573 us.)
         bool listed = false;
-        if (LISTS && keep && st.cl_cell && rad <= safe_r && rz + rz < 1.0f) {
+        const bool in_class = LISTS && keep && st.cl_cell && rz + rz < 1.0f;
+        const unsigned long long unsafe_m = LISTS ? __ballot(in_class && rad > safe_r) : 0ull;
+        const bool check = win_fast && (unsafe_m & (unsafe_m - 1ull)) != 0ull;  // two or more
+        if (in_class && (check || rad <= safe_r)) {
             const int k = (int)(rz * a.cl_inv_dz);
             if (k < a.cl_classes) {
                 const float ncx = -bx, ncy = -by;
@@ -1336,7 +1376,7 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
         gcy = G.y;
         gr = rad <= safe_r ? rad : -rad;
         gcell = pk;
-        // the listed grains (all narrow, all with rs > 0) take the
+        // the listed grains (all narrow) take the
         // concatenated walk below; the others the per-grain walk after it
         unsigned long long m = __ballot(keep && !listed);
         const bool walks = listed && len > 0;
@@ -1368,7 +1408,10 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
             // (the wave's LDS accesses run in order, so no barrier is needed)
             const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(lmask >> 32),
                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)lmask, 0u));
-            if (walks) s_grec[wid][rank] = make_float4(G.x, G.y, rad * rad, __int_as_float(p0 - excl + bias));
+            if (walks) {
+                s_grec[wid][rank] = make_float4(G.x, G.y, rad * rad, __int_as_float(p0 - excl + bias));
+                queue[rank] = pk;  // the cells, for the window checks (the queue is empty here)
+            }
             const unsigned char *grec = reinterpret_cast<const unsigned char *>(&s_grec[wid][0]);
             uint32_t *ends = s_ends[wid];
             // the last list's end is left out: lanes past the stream count as
@@ -1383,8 +1426,9 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
             // base in SGPRs (the batch's first entry, less the bias), a
             // 32-bit byte offset in one VGPR and the step's 128 bytes as its
             // immediate offset: no 64-bit address arithmetic.
-            auto batch = [&](auto stage, int sb) {
+            auto batch = [&](auto stage, auto checked, int sb) {
                 constexpr int STAGE = decltype(stage)::value;
+                constexpr bool CHECK = decltype(checked)::value;
                 if (lane < 2 * STAGE) ends[lane] = 0u;
                 __builtin_amdgcn_wave_barrier();
                 const int rel = my_end - sb;
@@ -1415,17 +1459,29 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
                     // both reads issue before the test's branches (as in the
                     // per-grain walk)
                     asm volatile("" ::"v"(r.x), "v"(r.y), "v"(r.z), "v"(r.w));
-                    test(true, r, gr.x, gr.y, gr.z);
+                    // A passing point at most safe_r from the centre in both
+                    // axes has the grain's cell in its window (splat_bounds);
+                    // beyond, the reference's window test decides.
+                    test(true, r, gr.x, gr.y, gr.z, [&](float dx, float dy, float xg, float yg) -> bool {
+                        if (!CHECK || fmaxf(fabsf(dx), fabsf(dy)) <= safe_r) return true;
+                        return in_window_fast(queue[own[i] >> 4], xg, yg);
+                    });
                 }
                 __builtin_amdgcn_wave_barrier();
             };
             // whole batches, then a shorter one where it holds the rest: the
             // lists of a small N are a few entries each
-            int sb = 0;
-            for (; total - sb > 64 * (kWalkStage / 2); sb += 64 * kWalkStage)
-                batch(std::integral_constant<int, kWalkStage>(), sb);
-            if (total - sb > 64 * (kWalkStage / 4)) batch(std::integral_constant<int, kWalkStage / 2>(), sb);
-            else if (total - sb > 0) batch(std::integral_constant<int, kWalkStage / 4>(), sb);
+            auto walk = [&](auto checked) {
+                int sb = 0;
+                for (; total - sb > 64 * (kWalkStage / 2); sb += 64 * kWalkStage)
+                    batch(std::integral_constant<int, kWalkStage>(), checked, sb);
+                if (total - sb > 64 * (kWalkStage / 4))
+                    batch(std::integral_constant<int, kWalkStage / 2>(), checked, sb);
+                else if (total - sb > 0)
+                    batch(std::integral_constant<int, kWalkStage / 4>(), checked, sb);
+            };
+            if (check) walk(std::true_type());
+            else walk(std::false_type());
         }
         while (m) {
             const int l = __ffsll((long long)m) - 1;
@@ -1481,6 +1537,7 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
             // issued before either is tested
             if (direct) {
                 const float ucx = lane_f(gcx, l), ucy = lane_f(gcy, l), urs2 = urs * urs;
+                auto no_check = [](float, float, float, float) { return true; };
                 for (int i0 = 0; i0 < ulen; i0 += 128) {
                     const int ia = i0 + lane, ib = ia + 64;
                     const int pa = position(up0 + ia), pb = position(up0 + ib);
@@ -1491,8 +1548,8 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
                     // branches after the dependent ones)
                     asm volatile("" ::"v"(ra.x), "v"(ra.y), "v"(ra.z), "v"(ra.w), "v"(rb.x), "v"(rb.y),
                                  "v"(rb.z), "v"(rb.w));
-                    test(ia < ulen, ra, ucx, ucy, urs2);
-                    if (i0 + 64 < ulen) test(ib < ulen, rb, ucx, ucy, urs2);
+                    test(ia < ulen, ra, ucx, ucy, urs2, no_check);
+                    if (i0 + 64 < ulen) test(ib < ulen, rb, ucx, ucy, urs2, no_check);
                 }
                 continue;
             }

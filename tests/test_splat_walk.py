@@ -97,3 +97,57 @@ def test_target_from_the_centre_finds_every_passing_pixel(z, out_side):
                 assert not np.any(inside & ((px != near[:, 0]) | (py != near[:, 1]))), (z, i)
                 hits += int(inside.sum())
     assert hits > 0
+
+
+@pytest.mark.parametrize("side,rm,delta", [(64, 0.1, 0.1), (4096, 0.05, 0.05), (4096, 0.3, 0.11), (1500, 0.012, 0.4),
+                                           (16000, 0.1, 0.1)])
+def test_points_within_safe_r_have_the_cell_in_their_window(side, rm, delta):
+    """A point whose f32 dx is at most safe_r = rm - 12 C 2^-24 has the
+    grain's cell in its f32 window, for centres drawn in their cell (at its
+    edges too) and dx up to safe_r; and q < i + 1, q >= i on the quotient is
+    the window test floor(q) <= i, floor(q) >= i."""
+    rng = np.random.default_rng(side + int(rm * 1e3))
+    M = 400_000
+    rm, delta = f32(rm), f32(delta)
+    C = side + float(rm) + 4.0 + 4.0
+    lim = float(rm) - 1.5 * C * 2.0 ** -21
+    safe_r = f32(lim)
+    if float(safe_r) > lim:
+        safe_r = np.nextafter(safe_r, f32(-np.inf))
+    if not safe_r > 0:
+        safe_r = f32(-1)
+    i = rng.integers(-int(3 / delta), int(side / delta), M)
+    u = rng.uniform(0, 1, M).astype(f32) * delta
+    edge = rng.integers(0, 3, M)
+    u = np.where(edge == 0, f32(0), np.where(edge == 1, np.nextafter(delta, f32(0)), u)).astype(f32)
+    cx = ((i.astype(f32) * delta).astype(f32) + u).astype(f32)
+    d = np.where(rng.random(M) < 0.7, safe_r, rng.uniform(-1, 1, M) * rm).astype(f32) * rng.choice([-1, 1], M)
+    xg = (cx + d.astype(f32)).astype(f32)
+    xg = np.nextafter(xg, (xg + rng.choice([-1, 0, 1], M)).astype(f32)).astype(f32)
+    dx = (xg - cx).astype(f32)
+    q_lo, q_hi = (xg - rm).astype(f32) / delta, (xg + rm).astype(f32) / delta
+    assert q_lo.dtype == f32
+    inside = (np.floor(q_lo) <= i) & (i <= np.floor(q_hi))
+    near = np.abs(dx) <= safe_r
+    assert not np.any(near & ~inside)
+    assert near.sum() > 0 or safe_r < 0
+    fi = i.astype(f32)
+    assert np.array_equal(inside, (q_lo < fi + f32(1)) & (q_hi >= fi))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,h,r,zoom,n,cell", [(64, 48, 0.1, 1.0, 32, None), (3001, 5, 0.08, 1.0, 40, None),
+                                               (5, 2500, 0.03, 1.0, 16, 0.2), (90, 37, 0.12, 2.0, 256, 0.05),
+                                               (41, 33, 0.24, 2.0, 100, None), (33, 40, 0.2, 0.5, 513, 0.31)])
+def test_constant_radius_planes_equal_the_oracle(hip_ctx, oracle, w, h, r, zoom, n, cell):
+    """A constant radius is the clamp radius itself: its grains walk the lists
+    with the window test on points near the clamp distance.  Thin long planes
+    take the coordinates (and with them the share of such points) up."""
+    from film_grain_amd import synth
+    from tests import fgcases
+    u = synth.sinusoid_field(w, h, w + h, n_waves=3)
+    case = fgcases.build_case(oracle, f"const_{w}x{h}", u, r, 0.0, "const", zoom=zoom, n_samples=n, seed=w * h + n,
+                              cell_delta=cell)
+    want = oracle.render_pixelwise(case.plane, case.lam, case.offsets_input)
+    got = hip_ctx.render_host("pixel", case.desc, case.lam, case.offsets_input)
+    assert int(np.sum(got != want)) == 0
