@@ -1608,6 +1608,7 @@ int batch_gen_setup(fg_batch *b, const char *what, hipStream_t s)
     }
     g.thr_blocks = thr[n];
     g.total_bins = bins[n];
+    g.draw_chunk = fg::draw_chunk(g.total_bins);
     g.list_blocks = lists[n];
     g.sort_blocks = (max_samples + fg::kBlock - 1) / fg::kBlock;
     if (g.thr_blocks > 0x7fffffffLL || g.list_blocks > 0x7fffffffLL) return set_error(b->ctx, FG_EINVAL, "batch too large");
@@ -1619,7 +1620,7 @@ int batch_gen_setup(fg_batch *b, const char *what, hipStream_t s)
     for (int p = 0; p < n; ++p) {
         const int k = b->kind[p] == 0 ? 0 : 1;
         kp[k].push_back(p);
-        ko[k].push_back(ko[k].back() + (bins[p + 1] - bins[p] + fg::kDrawChunk - 1) / fg::kDrawChunk);
+        ko[k].push_back(ko[k].back() + (bins[p + 1] - bins[p] + g.draw_chunk - 1) / g.draw_chunk);
     }
     put(thr.data(), thr.size() * 8, reinterpret_cast<const void **>(&g.thr_off));
     put(bins.data(), bins.size() * 8, reinterpret_cast<const void **>(&g.bin_off));

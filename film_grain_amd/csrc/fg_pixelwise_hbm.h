@@ -8,11 +8,15 @@
 namespace fg {
 
 constexpr int kBinSide = 16;  // a bin is 16 x 16 cells (one wave; a lane holds four cells)
-// The draw pass (bin_grains) gives each wave kDrawChunk consecutive bins of
-// a plane: the wave's set-up (its arguments, and in a batch the search for
-// its plane) is spread over the chunk's bins (on a batch of 64 uneven
-// images, 4 or 16 bins a wave are 0.3% and 0.5% slower than 8).
+// The draw pass (bin_grains) gives each wave at most kDrawChunk consecutive
+// bins of a plane: the wave's set-up (its arguments, and in a batch the search
+// for its plane) is spread over the chunk's bins, and the bins are drawn in
+// groups (10, 15 and 16 bins a wave: the 4K RGB frame 0%, 1% and 1% slower, a
+// 12-image batch 1%, 2% and 2%).  A small plane takes fewer bins a wave, so
+// that its waves fill the chip (draw_chunk; a 96x64 plane's 651 bins in
+// chunks of 8 left most SIMDs idle: 55 us, one bin a wave 13 us).
 constexpr int kDrawChunk = 8;
+int draw_chunk(long long bins);
 
 // The plane's extended cell grid: every cell some point's window can reach.
 struct PixGeom {
@@ -142,7 +146,7 @@ struct BatchPlane {
 // The generation of a batch's planes: the thresholds, the draws and the
 // sample tables each one launch over all planes, in which a workgroup (or
 // wave) finds its plane by a binary search over first-block offsets (one
-// entry more than the planes).  In the draw pass a wave takes kDrawChunk
+// entry more than the planes).  In the draw pass a wave takes draw_chunk
 // consecutive bins of one plane (the offsets count chunks).  Every pointer
 // is device memory.
 struct BatchGen {
@@ -159,6 +163,7 @@ struct BatchGen {
     const long long *kind_off[2];
     int n_kind[2];
     long long kind_chunks[2];     // chunks of the planes of each distribution
+    int draw_chunk;               // bins a chunk
     uint32_t *cnt;
     unsigned long long *mask;
     float4 *grains;

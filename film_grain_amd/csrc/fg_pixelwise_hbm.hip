@@ -131,12 +131,8 @@ __device__ __forceinline__ int compact_cells(const unsigned long long m[4], uint
     return n;
 }
 
-// A bin's per-cell LDS records, one 32-byte record per cell in two uint4
-// halves: after the empty-cell test, at the cell's slot q << 6 | l, the hash,
-// two seed words and the threshold of each nonempty cell; after the counts,
-// at the cell's compacted index (never above its slot, so the rewrite in
-// place reads every record before it is overwritten), its stream after the
-// count draws.
+// A group of bins' streams after the count draws, one 32-byte record per
+// nonempty cell in two uint4 halves.
 typedef uint4 BinRecs[2][256];
 
 __device__ __forceinline__ void put_u64x2(uint4 &r, uint64_t x, uint64_t y)
@@ -147,20 +143,20 @@ __device__ __forceinline__ uint64_t lo64(const uint4 &r) { return (uint64_t)r.x 
 __device__ __forceinline__ uint64_t hi64(const uint4 &r) { return (uint64_t)r.z | (uint64_t)r.w << 32; }
 
 
-// The grain draws of the bin's n compacted cells, whose streams are in rec
-// and whose counts' exclusive prefix is in pre (total: the bin's sum): cell
-// idx's grains go to grains[out0 + pre[idx] ...].  A lane takes the bin's
-// next cell whenever its own has no grain left, so the lanes stay busy
-// although counts differ.
+// The grain draws of a group of bins' n nonempty cells, whose coordinates are
+// in list (ci | cj << 16), streams in rec and counts' exclusive prefix in pre
+// (total: the group's sum): cell idx's grains go to grains[out0 + pre[idx]
+// ...].  A lane takes the group's next cell whenever its own has no grain
+// left, so the lanes stay busy although counts differ.
 template <int KIND>
-__device__ __forceinline__ void bin_draws(const PixelArgs &a, const PixGeom &g, int ci0, int cj0,
-                                          const uint16_t *list, int n, const BinRecs &rec, const uint32_t *pre,
-                                          uint32_t total, uint32_t out0, float4 *grains)
+__device__ __forceinline__ void bin_draws(const PixelArgs &a, const PixGeom &g, const uint32_t *list, int n,
+                                          const BinRecs &rec, const uint32_t *pre, uint32_t total, uint32_t out0,
+                                          float4 *grains)
 {
     Xoshiro rng{};
     uint32_t k = 0, kend = 0, dst = 0;
     float sx = 0.0f, sy = 0.0f, pkf = 0.0f;
-    int next = 0;  // uniform: the bin's next cell no lane has taken
+    int next = 0;  // uniform: the group's next cell no lane has taken
     for (;;) {
         while (next < n) {
             const bool need = k >= kend;
@@ -170,9 +166,7 @@ __device__ __forceinline__ void bin_draws(const PixelArgs &a, const PixGeom &g, 
                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0u));
             const int idx = next + rank;
             if (need && idx < n) {
-                const int cell = list[idx];
-                const int l = cell & 63, q = cell >> 6;
-                const int ci = ci0 + (l & 15), cj = cj0 + 4 * (l >> 4) + q;
+                const uint32_t pk = list[idx];
                 const uint32_t p0 = pre[idx];
                 const uint32_t p1 = idx + 1 < n ? pre[idx + 1] : total;
                 const uint4 r0 = rec[0][idx], r1 = rec[1][idx];
@@ -183,9 +177,9 @@ __device__ __forceinline__ void bin_draws(const PixelArgs &a, const PixGeom &g, 
                 k = 0;
                 kend = p1 - p0;
                 dst = out0 + p0;
-                sx = (float)(g.Ix0 + ci) * a.delta;
-                sy = (float)(g.Jy0 + cj) * a.delta;
-                pkf = __uint_as_float((uint32_t)ci | ((uint32_t)cj << 16));
+                sx = (float)(g.Ix0 + (int)(pk & 0xFFFFu)) * a.delta;
+                sy = (float)(g.Jy0 + (int)(pk >> 16)) * a.delta;
+                pkf = __uint_as_float(pk);
             }
             next = min(next + __popcll(mk), n);
         }
@@ -384,58 +378,93 @@ bin_count_planes_kernel(PixelArgs a, PixGeom g, FramePlanes fp)
     }
 }
 
-// Pass 2: per bin (one wave), the nonempty cells from the mask, their counts
-// (seeded in full) and their grains at bin_start[bin].
+// Pass 2: a wave's consecutive bins [b0, b1) (at most kDrawChunk), in groups
+// of as many consecutive bins as have at most 256 nonempty cells together
+// (one bin always does).  A group's nonempty cells are listed from the masks,
+// counted 64 at a time (seeded in full), and their grains drawn to
+// grains[bin_start[first bin] ...], the bins' ranges being consecutive.
+// Bounded by instruction issue.  Bin by bin, 50 nonempty cells (the 4K RGB
+// frame at N = 256) filled 50 of 64 lanes in the count and the first draw
+// round and left two or three rounds of a few lanes: 1.29 ms a plane; in
+// groups 0.96 ms (constant radius, 1080p at N = 32: 1.01 and 0.76 ms).
 template <int KIND>
-__device__ __forceinline__ void bin_grains_body(const PixelArgs &a, const PixGeom &g, const double *T,
-                                                const uint32_t *bin_start, const unsigned long long *bin_mask,
-                                                float4 *grains, int bin, uint16_t *list, uint32_t *pre, BinRecs &rec)
+__device__ __forceinline__ void draw_bins(const PixelArgs &a, const PixGeom &g, const double *T,
+                                          const uint32_t *bin_start, const unsigned long long *bin_mask,
+                                          float4 *grains, int b0, int b1, uint32_t *list, uint32_t *pre, BinRecs &rec)
 {
+    static_assert(kDrawChunk <= 16, "one lane holds one mask word of the chunk");
     const int lane = threadIdx.x & 63;
-    unsigned long long m[4];
+    // lane l: mask word l & 3 of bin b0 + (l >> 2), and the bin's cells
+    unsigned long long mw = 0ull;
+    if (b0 + (lane >> 2) < b1) mw = bin_mask[(size_t)b0 * 4 + lane];
+    int cells = __popcll(mw);
+    cells += __shfl_xor(cells, 1, 64);
+    cells += __shfl_xor(cells, 2, 64);
+    int bx = b0 % g.nbx, by = b0 / g.nbx;  // uniform: the next bin's column and row
+    for (int bin = b0; bin < b1;) {
+        const int first = bin;
+        int n = 0;
+        do {
+            const int l0 = (bin - b0) * 4;
+            const int nb = __builtin_amdgcn_readlane(cells, l0);
+            if (bin > first && n + nb > 256) break;
+            const uint32_t ci = (uint32_t)(bx * kBinSide + (lane & 15)), cj = (uint32_t)(by * kBinSide + 4 * (lane >> 4));
 #pragma unroll
-    for (int q = 0; q < 4; ++q) m[q] = bin_mask[(size_t)bin * 4 + q];
-    const int n = compact_cells(m, list);
-    int ci0, cj0;
-    bin_origin(g, bin, ci0, cj0);
-    // counts from full seeds
-    uint32_t carry = 0;
-    for (int base = 0; base < n; base += 64) {
-        uint32_t c = 0;
-        const int idx = base + lane;
-        if (idx < n) {
-            const int cell = list[idx];
-            const int l = cell & 63, q = cell >> 6;
-            const int i = g.Ix0 + ci0 + (l & 15), j = g.Jy0 + cj0 + 4 * (l >> 4) + q;
-            float sx, sy;
-            const double e = cell_threshold_at(a, T, i, j, sx, sy);
-            Xoshiro rng{};
-            c = cell_count_full(mix3(a.seed, kCellStream, i, j), e, rng);
-            put_u64x2(rec[0][idx], rng.s0, rng.s1);
-            put_u64x2(rec[1][idx], rng.s2, rng.s3);
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mw, l0 + q);
+                const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mw >> 32), l0 + q);
+                const int before = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+                const unsigned long long m = (unsigned long long)hi << 32 | lo;
+                if ((m >> lane) & 1ull) list[n + before] = ci | (cj + q) << 16;
+                n += __popcll(m);
+            }
+            ++bin;
+            if (++bx == g.nbx) {
+                bx = 0;
+                ++by;
+            }
+        } while (bin < b1);
+        if (n == 0) continue;
+        // counts from full seeds
+        uint32_t carry = 0;
+        for (int base = 0; base < n; base += 64) {
+            uint32_t c = 0;
+            const int idx = base + lane;
+            if (idx < n) {
+                const uint32_t pk = list[idx];
+                const int i = g.Ix0 + (int)(pk & 0xFFFFu), j = g.Jy0 + (int)(pk >> 16);
+                float sx, sy;
+                const double e = cell_threshold_at(a, T, i, j, sx, sy);
+                Xoshiro rng{};
+                c = cell_count_full(mix3(a.seed, kCellStream, i, j), e, rng);
+                put_u64x2(rec[0][idx], rng.s0, rng.s1);
+                put_u64x2(rec[1][idx], rng.s2, rng.s3);
+            }
+            const uint32_t incl = wave_inclusive_sum(c);
+            if (idx < n) pre[idx] = carry + incl - c;
+            carry += __shfl(incl, 63, 64);
         }
-        const uint32_t incl = wave_inclusive_sum(c);
-        if (idx < n) pre[idx] = carry + incl - c;
-        carry += __shfl(incl, 63, 64);
+        bin_draws<KIND>(a, g, list, n, rec, pre, carry, bin_start[first], grains);
     }
-    bin_draws<KIND>(a, g, ci0, cj0, list, n, rec, pre, carry, bin_start[bin], grains);
 }
 
 template <int KIND>
 __global__ __launch_bounds__(kBlock, 4) void bin_grains_kernel(PixelArgs a, PixGeom g, const double *T,
                                                                const uint32_t *bin_start,
-                                                               const unsigned long long *bin_mask, float4 *grains)
+                                                               const unsigned long long *bin_mask, float4 *grains,
+                                                               int chunk)
 {
     constexpr int NW = kBlock / 64;
-    __shared__ uint16_t s_list[NW][256];
+    __shared__ uint32_t s_list[NW][256];
     __shared__ uint32_t s_pre[NW][256];
     __shared__ BinRecs s_rec[NW];
     const int wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if (a.grain_total && *a.grain_total > a.grain_cap) return;
-    const int b0 = (blockIdx.x * NW + wid) * kDrawChunk, b1 = min(g.nbx * g.nby, b0 + kDrawChunk);
-#pragma unroll 1
-    for (int bin = b0; bin < b1; ++bin)
-        bin_grains_body<KIND>(a, g, T, bin_start, bin_mask, grains, bin, s_list[wid], s_pre[wid], s_rec[wid]);
+    const long long b0 = (long long)(blockIdx.x * NW + wid) * chunk;
+    const int nbins = g.nbx * g.nby;
+    if (b0 >= nbins) return;
+    draw_bins<KIND>(a, g, T, bin_start, bin_mask, grains, (int)b0, (int)min((long long)nbins, b0 + chunk), s_list[wid],
+                    s_pre[wid], s_rec[wid]);
 }
 
 // The batch's generation kernels run over all its planes in one launch each:
@@ -480,7 +509,7 @@ template <int KIND>
 __global__ __launch_bounds__(kBlock, 4) void batch_bin_grains_kernel(BatchGen bg)
 {
     constexpr int NW = kBlock / 64;
-    __shared__ uint16_t s_list[NW][256];
+    __shared__ uint32_t s_list[NW][256];
     __shared__ uint32_t s_pre[NW][256];
     __shared__ BinRecs s_rec[NW];
     const int wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -492,14 +521,10 @@ __global__ __launch_bounds__(kBlock, 4) void batch_bin_grains_kernel(BatchGen bg
     const int p = cload(bg.kind_plane[KIND] + i);
     const BatchPlane &bp = cplane(bg.planes, p);
     if (bp.a.grain_total && *bp.a.grain_total > bp.a.grain_cap) return;
-    const int b0 = (int)(gc - cload(off + i)) * kDrawChunk;
-    const int b1 = min(bp.geo.nbx * bp.geo.nby, b0 + kDrawChunk);
-    const double *T = cload(bg.T + p);
-    const unsigned long long *mask = bg.mask + 4 * cload(bg.bin_off + p);
-#pragma unroll 1
-    for (int bin = b0; bin < b1; ++bin)
-        bin_grains_body<KIND>(bp.a, bp.geo, T, bp.bin_start, mask, bg.grains, bin, s_list[wid], s_pre[wid],
-                              s_rec[wid]);
+    const int b0 = (int)(gc - cload(off + i)) * bg.draw_chunk;
+    const int b1 = min(bp.geo.nbx * bp.geo.nby, b0 + bg.draw_chunk);
+    draw_bins<KIND>(bp.a, bp.geo, cload(bg.T + p), bp.bin_start, bg.mask + 4 * cload(bg.bin_off + p), bg.grains, b0, b1,
+                    s_list[wid], s_pre[wid], s_rec[wid]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1691,6 +1716,12 @@ hipError_t launch_threshold(const PixelArgs &a, double *T, hipStream_t s)
     return hipGetLastError();
 }
 
+int draw_chunk(long long bins)
+{
+    // 2048 waves are two per SIMD of the 256 CUs
+    return (int)std::max<long long>(1, std::min<long long>(kDrawChunk, bins / 2048));
+}
+
 // chunk bins a wave
 static dim3 bin_grid(const PixGeom &g, int chunk)
 {
@@ -1730,12 +1761,13 @@ hipError_t launch_bin_grains(const PixelArgs &a, const PixGeom &g, int dist_kind
                              const uint32_t *bin_start, const unsigned long long *bin_mask, float4 *grains,
                              hipStream_t s)
 {
+    const int chunk = draw_chunk((long long)g.nbx * g.nby);
     if (dist_kind == 0)
-        hipLaunchKernelGGL((bin_grains_kernel<0>), bin_grid(g, kDrawChunk), dim3(kBlock), 0, s, a, g, T, bin_start, bin_mask,
-                           grains);
+        hipLaunchKernelGGL((bin_grains_kernel<0>), bin_grid(g, chunk), dim3(kBlock), 0, s, a, g, T, bin_start, bin_mask,
+                           grains, chunk);
     else
-        hipLaunchKernelGGL((bin_grains_kernel<1>), bin_grid(g, kDrawChunk), dim3(kBlock), 0, s, a, g, T, bin_start, bin_mask,
-                           grains);
+        hipLaunchKernelGGL((bin_grains_kernel<1>), bin_grid(g, chunk), dim3(kBlock), 0, s, a, g, T, bin_start, bin_mask,
+                           grains, chunk);
     return hipGetLastError();
 }
 
