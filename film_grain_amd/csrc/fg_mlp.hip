@@ -9,13 +9,12 @@
 //
 // Layout.  Parameters are one f32 array (fg_mlp.h offsets): W1 [16][64]
 // (rows 12..15 zero), b1 [64], W2 [64][64] (input-major), b2 [64], w3 [64],
-// b3.  Each workgroup converts them to BF16 in LDS, in the orders the matrix
-// instructions read: W1T [64][16], W2T [64][64] (output-major) and W2 [64][64].
-// Features are BF16 [n][16].  A wave works on 16 rows at a time:
+// b3.  Features are BF16 [n][16].  A wave works on 16 rows at a time, with
+// the weights as BF16 matrix operands in its registers:
 //   layer 1: Z1 = X W1 + b1      4 x v_mfma_f32_16x16x16_bf16 (one per 16 outputs)
 //   layer 2: Z2 = H1 W2 + b2     8 x v_mfma_f32_16x16x32_bf16, H1 = relu(Z1) in BF16
-//                                 through LDS (accumulator rows -> operand rows)
-//   layer 3: y = H2 . w3 + b3     FP32 dot products (a 64-vector), H2 = relu(Z2)
+//   layer 3: y = H2 . w3 + b3    FP32 dot products (a 64-vector), H2 = relu(Z2)
+// The biases are the accumulators' initial values.
 // Backward of the loss per row (fused, per tile), either the squared error to
 // a target t, L = (y - t)^2, g = dL/dy = 2 (y - t), or the Gaussian negative
 // log-likelihood of a residual t under the predicted log std y,
@@ -42,92 +41,39 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
-// f32 -> bf16 bits, round to nearest even (NaN kept quiet).
-__device__ __forceinline__ uint16_t bf16_bits(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
 __device__ __forceinline__ float bf16_float(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
-struct MlpLds {
-    uint16_t w1t[64 * 16];  // [j][k]
-    uint16_t w2t[64 * 64];  // [j_out][k_in]
-    uint16_t w2[64 * 64];   // [k_in][j_out]
-    float b1[64], b2[64], w3[64], b3;
-    uint16_t h[4][16 * 64];  // per wave: a 16 x 64 BF16 tile (H1, then dZ2)
-    uint16_t x[4][16 * 16];  // per wave: the feature tile
-};
+typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 
-__device__ void mlp_load(const float *P, MlpLds &s)
+// relu and round to BF16 (v_cvt_pk_bf16_f32: nearest even).  The median with
+// the largest finite value is one instruction where fmaxf takes two (it first
+// quiets its operand); an infinity rounds to BF16 infinity from there as well,
+// and a NaN gives 0 either way.
+__device__ __forceinline__ v4bf relu_bf16(v4f c)
 {
-    for (int i = threadIdx.x; i < 64 * 16; i += blockDim.x) {
-        const int j = i / 16, k = i % 16;
-        s.w1t[i] = bf16_bits(P[kMlpW1 + k * 64 + j]);
-    }
-    for (int i = threadIdx.x; i < 64 * 64; i += blockDim.x) {
-        const int j = i / 64, k = i % 64;
-        s.w2t[i] = bf16_bits(P[kMlpW2 + k * 64 + j]);
-        s.w2[i] = bf16_bits(P[kMlpW2 + i]);
-    }
-    for (int i = threadIdx.x; i < 64; i += blockDim.x) {
-        s.b1[i] = P[kMlpB1 + i];
-        s.b2[i] = P[kMlpB2 + i];
-        s.w3[i] = bf16_float(bf16_bits(P[kMlpW3 + i]));
-    }
-    if (threadIdx.x == 0) s.b3 = P[kMlpB3];
-    __syncthreads();
+    v4f h;
+    for (int i = 0; i < 4; ++i) h[i] = __builtin_amdgcn_fmed3f(c[i], 0.0f, 3.402823466e+38f);
+    return __builtin_convertvector(h, v4bf);
+}
+__device__ __forceinline__ v8bf join(v4bf a, v4bf b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+__device__ __forceinline__ v4f mfma16(v4bf a, v4bf b, v4f c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(v4s, a), __builtin_bit_cast(v4s, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ v4f mfma32(v8bf a, v8bf b, v4f c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// Forward of one 16-row tile for the calling wave.  z1/z2 receive the
-// pre-activations in accumulator layout (4 column blocks x 4 rows), y the
-// row outputs (lanes of each 16-lane group hold the same 4 rows).
-__device__ __forceinline__ void mlp_tile_forward(const MlpLds &s, uint16_t *hbuf, const uint16_t *xt, v4f z1[4],
-                                                 v4f z2[4], float y[4])
+// Features 4g..4g+3 of a row: 8 bytes, in one load where the rows are so
+// aligned (aligned: uniform).
+__device__ __forceinline__ v4bf load_x(const uint16_t *X, long long row, int g, bool aligned)
 {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    // layer 1: A = X[r][4g..4g+3], B = W1[4g..][cb*16 + r]
-    v4s a1;
-    for (int t = 0; t < 4; ++t) a1[t] = (short)xt[r * 16 + 4 * g + t];
-    for (int cb = 0; cb < 4; ++cb) {
-        v4s b;
-        for (int t = 0; t < 4; ++t) b[t] = (short)s.w1t[(cb * 16 + r) * 16 + 4 * g + t];
-        v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
-        c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, b, c, 0, 0, 0);
-        const float bias = s.b1[cb * 16 + r];
-        for (int i = 0; i < 4; ++i) {
-            c[i] += bias;
-            hbuf[(4 * g + i) * 64 + cb * 16 + r] = bf16_bits(fmaxf(c[i], 0.0f));
-        }
-        z1[cb] = c;
-    }
-    // layer 2: A = H1[r][kc*32 + 8g..+7], B = W2[kc*32 + 8g..][cb*16 + r]
-    v8bf a2[2];
-    for (int kc = 0; kc < 2; ++kc)
-        for (int t = 0; t < 8; ++t) a2[kc][t] = __builtin_bit_cast(__bf16, hbuf[r * 64 + kc * 32 + 8 * g + t]);
-    for (int cb = 0; cb < 4; ++cb) {
-        v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int kc = 0; kc < 2; ++kc) {
-            v8bf b;
-            for (int t = 0; t < 8; ++t)
-                b[t] = __builtin_bit_cast(__bf16, s.w2t[(cb * 16 + r) * 64 + kc * 32 + 8 * g + t]);
-            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[kc], b, c, 0, 0, 0);
-        }
-        const float bias = s.b2[cb * 16 + r];
-        for (int i = 0; i < 4; ++i) c[i] += bias;
-        z2[cb] = c;
-    }
-    // layer 3: y[row] = sum_j relu(Z2[row][j]) w3[j] + b3; lane r of group g
-    // holds columns r, 16 + r, 32 + r, 48 + r of rows 4g..4g+3, so the sum
-    // runs over its four columns, then over the 16 lanes of the group
-    for (int i = 0; i < 4; ++i) {
-        float acc = 0.0f;
-        for (int cb = 0; cb < 4; ++cb) acc += fmaxf(z2[cb][i], 0.0f) * s.w3[cb * 16 + r];
-        for (int o = 1; o < 16; o <<= 1) acc += __shfl_xor(acc, o, 64);
-        y[i] = acc + s.b3;
-    }
+    const uint16_t *p = X + row * 16 + 4 * g;
+    if (aligned) return *reinterpret_cast<const v4bf *>(p);
+    v4bf x;
+    for (int t = 0; t < 4; ++t) x[t] = __builtin_bit_cast(__bf16, p[t]);
+    return x;
 }
 
 // Forward pass for inference, without LDS: the layers are computed
@@ -147,56 +93,112 @@ __device__ __forceinline__ int mlp_h1_column(int kc, int g, int t)
     return kc * 32 + (t < 4 ? 4 * g + t : 16 + 4 * g + (t - 4));
 }
 
-__global__ __launch_bounds__(256) void mlp_forward_kernel(const float *P, const uint16_t *X, long long n, float *out)
+// The layers' weights as matrix operands of lane (r, g), the same registers
+// serving as A of the transposed product and as B of the plain one (the
+// operand layouts mirror each other).
+struct MlpWeights {
+    v4bf w1[4];     // W1[4g + t][cb * 16 + r]
+    v8bf w2[4][2];  // W2[mlp_h1_column(kc, g, t)][cb * 16 + r]
+};
+// The workgroup's copy of the operands, lane by lane.  It is filled by short
+// loops over the parameters, coalesced (straight into registers they are 140
+// gathers a lane).
+struct MlpOperands {
+    __bf16 w1[4][64][4];
+    __bf16 w2[4][2][64][8];
+};
+// Where element (outer column, inner index) of a 64 x 64 operand lies: the
+// inverse of mlp_h1_column.
+__device__ __forceinline__ int mlp_operand_at(int outer, int inner)
 {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-    v4s a1[4];
-    v8bf a2[4][2];
-    float b1[4][4], b2[4][4], w3[4][4];
+    const int cb = outer >> 4, r = outer & 15, kc = inner >> 5, kk = inner & 31;
+    const int g = (kk & 15) >> 2, t = (kk & 3) + ((kk >> 4) << 2);
+    return ((cb * 2 + kc) * 64 + g * 16 + r) * 8 + t;
+}
+__device__ __forceinline__ void fill_operands(const float *P, MlpOperands &s)
+{
+#pragma unroll 1
+    for (int i = threadIdx.x; i < 16 * 64; i += blockDim.x) {
+        const int k = i >> 6, j = i & 63;
+        s.w1[j >> 4][(k >> 2) * 16 + (j & 15)][k & 3] = (__bf16)P[kMlpW1 + i];
+    }
+#pragma unroll 2
+    for (int i = threadIdx.x; i < 64 * 64; i += blockDim.x)
+        (&s.w2[0][0][0][0])[mlp_operand_at(i & 63, i >> 6)] = (__bf16)P[kMlpW2 + i];
+}
+__device__ __forceinline__ void load_weights(const MlpOperands &s, MlpWeights &w, int lane)
+{
     for (int cb = 0; cb < 4; ++cb) {
-        for (int t = 0; t < 4; ++t) a1[cb][t] = (short)bf16_bits(P[kMlpW1 + (4 * g + t) * 64 + cb * 16 + r]);
-        for (int kc = 0; kc < 2; ++kc)
-            for (int t = 0; t < 8; ++t)
-                a2[cb][kc][t] =
-                    __builtin_bit_cast(__bf16, bf16_bits(P[kMlpW2 + mlp_h1_column(kc, g, t) * 64 + cb * 16 + r]));
+        w.w1[cb] = *reinterpret_cast<const v4bf *>(s.w1[cb][lane]);
+        for (int kc = 0; kc < 2; ++kc) w.w2[cb][kc] = *reinterpret_cast<const v8bf *>(s.w2[cb][kc][lane]);
+    }
+}
+
+// Bounded by instruction issue: 12 matrix instructions and about 100 VALU per
+// 16 rows, which do not overlap fully.  2.07M rows (75 MB): 45 us with the
+// conversions in hardware, fused multiply-adds and the biases as initial
+// accumulators; 88 us with conversions in software.  More rows in flight (two
+// to eight tiles ahead, four at once) and two or four waves per SIMD instead
+// of three: no difference.
+constexpr int kTiles = 2;  // 16-row tiles a wave works on at once
+__global__ __launch_bounds__(256, 3) void mlp_forward_kernel(const float *P, const uint16_t *X, long long n, float *out,
+                                                          bool aligned)
+{
+    __shared__ __align__(16) MlpOperands s_op;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    fill_operands(P, s_op);
+    __syncthreads();
+    MlpWeights w;
+    load_weights(s_op, w, lane);
+    v4f b1[4], b2[4], w3[4];
+    for (int cb = 0; cb < 4; ++cb)
         for (int i = 0; i < 4; ++i) {
             const int j = cb * 16 + 4 * g + i;
             b1[cb][i] = P[kMlpB1 + j];
             b2[cb][i] = P[kMlpB2 + j];
-            w3[cb][i] = bf16_float(bf16_bits(P[kMlpW3 + j]));
+            w3[cb][i] = (float)(__bf16)P[kMlpW3 + j];
         }
-    }
     const float b3 = P[kMlpB3];
     const long long tiles = (n + 15) / 16;
-    const long long stride = (long long)gridDim.x * 4;
-    for (long long tt = (long long)blockIdx.x * 4 + wid; tt < tiles; tt += stride) {
-        const long long row = tt * 16 + r;
-        v4s x = {0, 0, 0, 0};
-        if (row < n) {
-            const uint2 v = *reinterpret_cast<const uint2 *>(X + row * 16 + 4 * g);
-            x[0] = (short)(v.x & 0xFFFFu);
-            x[1] = (short)(v.x >> 16);
-            x[2] = (short)(v.y & 0xFFFFu);
-            x[3] = (short)(v.y >> 16);
+    const long long stride = (long long)gridDim.x * 4 * kTiles;
+    const v4bf zero = {};
+    long long tt = ((long long)blockIdx.x * 4 + wid) * kTiles;
+    v4bf x[kTiles], xn[kTiles];  // this step's rows, and the next one's, in flight meanwhile
+    auto fetch = [&](v4bf *v, long long at) {
+        for (int u = 0; u < kTiles; ++u) {
+            const long long row = (at + u) * 16 + r;
+            v[u] = row < n ? load_x(X, row, g, aligned) : zero;
         }
+    };
+    fetch(x, tt);
+    for (; tt < tiles; tt += stride) {
+        fetch(xn, tt + stride);
         // layer 1 (transposed) and the B operand of layer 2
-        v8bf h[2];
-        for (int cb = 0; cb < 4; ++cb) {
-            v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
-            c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1[cb], x, c, 0, 0, 0);
-            for (int i = 0; i < 4; ++i)
-                h[cb >> 1][(cb & 1) * 4 + i] = __builtin_bit_cast(__bf16, bf16_bits(fmaxf(c[i] + b1[cb][i], 0.0f)));
+        v8bf h0[kTiles], h1[kTiles];
+        for (int u = 0; u < kTiles; ++u) {
+            v4bf h[4];
+            for (int cb = 0; cb < 4; ++cb) h[cb] = relu_bf16(mfma16(w.w1[cb], x[u], b1[cb]));
+            h0[u] = join(h[0], h[1]);
+            h1[u] = join(h[2], h[3]);
         }
         // layer 2 (transposed) and layer 3
-        float acc = 0.0f;
-        for (int cb = 0; cb < 4; ++cb) {
-            v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int kc = 0; kc < 2; ++kc) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[cb][kc], h[kc], c, 0, 0, 0);
-            for (int i = 0; i < 4; ++i) acc += fmaxf(c[i] + b2[cb][i], 0.0f) * w3[cb][i];
+        float y[kTiles];
+        for (int u = 0; u < kTiles; ++u) {
+            float acc[4];
+            for (int cb = 0; cb < 4; ++cb) {
+                const v4f c = mfma32(w.w2[cb][1], h1[u], mfma32(w.w2[cb][0], h0[u], b2[cb]));
+                acc[cb] = fmaxf(c[0], 0.0f) * w3[cb][0];
+                for (int i = 1; i < 4; ++i) acc[cb] = __builtin_fmaf(fmaxf(c[i], 0.0f), w3[cb][i], acc[cb]);
+            }
+            y[u] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
         }
-        acc += __shfl_xor(acc, 16, 64);
-        acc += __shfl_xor(acc, 32, 64);
-        if (g == 0 && row < n) out[row] = acc + b3;
+        for (int u = 0; u < kTiles; ++u) {
+            y[u] += __shfl_xor(y[u], 16, 64);
+            y[u] += __shfl_xor(y[u], 32, 64);
+            const long long row = (tt + u) * 16 + r;
+            if (g == 0 && row < n) out[row] = y[u] + b3;
+        }
+        for (int u = 0; u < kTiles; ++u) x[u] = xn[u];
     }
 }
 
@@ -204,128 +206,208 @@ __global__ __launch_bounds__(256) void mlp_forward_kernel(const float *P, const 
 // Gaussian negative log-likelihood of the residual) over rows [0, n) with
 // loss scale 1 / n_total; gradients are added to grad (kMlpParams f32) and
 // the unscaled loss sum to *loss.
-__global__ __launch_bounds__(256) void mlp_grad_kernel(const float *P, const uint16_t *X, const float *target,
-                                                       long long n, float inv_total, int loss_kind, float *grad,
-                                                       float *loss)
+//
+// Every layer is computed in both layouts, plain (lane (r, g): rows 4g..4g+3, column r of a block of
+// 16) and transposed (lane: row r, columns 4g..4g+3), by the same operands in
+// swapped places: the plain form is what the products over rows (dW1, dW2)
+// take as operands, the transposed form what the next product along the
+// layers takes, so nothing crosses lanes but y and its gradient, and LDS
+// holds only W2's backward operands and the T-layout vectors.  X in the plain
+// layout is X times the identity.
+// Bounded by instruction issue at many rows (2M rows: 0.17 ms, 650 us before);
+// at few by the set-up and the atomics on grad, kMlpParams a workgroup: one
+// workgroup per 256 rows up to one per CU (per 1024 rows: 34 us instead of 27
+// at 65536 rows).  65536 rows: 195 us with a workgroup per 64 rows, the
+// transposes through LDS and the reduction by LDS float atomics.
+constexpr int kGradBlock = 512;
+__global__ __launch_bounds__(kGradBlock, 2) void mlp_grad_kernel(const float *P, const uint16_t *X,
+                                                                 const float *target, long long n, float inv_total,
+                                                                 int loss_kind, float *grad, float *loss, bool aligned)
 {
-    __shared__ MlpLds s;
-    __shared__ float s_grad[kMlpParams];
-    __shared__ float s_loss;
-    mlp_load(P, s);
-    for (int i = threadIdx.x; i < kMlpParams; i += blockDim.x) s_grad[i] = 0.0f;
-    if (threadIdx.x == 0) s_loss = 0.0f;
-    __syncthreads();
+    constexpr int NW = kGradBlock / 64;
+    __shared__ __align__(16) MlpOperands s_op;
+    __shared__ v8bf s_w2[4][2][64];   // lane (r, g): W2[cb * 16 + r][mlp_h1_column(kc, g, t)]
+    __shared__ v4f s_b1[16], s_b2[16], s_w3[16];
+    __shared__ v4f s_part[4][20][64];  // the final reduction
+    __shared__ float s_vec[NW][194];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    fill_operands(P, s_op);
+#pragma unroll 2
+    for (int i = threadIdx.x; i < 64 * 64; i += kGradBlock)
+        reinterpret_cast<__bf16 *>(&s_w2[0][0][0])[mlp_operand_at(i >> 6, i & 63)] = (__bf16)P[kMlpW2 + i];
+    if (threadIdx.x < 64) {
+        const int j = threadIdx.x;
+        s_b1[j >> 2][j & 3] = P[kMlpB1 + j];
+        s_b2[j >> 2][j & 3] = P[kMlpB2 + j];
+        s_w3[j >> 2][j & 3] = (float)(__bf16)P[kMlpW3 + j];
+    }
+    __syncthreads();
+    MlpWeights w;
+    load_weights(s_op, w, lane);
+    float b1n[4], b2n[4], w3n[4];
+    for (int cb = 0; cb < 4; ++cb) {
+        b1n[cb] = P[kMlpB1 + cb * 16 + r];
+        b2n[cb] = P[kMlpB2 + cb * 16 + r];
+        w3n[cb] = (float)(__bf16)P[kMlpW3 + cb * 16 + r];
+    }
+    const float b3 = P[kMlpB3];
+    v4bf ident;
+    for (int t = 0; t < 4; ++t) ident[t] = (__bf16)(4 * g + t == r ? 1.0f : 0.0f);
+    const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
     v4f dw2[4][4], dw1[4];
     for (int a = 0; a < 4; ++a) {
-        dw1[a] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-        for (int b = 0; b < 4; ++b) dw2[a][b] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+        dw1[a] = zero4;
+        for (int b = 0; b < 4; ++b) dw2[a][b] = zero4;
     }
     float db1[4] = {0, 0, 0, 0}, db2[4] = {0, 0, 0, 0}, dw3[4] = {0, 0, 0, 0}, db3 = 0.0f, lsum = 0.0f;
-    const long long tiles = (n + 15) / 16;
-    for (long long t = (long long)blockIdx.x * 4 + wid; t < tiles; t += (long long)gridDim.x * 4) {
-        uint16_t *xt = s.x[wid];
-        uint16_t *hb = s.h[wid];
-        for (int i = lane; i < 256; i += 64) {
-            const long long row = t * 16 + i / 16;
-            xt[i] = row < n ? X[row * 16 + (i % 16)] : (uint16_t)0;
+    const long long tiles = (n + 15) / 16, stride = (long long)gridDim.x * NW;
+    long long tt = (long long)blockIdx.x * NW + wid;
+    v4bf x = {};
+    float t = 0.0f;
+    if (tt < tiles && tt * 16 + r < n) {
+        x = load_x(X, tt * 16 + r, g, aligned);
+        t = target[tt * 16 + r];
+    }
+    for (; tt < tiles; tt += stride) {
+        // keeps the LDS operands from being held in registers all loop long,
+        // where they spilled
+        asm volatile("" ::: "memory");
+        const long long row = tt * 16 + r, next = row + stride * 16;
+        v4bf xnext = {};
+        float tnext = 0.0f;
+        if (next < n) {  // the next tile's, in flight meanwhile
+            xnext = load_x(X, next, g, aligned);
+            tnext = target[next];
         }
-        v4f z1[4], z2[4];
-        float y[4];
-        mlp_tile_forward(s, hb, xt, z1, z2, y);
-        // output gradient (rows past n contribute nothing)
-        float gr[4];
-        for (int i = 0; i < 4; ++i) {
-            const long long row = t * 16 + 4 * g + i;
-            if (row >= n) {
-                gr[i] = 0.0f;
-                continue;
+        // layer 1 transposed
+        v4bf h[4];
+        for (int cb = 0; cb < 4; ++cb) h[cb] = relu_bf16(mfma16(w.w1[cb], x, s_b1[cb * 4 + g]));
+        const v8bf h0 = join(h[0], h[1]), h1 = join(h[2], h[3]);
+        // layer 2 transposed, y of row r and its gradient
+        float y = 0.0f;
+        uint32_t m2 = 0;  // transposed: Z2 > 0
+        for (int cb = 0; cb < 4; ++cb) {
+            const v4f c = mfma32(w.w2[cb][1], h1, mfma32(w.w2[cb][0], h0, s_b2[cb * 4 + g]));
+            const v4f w3 = s_w3[cb * 4 + g];
+            for (int i = 0; i < 4; ++i) {
+                m2 |= c[i] > 0.0f ? 1u << (cb * 4 + i) : 0u;
+                y = __builtin_fmaf(fmaxf(c[i], 0.0f), w3[i], y);
             }
-            const float t = target[row];
+        }
+        y += __shfl_xor(y, 16, 64);
+        y += __shfl_xor(y, 32, 64);
+        y += b3;
+        float gy = 0.0f;  // rows past n contribute nothing
+        if (row < n) {
+            float l;
             if (loss_kind == 1) {
-                const float e = expf(fminf(fmaxf(-2.0f * y[i], -80.0f), 80.0f)) * t * t;
-                gr[i] = (1.0f - e) * inv_total;
-                if (r == 0) lsum += y[i] + 0.5f * e;
+                const float e = expf(fminf(fmaxf(-2.0f * y, -80.0f), 80.0f)) * t * t;
+                gy = (1.0f - e) * inv_total;
+                l = y + 0.5f * e;
             } else {
-                const float d = y[i] - t;
-                gr[i] = 2.0f * d * inv_total;
-                if (r == 0) lsum += d * d;
+                const float d = y - t;
+                gy = 2.0f * d * inv_total;
+                l = d * d;
+            }
+            if (g == 0) {
+                lsum += l;
+                db3 += gy;
             }
         }
-        // layer 3 and dZ2 (accumulator layout), dW2 = H1^T dZ2 on MFMA
-        v4f dz2[4];
+        // dZ2 transposed, the A operand of dZ1 = dZ2 W2^T
+        v4bf zt[4];
         for (int cb = 0; cb < 4; ++cb) {
-            const float w = s.w3[cb * 16 + r];
-            for (int i = 0; i < 4; ++i) {
-                const float h2 = fmaxf(z2[cb][i], 0.0f);
-                dw3[cb] += gr[i] * h2;
-                dz2[cb][i] = z2[cb][i] > 0.0f ? gr[i] * w : 0.0f;
-                db2[cb] += dz2[cb][i];
-            }
+            const v4f w3 = s_w3[cb * 4 + g];
+            v4f d;
+            for (int i = 0; i < 4; ++i) d[i] = (m2 >> (cb * 4 + i)) & 1u ? gy * w3[i] : 0.0f;
+            zt[cb] = __builtin_convertvector(d, v4bf);
         }
-        if (r == 0)
-            for (int i = 0; i < 4; ++i) db3 += gr[i];
-        // dZ2 as BF16 B operand (rows 4g.., column r) and A^T operand via LDS
-        v4s bz[4];
-        for (int cb = 0; cb < 4; ++cb)
-            for (int i = 0; i < 4; ++i) bz[cb][i] = (short)bf16_bits(dz2[cb][i]);
-        // A = H1^T[kb*16 + r][rows 4g..4g+3] from the H1 tile (row-major)
-        for (int kb = 0; kb < 4; ++kb) {
-            v4s a;
-            for (int i = 0; i < 4; ++i) a[i] = (short)hb[(4 * g + i) * 64 + kb * 16 + r];
-            for (int cb = 0; cb < 4; ++cb)
-                dw2[kb][cb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bz[cb], dw2[kb][cb], 0, 0, 0);
-        }
-        // dH1 = dZ2 W2^T: A = dZ2[r][kc*32 + 8g..] through LDS, B[b][a] = W2[a][b]
-        for (int cb = 0; cb < 4; ++cb)
-            for (int i = 0; i < 4; ++i) hb[(4 * g + i) * 64 + cb * 16 + r] = (uint16_t)bz[cb][i];
-        v8bf az[2];
-        for (int kc = 0; kc < 2; ++kc)
-            for (int q = 0; q < 8; ++q) az[kc][q] = __builtin_bit_cast(__bf16, hb[r * 64 + kc * 32 + 8 * g + q]);
-        v4f dz1[4];
+        const v8bf z0 = join(zt[0], zt[1]), z1 = join(zt[2], zt[3]);
+        // layer 2 plain: dw3, db2 and dZ2
+        float gr[4];
+        for (int i = 0; i < 4; ++i) gr[i] = __shfl(gy, 4 * g + i, 64);
+        v4bf zn[4];
         for (int cb = 0; cb < 4; ++cb) {
-            v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int kc = 0; kc < 2; ++kc) {
-                v8bf b;
-                for (int q = 0; q < 8; ++q)
-                    b[q] = __builtin_bit_cast(__bf16, s.w2[(cb * 16 + r) * 64 + kc * 32 + 8 * g + q]);
-                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(az[kc], b, c, 0, 0, 0);
-            }
+            const v4f c =
+                mfma32(h1, w.w2[cb][1], mfma32(h0, w.w2[cb][0], (v4f){b2n[cb], b2n[cb], b2n[cb], b2n[cb]}));
+            v4f d;
             for (int i = 0; i < 4; ++i) {
-                c[i] = z1[cb][i] > 0.0f ? c[i] : 0.0f;
+                dw3[cb] = __builtin_fmaf(gr[i], fmaxf(c[i], 0.0f), dw3[cb]);
+                d[i] = c[i] > 0.0f ? gr[i] * w3n[cb] : 0.0f;
+                db2[cb] += d[i];
+            }
+            zn[cb] = __builtin_convertvector(d, v4bf);
+        }
+        // layer 1 and dZ1 plain, and the products over the rows
+        const v4bf xn = __builtin_convertvector(mfma16(x, ident, zero4), v4bf);
+        for (int cb = 0; cb < 4; ++cb) {
+            const v4f a1 = mfma16(x, w.w1[cb], (v4f){b1n[cb], b1n[cb], b1n[cb], b1n[cb]});
+            const v4bf hn = relu_bf16(a1);
+            for (int k = 0; k < 4; ++k) dw2[cb][k] = mfma16(hn, zn[k], dw2[cb][k]);
+            v4f c = mfma32(z1, s_w2[cb][1][lane], mfma32(z0, s_w2[cb][0][lane], zero4));
+            for (int i = 0; i < 4; ++i) {
+                c[i] = a1[i] > 0.0f ? c[i] : 0.0f;
                 db1[cb] += c[i];
             }
-            dz1[cb] = c;
+            dw1[cb] = mfma16(xn, __builtin_convertvector(c, v4bf), dw1[cb]);
         }
-        // dW1 = X^T dZ1: A = X^T[r][rows 4g..] (feature r), B = dZ1 (BF16)
-        v4s ax;
-        for (int i = 0; i < 4; ++i) ax[i] = (short)xt[(4 * g + i) * 16 + r];
-        for (int cb = 0; cb < 4; ++cb) {
-            v4s b;
-            for (int i = 0; i < 4; ++i) b[i] = (short)bf16_bits(dz1[cb][i]);
-            dw1[cb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ax, b, dw1[cb], 0, 0, 0);
-        }
+        x = xnext;
+        t = tnext;
     }
-    // reduce: accumulator blocks hold D[4g+i][r]
-    for (int kb = 0; kb < 4; ++kb)
-        for (int cb = 0; cb < 4; ++cb)
-            for (int i = 0; i < 4; ++i)
-                atomicAdd(&s_grad[kMlpW2 + (kb * 16 + 4 * g + i) * 64 + cb * 16 + r], dw2[kb][cb][i]);
+    // Reduce over the workgroup without LDS float atomics (those took 57 us of
+    // 82 at 65536 rows): the upper four waves hand their accumulators to the
+    // lower four through LDS, those leave theirs there, and every thread sums
+    // four and adds to grad.  Accumulator blocks hold D[4g+i][r].
     for (int cb = 0; cb < 4; ++cb)
-        for (int i = 0; i < 4; ++i) atomicAdd(&s_grad[kMlpW1 + (4 * g + i) * 64 + cb * 16 + r], dw1[cb][i]);
-    for (int cb = 0; cb < 4; ++cb) {
-        atomicAdd(&s_grad[kMlpB1 + cb * 16 + r], db1[cb]);
-        atomicAdd(&s_grad[kMlpB2 + cb * 16 + r], db2[cb]);
-        atomicAdd(&s_grad[kMlpW3 + cb * 16 + r], dw3[cb]);
+        for (int o = 16; o < 64; o <<= 1) {
+            db1[cb] += __shfl_xor(db1[cb], o, 64);
+            db2[cb] += __shfl_xor(db2[cb], o, 64);
+            dw3[cb] += __shfl_xor(dw3[cb], o, 64);
+        }
+    for (int o = 1; o < 64; o <<= 1) {
+        db3 += __shfl_xor(db3, o, 64);
+        lsum += __shfl_xor(lsum, o, 64);
     }
-    if (r == 0) {
-        atomicAdd(&s_grad[kMlpB3], db3);
-        atomicAdd(&s_loss, lsum);
+    if (g == 0)
+        for (int cb = 0; cb < 4; ++cb) {
+            s_vec[wid][cb * 16 + r] = db1[cb];
+            s_vec[wid][64 + cb * 16 + r] = db2[cb];
+            s_vec[wid][128 + cb * 16 + r] = dw3[cb];
+        }
+    if (lane == 0) {
+        s_vec[wid][192] = db3;
+        s_vec[wid][193] = lsum;
     }
+    auto each = [&](auto f) {
+        for (int kb = 0; kb < 4; ++kb) {
+            for (int cb = 0; cb < 4; ++cb) f(kb * 4 + cb, dw2[kb][cb]);
+            f(16 + kb, dw1[kb]);
+        }
+    };
+    if (wid >= 4) each([&](int k, v4f &v) { s_part[wid - 4][k][lane] = v; });
     __syncthreads();
-    for (int i = threadIdx.x; i < kMlpParams; i += blockDim.x)
-        if (s_grad[i] != 0.0f) atomicAdd(&grad[i], s_grad[i]);
-    if (threadIdx.x == 0) atomicAdd(loss, s_loss);
+    if (wid < 4) each([&](int k, v4f &v) { s_part[wid][k][lane] = v + s_part[wid][k][lane]; });
+    __syncthreads();
+#pragma unroll 1
+    for (int e = threadIdx.x; e < 20 * 256; e += kGradBlock) {
+        // element i of block k's lane l, lanes of a row first
+        const int k = e >> 8, l = ((e >> 6) & 3) * 16 + (e & 15), i = (e >> 4) & 3;
+        const float v = (s_part[0][k][l][i] + s_part[1][k][l][i]) + (s_part[2][k][l][i] + s_part[3][k][l][i]);
+        const int row = 4 * (l >> 4) + i;
+        const int at = k < 16 ? kMlpW2 + ((k >> 2) * 16 + row) * 64 + (k & 3) * 16 + (l & 15)
+                              : kMlpW1 + row * 64 + (k & 3) * 16 + (l & 15);
+        if (v != 0.0f) atomicAdd(&grad[at], v);
+    }
+    if (threadIdx.x < 194) {
+        float v = 0.0f;
+        for (int q = 0; q < NW; ++q) v += s_vec[q][threadIdx.x];
+        const int j = threadIdx.x & 63, which = threadIdx.x >> 6;
+        float *dst = which == 0 ? grad + kMlpB1 + j
+                     : which == 1 ? grad + kMlpB2 + j
+                     : which == 2 ? grad + kMlpW3 + j
+                                  : (j == 0 ? grad + kMlpB3 : loss);
+        if (v != 0.0f) atomicAdd(dst, v);
+    }
 }
 
 // Adam (Kingma & Ba 2015) with bias correction; rows 12..15 of W1 stay 0.
@@ -351,13 +433,19 @@ __global__ void mlp_adam_kernel(float *P, const float *grad, float *m, float *v,
 // variance of u over its 3x3 neighbourhood (edges clamped), the gradient
 // magnitude (central differences), u (1 - u), the radius law, filter sigma and
 // zoom (scaled to order one), and the channel one-hot.
+// Bounded by its stores, 32 bytes a pixel: two 16-byte stores where the rows
+// are so aligned (wide), and the pixel's row by a 32-bit division where the
+// plane has fewer than 2^32 pixels (2.07M pixels: 18 us; 50 us with 16
+// two-byte stores and a 64-bit division).
 __global__ __launch_bounds__(256) void feature_kernel(const float *u, int in_w, int in_h, int out_w, int out_h,
                                                       float inv_zoom, float f_radius, float f_sd, float f_sigma,
-                                                      float f_zoom, int channel, uint16_t *X)
+                                                      float f_zoom, int channel, uint16_t *X, bool wide)
 {
     const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (p >= (long long)out_w * out_h) return;
-    const int y = (int)(p / out_w), x = (int)(p - (long long)y * out_w);
+    const long long n = (long long)out_w * out_h;
+    if (p >= n) return;
+    const int y = n <= 0xFFFFFFFFLL ? (int)((uint32_t)p / (uint32_t)out_w) : (int)(p / out_w);
+    const int x = (int)(p - (long long)y * out_w);
     const int ix = min(max((int)floorf(((float)x + 0.5f) * inv_zoom), 0), in_w - 1);
     const int iy = min(max((int)floorf(((float)y + 0.5f) * inv_zoom), 0), in_h - 1);
     auto at = [&](int dx, int dy) {
@@ -379,7 +467,17 @@ __global__ __launch_bounds__(256) void feature_kernel(const float *u, int in_w, 
                    f_sigma, f_zoom,     channel == 0 ? 1.0f : 0.0f, channel == 1 ? 1.0f : 0.0f,
                    channel == 2 ? 1.0f : 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     uint16_t *dst = X + p * 16;
-    for (int i = 0; i < 16; ++i) dst[i] = bf16_bits(f[i]);
+    if (wide) {
+        v8bf lo, hi;
+        for (int i = 0; i < 8; ++i) {
+            lo[i] = (__bf16)f[i];
+            hi[i] = (__bf16)f[8 + i];
+        }
+        reinterpret_cast<v8bf *>(dst)[0] = lo;
+        reinterpret_cast<v8bf *>(dst)[1] = hi;
+    } else {
+        for (int i = 0; i < 16; ++i) dst[i] = __builtin_bit_cast(uint16_t, (__bf16)f[i]);
+    }
 }
 
 // Sample budget n = clamp(ceil(c * s), nmin, nmax) per pixel, from s =
@@ -570,22 +668,22 @@ hipError_t launch_budget_scale(const float *pred, long long n, float s_mult, dou
 hipError_t launch_mlp_forward(const float *P, const uint16_t *X, long long n, float *out, hipStream_t s)
 {
     // waves loop over 16-row tiles.  Each wave first loads the whole network
-    // into registers (138 VGPRs: 3 waves per SIMD), so the grid is one
-    // resident round of waves (3 workgroups of 4 waves per CU on 256 CUs)
-    // and each wave amortises that load over many tiles.
+    // into registers, so the grid is one resident round of waves (three
+    // workgroups of 4 waves per CU on 256 CUs) and each wave amortises that
+    // load over many tiles.
     const long long tiles = (n + 15) / 16;
-    const unsigned grid = (unsigned)std::min<long long>((tiles + 3) / 4, 768);
-    hipLaunchKernelGGL(mlp_forward_kernel, dim3(std::max(grid, 1u)), dim3(256), 0, s, P, X, n, out);
+    const unsigned grid = (unsigned)std::min<long long>((tiles + 4 * kTiles - 1) / (4 * kTiles), 768);
+    hipLaunchKernelGGL(mlp_forward_kernel, dim3(std::max(grid, 1u)), dim3(256), 0, s, P, X, n, out,
+                       reinterpret_cast<uintptr_t>(X) % 8 == 0);
     return hipGetLastError();
 }
 
 hipError_t launch_mlp_grad(const float *P, const uint16_t *X, const float *target, long long n, float inv_total,
                            int loss_kind, float *grad, float *loss, hipStream_t s)
 {
-    const long long tiles = (n + 15) / 16;
-    const unsigned grid = (unsigned)std::min<long long>((tiles + 3) / 4, 1024);
-    hipLaunchKernelGGL(mlp_grad_kernel, dim3(std::max(grid, 1u)), dim3(256), 0, s, P, X, target, n, inv_total,
-                       loss_kind, grad, loss);
+    const unsigned grid = (unsigned)std::min<long long>((n + 255) / 256, 256);
+    hipLaunchKernelGGL(mlp_grad_kernel, dim3(std::max(grid, 1u)), dim3(kGradBlock), 0, s, P, X, target, n, inv_total,
+                       loss_kind, grad, loss, reinterpret_cast<uintptr_t>(X) % 8 == 0);
     return hipGetLastError();
 }
 
@@ -602,7 +700,8 @@ hipError_t launch_features(const float *u, int in_w, int in_h, int out_w, int ou
 {
     const long long n = (long long)out_w * out_h;
     hipLaunchKernelGGL(feature_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, u, in_w, in_h, out_w, out_h,
-                       1.0f / zoom, radius / 0.3f, sd / 0.15f, sigma / 2.0f, zoom / 4.0f, channel, X);
+                       1.0f / zoom, radius / 0.3f, sd / 0.15f, sigma / 2.0f, zoom / 4.0f, channel, X,
+                       reinterpret_cast<uintptr_t>(X) % 16 == 0);
     return hipGetLastError();
 }
 

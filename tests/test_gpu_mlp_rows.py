@@ -1,0 +1,76 @@
+"""The error model's kernels at row counts around their tiles (16 rows, two
+tiles a step, a workgroup per 256 gradient rows) and with feature rows that
+are not 8-byte aligned, against the CPU fp32 reference; NaN features."""
+import numpy as np
+import pytest
+
+from film_grain_amd import synth
+from tests import mlp_ref
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(rng, n, shift):
+    import torch
+    P = rng.normal(0, 0.3, mlp_ref.N_PARAMS).astype(np.float32)
+    P[mlp_ref.P_W1 + 12 * 64:mlp_ref.P_B1] = 0.0
+    X = np.zeros((n, 16), np.float32)
+    X[:, :12] = rng.uniform(-1, 1, (n, 12))
+    X = mlp_ref.bf16(X)
+    bits = (np.ascontiguousarray(X).view(np.uint32) >> 16).astype(np.uint16).view(np.int16)
+    buf = torch.zeros(n * 16 + shift, dtype=torch.int16, device="cuda:0")
+    buf[shift:] = torch.from_numpy(bits.reshape(-1)).to("cuda:0")
+    return P, X, buf[shift:].view(n, 16)
+
+
+@pytest.mark.parametrize("n,shift", [(1, 0), (15, 0), (17, 1), (32, 0), (33, 3), (255, 0), (257, 1), (4097, 0),
+                                     (65537, 0), (200001, 1)])
+@pytest.mark.parametrize("kind", ["squared", "nll"])
+def test_rows_around_the_tiles(hip_ctx, n, shift, kind):
+    import torch
+    rng = np.random.default_rng(n)
+    P, X, Xd = _case(rng, n, shift)
+    t = rng.normal(0, 1, n).astype(np.float32)
+    Pd, td = torch.from_numpy(P).to("cuda:0"), torch.from_numpy(t).to("cuda:0")
+    guard = torch.full((n + 64,), 7.0, device="cuda:0")
+    hip_ctx.mlp_forward(Pd, Xd, out=guard[:n])
+    assert torch.all(guard[n:] == 7.0)  # rows past n are not written
+    y_ref = mlp_ref.forward(P, X)[-1]
+    assert np.abs(guard[:n].cpu().numpy() - y_ref).max() <= 1e-3 * (np.abs(y_ref).max() + 1e-6)
+    grad = torch.zeros(mlp_ref.N_PARAMS, dtype=torch.float32, device="cuda:0")
+    loss = torch.zeros(1, dtype=torch.float32, device="cuda:0")
+    hip_ctx.mlp_grad(Pd, Xd, td, grad, loss, loss_kind=kind)
+    g_ref, l_ref = mlp_ref.grad(P, X, t, loss=kind)
+    # the reference rounds the same operands to BF16; one that falls on the
+    # other side of a rounding is off by 2^-8 of one row's term
+    d = np.linalg.norm(grad.cpu().numpy() - g_ref) / np.linalg.norm(g_ref)
+    assert d <= 2.0 ** -8, (n, kind, d)
+    assert abs(float(loss.item()) - l_ref) <= 1e-4 * abs(l_ref) + 1e-6
+
+
+def test_nan_features_act_as_before_the_first_relu(hip_ctx):
+    """A NaN feature makes its row's first layer NaN, which relu turns to 0;
+    the other rows of its tile are untouched."""
+    import torch
+    rng = np.random.default_rng(5)
+    P, X, Xd = _case(rng, 48, 0)
+    Xd = Xd.clone()
+    Xd[20, 3] = 0x7FC0
+    y = hip_ctx.mlp_forward(torch.from_numpy(P).to("cuda:0"), Xd).cpu().numpy()
+    y_ref = mlp_ref.forward(P, X)[-1]
+    rows = np.arange(48) != 20
+    assert np.abs(y - y_ref)[rows].max() <= 1e-3 * np.abs(y_ref).max()
+    h2 = np.maximum(P[mlp_ref.P_B2:mlp_ref.P_B2 + 64], 0)
+    want = float(h2 @ mlp_ref.bf16(P[mlp_ref.P_W3:mlp_ref.P_W3 + 64]) + P[mlp_ref.P_B3])
+    assert abs(y[20] - want) <= 1e-4 * max(1.0, abs(want))
+
+
+@pytest.mark.parametrize("shift", [0, 1, 4])
+def test_feature_rows_at_any_alignment(hip_ctx, shift):
+    import torch
+    u = torch.from_numpy(synth.sinusoid_field(37, 23, 4, n_waves=3)).to("cuda:0")
+    want = hip_ctx.mlp_features(u, 55, 34, 1.5, 0.1, 0.05, 0.8, 1)
+    buf = torch.full((55 * 34 * 16 + 2 * shift + 16,), 123, dtype=torch.int16, device="cuda:0")
+    hip_ctx.mlp_features(u, 55, 34, 1.5, 0.1, 0.05, 0.8, 1, out=buf[shift:shift + 55 * 34 * 16])
+    assert torch.equal(buf[shift:shift + 55 * 34 * 16].view(-1, 16), want)
+    assert torch.all(buf[:shift] == 123) and torch.all(buf[shift + 55 * 34 * 16:] == 123)
