@@ -362,10 +362,15 @@ bin_count_planes_kernel(PixelArgs a, PixGeom g, FramePlanes fp)
         }
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            unsigned long long x = c[p];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-            total[p] += x;
+            if (__ballot(c[p] >= 1u << 26) == 0ull) {
+                // 64 counts below 2^26 sum in 32 bits
+                total[p] += (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_sum(c[p]), 63);
+            } else {
+                unsigned long long x = c[p];
+#pragma unroll 1
+                for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+                total[p] += x;
+            }
         }
     }
 #pragma unroll
