@@ -45,7 +45,7 @@ def grain_space(desc):
     shape and workgroup size."""
     words = (desc.n_samples + 31) // 32
     out = []
-    for tw, th in [(16, 16), (32, 16), (32, 32), (64, 16), (64, 32), (64, 64), (128, 32), (128, 64)]:
+    for tw, th in [(16, 16), (32, 16), (32, 32), (48, 32), (64, 16), (64, 24), (64, 28), (64, 32), (64, 64), (128, 32), (128, 64)]:
         if tw * th * words * 4 > 96 * 1024:
             continue
         for block in (256, 512):

@@ -1213,23 +1213,32 @@ int do_grainwise(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lambda, con
         fg::SampleTable st{};
         mark(ctx, 0, s);
         hipError_t e = fg::launch_sample_table(a.offs, a.n_samples, 1.0f, q, ctx->samples.p, &st, s);
-        // constant radius with a narrow window (2R + 1/Q <= 0.35 output px):
-        // candidate lists per cell of the grain's fractional target, about
-        // N (2R + 1/Q)^2 samples each instead of a run of N (2R + 1/Q)
-        const int cq = 64;
+        // Candidate lists for narrow grains, about N (2R + 1/Q)^2 samples each
+        // instead of a run of N (2R + 1/Q): one class for a constant radius
+        // below 0.45 output pixels (the kernel's narrow limit is 1/2 less its
+        // widening; a plane too large for that takes its general test), the
+        // classes up to the largest narrow radius for a lognormal law.
         const float r_out = std::min(d->radius_mean, d->rm) * d->zoom;
-        if (e == hipSuccess && d->dist_kind == 0 && r_out > 0.0f && 2.0f * r_out + 1.0f / (float)cq <= 0.35f) {
-            const size_t nstart = (size_t)cq * cq + 1;
-            if ((rc = ensure_bytes(ctx, ctx->cells, nstart * 4 + (size_t)cq * cq * a.n_samples * 2 + 64, what)) !=
+        const bool lognorm = d->dist_kind != 0;
+        if (lognorm || (r_out > 0.0f && r_out <= 0.45f)) {
+            const int cq = lognorm ? fg::kGrainClassQ : fg::kGrainConstQ;
+            const int classes =
+                lognorm ? std::max(1, std::min(cq, (int)std::ceil(std::min(a.r_out_max, 0.5f) * 2.0f * cq))) : 1;
+            const size_t cells = (size_t)classes * cq * cq;
+            if ((rc = ensure_bytes(ctx, ctx->cells, 256 + cells * sizeof(uint2) + cells * a.n_samples * 2 + 256, what)) !=
                 FG_OK)
                 return rc;
-            uint32_t *cs = static_cast<uint32_t *>(ctx->cells.p);
-            uint16_t *cl = reinterpret_cast<uint16_t *>(cs + nstart);
+            unsigned char *cb = static_cast<unsigned char *>(ctx->cells.p);
+            uint2 *cell = reinterpret_cast<uint2 *>(cb + 256);
+            uint16_t *list = reinterpret_cast<uint16_t *>(cell + cells);
             const float c_base = (float)std::max(a.out_w, a.out_h) + a.r_out_max + 8.0f;
-            e = fg::launch_cell_lists(st, a.n_samples, cq, r_out, c_base, cs, cl, s);
-            a.cell_start = cs;
-            a.cell_list = cl;
-            a.cell_q = cq;
+            if (e == hipSuccess)
+                e = fg::launch_grain_lists(st, cq, classes, lognorm ? 0.0f : r_out, c_base,
+                                           reinterpret_cast<uint32_t *>(cb), cell, list, a.status, s);
+            a.gl_cell = cell;
+            a.gl_list = list;
+            a.gl_classes = classes;
+            a.r_list = r_out;
         }
         if (e == hipSuccess) e = fg::launch_pixel_state(a, s);
         if (e == hipSuccess) e = fg::launch_grain_tile_weights(a, st, order.w, order.ids, s);

@@ -218,6 +218,104 @@ __device__ __forceinline__ float from_lane_f(float v, int ba)
     return __int_as_float(__builtin_amdgcn_ds_bpermute(ba, __float_as_int(v)));
 }
 
+// LDS locations as 32-bit LDS addresses: a bitset word's address held in a
+// sample record is used as it is, with no workgroup base added per hit
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+__device__ __forceinline__ uint32_t lds_addr(uint32_t *p)
+{
+    return (uint32_t)(uintptr_t)(lds_u32 *)p;
+}
+__device__ __forceinline__ void lds_or(uint32_t addr, uint32_t v)
+{
+    __hip_atomic_fetch_or((lds_u32 *)(uintptr_t)addr, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// a * b + c for a, b < 2^24 with one full-rate v_mad_u32_u24 (b uniform).
+// Written out because the compiler turns two such terms into two products
+// and a three-way add.
+__device__ __forceinline__ uint32_t mad_u24(uint32_t a, uint32_t b, uint32_t c)
+{
+    uint32_t d;
+    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(b), "v"(c));
+    return d;
+}
+
+// The candidate lists of a wave's grains, concatenated in lane order into one
+// stream of `total` entries, walked 64 entries a step.  The grains with a list
+// are numbered by their place in that order (their rank); rank k has a 16-byte
+// record at rec + 16 k (the wave's own LDS) whose last word is its first list
+// position, less its first stream entry, plus bias.  The stream's entry e
+// belongs to the grain whose rank is the number of lists that end before e: a
+// set bit per list end (its last entry, my_end per lane; -1 for none, and for
+// the stream's last list, so that lanes past the stream count as its entries)
+// in a bitset of the batch's entries (ends, 2 STAGE words of the wave's LDS),
+// so that a step's owners are a count of the set bits below each lane (two
+// v_mbcnt) on top of the count before the step.  (Taking the owners from a
+// scalar loop over the grains that start within the step was half of the
+// walk's scalar instructions: the splat of a 4K RGB frame at N = 256 took
+// 13.6 ms and takes 11.2.)
+//
+// A batch is STAGE steps: their owners first, then all their list loads in
+// flight together, then test(owner's record offset, entry) for each: one
+// global latency per batch of steps instead of one per step.  Lanes past the
+// stream read its last entry (the stream's last pair again: its bit is ORed
+// twice, which changes nothing).  A step from s loads stream entry s +
+// min(lane, total - 1 - s), and the steps of a batch that start past the
+// stream have s < total + 64 (STAGE - 1); with bias = total + 64 STAGE the
+// lane's part of the list position is positive: a load takes a base in SGPRs
+// (the batch's first entry, less the bias), a valid unsigned 32-bit offset in
+// one VGPR and the step's 128 bytes as its immediate offset, no 64-bit address
+// arithmetic.  Whole batches come first, then a shorter one where it holds
+// the rest: the lists of a small N are a few entries each.
+//
+// The wave's LDS accesses run in order, so no barrier is needed.
+template <int STAGE, class Test>
+__device__ __forceinline__ void walk_batch(int sb, int total, int bias, int my_end, uint32_t *ends,
+                                           const unsigned char *rec, const unsigned char *list, uint32_t &before,
+                                           Test &&test)
+{
+    const int lane = threadIdx.x & 63;
+    if (lane < 2 * STAGE) ends[lane] = 0u;
+    __builtin_amdgcn_wave_barrier();
+    const int rel = my_end - sb;
+    if ((unsigned)rel < 64u * STAGE && my_end >= 0) lds_or(lds_addr(ends + (rel >> 5)), 1u << (rel & 31));
+    __builtin_amdgcn_wave_barrier();
+    const unsigned char *lbb = list + 2 * ((long long)sb - bias);
+    uint32_t own[STAGE], pn[STAGE];
+#pragma unroll
+    for (int i = 0; i < STAGE; ++i) {
+        const uint2 e = *reinterpret_cast<const uint2 *>(ends + 2 * i);
+        own[i] = __builtin_amdgcn_mbcnt_hi(e.y, __builtin_amdgcn_mbcnt_lo(e.x, before)) << 4;
+        before += __popc(e.x) + __popc(e.y);
+    }
+#pragma unroll
+    for (int i = 0; i < STAGE; ++i) {
+        const uint32_t pos = *reinterpret_cast<const uint32_t *>(rec + own[i] + 12) +
+                             (uint32_t)min(lane, total - 1 - (sb + 64 * i));
+        pn[i] = (uint32_t)*reinterpret_cast<const uint16_t *>(lbb + 128 * i + (pos << 1));
+    }
+#pragma unroll
+    for (int i = 0; i < STAGE; ++i) {
+        if (sb + 64 * i >= total) break;
+        test(own[i], pn[i]);
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int STAGE, class Test>
+__device__ __forceinline__ void walk_lists(int total, int bias, int my_end, uint32_t *ends, const unsigned char *rec,
+                                           const unsigned char *list, Test &&test)
+{
+    static_assert(STAGE >= 4, "batches of STAGE, STAGE / 2 and STAGE / 4 steps");
+    uint32_t before = 0;  // list ends before the step
+    int sb = 0;
+    for (; total - sb > 64 * (STAGE / 2); sb += 64 * STAGE)
+        walk_batch<STAGE>(sb, total, bias, my_end, ends, rec, list, before, test);
+    if (total - sb > 64 * (STAGE / 4))
+        walk_batch<STAGE / 2>(sb, total, bias, my_end, ends, rec, list, before, test);
+    else if (total - sb > 0)
+        walk_batch<STAGE / 4>(sb, total, bias, my_end, ends, rec, list, before, test);
+}
+
 }  // namespace fg
 
 #endif

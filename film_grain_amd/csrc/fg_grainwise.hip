@@ -326,27 +326,42 @@ hipError_t launch_grain_tile_weights(const GrainArgs &a, const SampleTable &st, 
     return hipGetLastError();
 }
 
-// Entries of a round's concatenated candidate lists that the per-wave owner
-// map holds (256 B per wave keeps a 64x32 tile's workgroup at 40 KB of LDS,
-// four per CU).
-constexpr int kOwnerMap = 256;
+// How a plane's grains find their samples: constant radius through candidate
+// lists, constant radius through runs of the sample order (grains too wide for
+// lists), lognormal radii through lists where narrow and runs where not.
+enum GrainMode { kConstLists, kConstRuns, kLognormal };
 
-// Entry pos of a candidate list: a 32-bit byte offset from the list's base,
-// so that the load takes the base in SGPRs and the offset in one VGPR (no
-// 64-bit address arithmetic in the walk's steps: 19.55 -> 19.28 ms at C3).
-__device__ __forceinline__ int list_at(const uint16_t *list, uint32_t pos)
-{
-    return (int)*reinterpret_cast<const uint16_t *>(reinterpret_cast<const unsigned char *>(list) + (pos << 1));
-}
+// Steps of the list walk in flight together: a round of 64 grains has about
+// two entries a grain at the constant-radius workload (r = 0.05, N = 128) and
+// five to twenty under lognormal laws.
+constexpr int grain_stage(int mode) { return mode == kConstLists ? 4 : 8; }
+constexpr int kGrainStageMax = 8;
+// Words a wave keeps for its round: the listed grains' records (16 bytes
+// each), then the candidate queue of the others.
+constexpr int kGrainWaveWords = 256;
+static_assert(kGrainWaveWords >= kQueueCap, "the queue shares the records' room");
 
-template <int KIND, int BLOCK>
-__global__ __launch_bounds__(BLOCK, 8) void grainwise_sorted(GrainArgs a, SampleTable st)
+// Waves per SIMD each mode's registers are held to (lognormal draws need f64
+// transcendentals; at eight waves they spilled 25 registers).
+constexpr int grain_waves(int mode) { return mode == kLognormal ? 5 : 8; }
+
+// Per output tile: rounds of one grain per lane, each drawn from its input
+// pixel's stream and its samples found through its list or run.
+// Bounded by instruction issue: the draws (repeated for each tile whose halo
+// holds the pixel) and about 28 VALU per list entry.  Before lognormal laws
+// had lists their lanes walked runs in lockstep, every candidate by its box
+// and the queue: 1021x767 at zoom 2, r = 0.1 / 0.03, N = 128 took 7.1 ms and
+// takes 1.6; a 1280x720 plane, r = 0.1 / 0.05, N = 64, 2.69 and 0.73.  The
+// constant-radius plane of 4096x4096 (r = 0.05, N = 128; owners from a byte
+// map, boxes evaluated for every entry, 64x32 tiles): 16.7 and 14.6 ms.
+template <int MODE, int BLOCK>
+__global__ __launch_bounds__(BLOCK, grain_waves(MODE)) void grainwise_sorted(GrainArgs a, SampleTable st)
 {
-    constexpr int NW = BLOCK / 64;
+    constexpr int NW = BLOCK / 64, STAGE = grain_stage(MODE);
+    constexpr bool LISTS = MODE != kConstRuns, RUNS = MODE != kConstLists;
     extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ uint32_t s_queue[NW][kQueueCap];
-    // per wave, the owner lane of each entry of a round's concatenated lists
-    __shared__ uint8_t s_owner[NW][kOwnerMap];
+    __shared__ __align__(16) uint32_t s_wave[NW][kGrainWaveWords];
+    __shared__ __align__(16) uint32_t s_ends[NW][2 * kGrainStageMax];
     // the region's next pixel that no lane has taken
     __shared__ int s_next;
 
@@ -364,27 +379,31 @@ __global__ __launch_bounds__(BLOCK, 8) void grainwise_sorted(GrainArgs a, Sample
     const float fy0 = uniform_f((float)Y0), fy1 = uniform_f((float)(Y1 - 1));
     const int words = a.words, N = a.n_samples, Q = st.qbuckets;
     const int tile_words = a.tile_w * a.tile_h * words;
+    const uint32_t w4 = (uint32_t)words * 4u, row_b = (uint32_t)a.tile_w * w4;
 
-    // ---- LDS: bitset | xy[N] | k[N] | qidx[Q + 1] ----
+    // ---- LDS: (X, word, bit)[N] | qidx[Q + 1] | bitset ----
+    // Per sorted position one 16-byte record: the sample's scaled offset, the
+    // LDS address of its bitset word for pixel 0 and its bit's mask (as in the
+    // splat); a list entry is its byte offset.
     size_t off = 0;
-    uint32_t *bits = reinterpret_cast<uint32_t *>(lds);
-    off += ((size_t)tile_words * 4 + 15) & ~(size_t)15;
-    float2 *sxy = reinterpret_cast<float2 *>(lds + off);
-    off += ((size_t)N * 8 + 15) & ~(size_t)15;
-    uint16_t *sk = reinterpret_cast<uint16_t *>(lds + off);
-    off += ((size_t)N * 2 + 15) & ~(size_t)15;
+    float4 *srec = reinterpret_cast<float4 *>(lds);
+    off += (size_t)N * 16;
     uint16_t *sq = reinterpret_cast<uint16_t *>(lds + off);
-    off += ((size_t)(Q + 1) * 2 + 15) & ~(size_t)15;
+    if (RUNS) off += ((size_t)(Q + 1) * 2 + 15) & ~(size_t)15;
+    uint32_t *bits = reinterpret_cast<uint32_t *>(lds + off);
+    off += ((size_t)tile_words * 4 + 15) & ~(size_t)15;
     if (off > (size_t)a.lds_bytes) {
         if (tid == 0) atomicOr(a.status, kStatusRegion);
         return;
     }
     for (int w = tid; w < tile_words; w += BLOCK) bits[w] = 0u;
     for (int k = tid; k < N; k += BLOCK) {
-        sxy[k] = st.xy[k];
-        sk[k] = st.k[k];
+        const float2 X = st.xy[k];
+        const uint32_t ki = st.k[k];
+        srec[k] = make_float4(X.x, X.y, __uint_as_float(lds_addr(bits + (ki >> 5))), __uint_as_float(1u << (ki & 31u)));
     }
-    for (int q = tid; q <= Q; q += BLOCK) sq[q] = st.qidx[q];
+    if (RUNS)
+        for (int q = tid; q <= Q; q += BLOCK) sq[q] = st.qidx[q];
     if (tid == 0) s_next = 0;
     const float4 ext0 = *st.ext;
     const float4 ext = make_float4(uniform_f(ext0.x), uniform_f(ext0.y), uniform_f(ext0.z), uniform_f(ext0.w));
@@ -399,11 +418,25 @@ __global__ __launch_bounds__(BLOCK, 8) void grainwise_sorted(GrainArgs a, Sample
     const float C = (float)max(a.out_w, a.out_h) + fmaxf(fmaxf(fabsf(ext.x), fabsf(ext.y)),
                                                          fmaxf(fabsf(ext.z), fabsf(ext.w))) + Rmax + 8.0f;
     const float eps = uniform_f(C * 9.5367431640625e-07f + 1.52587890625e-05f);  // C * 2^-20 + 2^-16
+    // a grain below this radius covers pixels nearest its target alone
+    const float narrow_r = uniform_f(0.5f - (eps + eps));
+    // within this of the radius a passing pixel's bounds() box is looked at
+    const float edge = uniform_f(C * 4.76837158203125e-07f);  // C * 2^-21
     const float Qf = uniform_f((float)Q);
-    uint32_t *queue = s_queue[wid];
+    uint32_t *queue = s_wave[wid];
     int qcount = 0;
     // the lane's current grain: target origin and output radius
     float gbx = 0.0f, gby = 0.0f, gR = 0.0f;
+
+    auto hit = [&](int tx, int ty, const float4 &r) {
+        lds_or(mad_u24((uint32_t)ty, row_b, mad_u24((uint32_t)tx, w4, __float_as_uint(r.z))), __float_as_uint(r.w));
+    };
+    // The pixels of bounds() of src/grainwise.rs:126-142 before its clamp (the
+    // tile lies inside the image, so meeting the tile is the clamp).
+    auto bounds = [](float t, float R, float &lo, float &hi) {
+        lo = ceilf((t - R) - 0.5f);
+        hi = floorf((t + R) - 0.5f);
+    };
 
     // Entries: lane (6 bits) | sorted position << 6 (11 bits) | tile column
     // << 17 (7 bits) | tile row << 24 (8 bits).  The reference's disk test
@@ -416,13 +449,11 @@ __global__ __launch_bounds__(BLOCK, 8) void grainwise_sorted(GrainArgs a, Sample
         const float bx = __shfl(gbx, l, 64), by = __shfl(gby, l, 64), R = __shfl(gR, l, 64);
         if (lane >= n) return;
         const int p = (int)((e >> 6) & 0x7FFu), tx = (int)((e >> 17) & 0x7Fu), ty = (int)(e >> 24);
-        const float2 X = sxy[p];
-        const int k = sk[p];
-        const float txp = bx + X.x, typ = by + X.y;
+        const float4 r = srec[p];
+        const float txp = bx + r.x, typ = by + r.y;
         const float dy = ((float)(Y0 + ty) + 0.5f) - typ;
-        const float dy2 = dy * dy;
         const float dx = ((float)(X0 + tx) + 0.5f) - txp;
-        if (dx * dx + dy2 <= R * R) atomicOr(&bits[(ty * a.tile_w + tx) * words + (k >> 5)], 1u << (k & 31));
+        if (dx * dx + dy * dy <= R * R) hit(tx, ty, r);
     };
     auto push = [&](bool cand, uint32_t entry) {
         const unsigned long long mask = __ballot(cand);
@@ -454,7 +485,7 @@ __global__ __launch_bounds__(BLOCK, 8) void grainwise_sorted(GrainArgs a, Sample
             const int cnt = __popcll(m);
             int base = 0;
             if (lane == 0) base = atomicAdd(&s_next, cnt);
-            base = __shfl(base, 0, 64);
+            base = __builtin_amdgcn_readfirstlane(base);
             more = base + cnt < npx;
             const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -474,73 +505,148 @@ __global__ __launch_bounds__(BLOCK, 8) void grainwise_sorted(GrainArgs a, Sample
             }
         }
         if (!__any(done < q)) break;
-        {
-            // the lane's next grain (src/grainwise.rs:48-67)
-            int p0 = 0, len = 0;
-            float bx = 0.0f, by = 0.0f, R = 0.0f;
-            if (done < q) {
-                const float cx = fx + uniform_f32(rng, 1.0f);
-                const float cy = fy + uniform_f32(rng, 1.0f);
-                float rad = KIND == 0 ? a.r_const : lognormal_f32(rng, a.log_mu, a.log_sigma, d_zig_x, d_zig_f);
-                ++done;
-                if (rad > a.rm) rad = a.rm;
-                R = rad * z;
-                bx = cx * z;
-                by = cy * z;
-                // skip radii <= 0 and grains whose boxes miss the tile for
-                // every sample (bounds() is monotone in the target); one mask,
-                // not a chain of branches
-                const bool keep = ((int)(rad > 0.0f) & (int)(R > 0.0f) &
-                                   (int)(floorf(((bx + ext.y) + R) - 0.5f) >= fx0) &
-                                   (int)(ceilf(((bx + ext.x) - R) - 0.5f) <= fx1) &
-                                   (int)(floorf(((by + ext.w) + R) - 0.5f) >= fy0) &
-                                   (int)(ceilf(((by + ext.z) - R) - 0.5f) <= fy1)) != 0;
-                if (keep && a.cell_q > 0) {
-                    // the candidate list of the cell of (A, B), the fractions
-                    // of the grain's x and y targets (build_cell_lists)
-                    const float ncx = R - (bx - 0.5f), ncy = R - (by - 0.5f);
-                    const float A = ncx - floorf(ncx), B = ncy - floorf(ncy);
-                    const float cq = (float)a.cell_q;
-                    const int qa = min(max((int)(A * cq), 0), a.cell_q - 1);
-                    const int qb = min(max((int)(B * cq), 0), a.cell_q - 1);
-                    const int c = qb * a.cell_q + qa;
-                    p0 = (int)a.cell_start[c];
-                    len = (int)a.cell_start[c + 1] - p0;
-                } else if (keep) {
-                    const float nc = R - (bx - 0.5f);
-                    const float A = nc - floorf(nc);
-                    const float lo = (A - (R + R)) - eps, hi = A + eps;
-                    if (!(lo * Qf > -2.0f * Qf) || !(hi * Qf < 2.0f * Qf) ||
-                        (int)floorf(hi * Qf) + 1 - (int)floorf(lo * Qf) >= Q) {
-                        len = N;
-                    } else {
-                        int lq = (int)floorf(lo * Qf), hq = (int)floorf(hi * Qf) + 1;
-                        if (lq < 0) {
-                            lq += Q;
-                            hq += Q;
-                        }
-                        lq = min(max(lq, 0), Q - 1);
-                        hq = min(max(hq, lq + 1), 2 * Q);
-                        p0 = sq[lq];
-                        const int end = hq <= Q ? (int)sq[hq] : N + (int)sq[hq - Q];
-                        len = end - p0;
+        // the lane's next grain (src/grainwise.rs:48-67)
+        int p0 = 0, len = 0;
+        bool listed = false;
+        float bx = 0.0f, by = 0.0f, R = 0.0f;
+        if (done < q) {
+            const float cx = fx + uniform_f32(rng, 1.0f);
+            const float cy = fy + uniform_f32(rng, 1.0f);
+            float rad = MODE == kLognormal ? lognormal_f32(rng, a.log_mu, a.log_sigma, d_zig_x, d_zig_f) : a.r_const;
+            ++done;
+            if (rad > a.rm) rad = a.rm;
+            R = rad * z;
+            bx = cx * z;
+            by = cy * z;
+            // skip radii <= 0 and grains whose boxes miss the tile for
+            // every sample (bounds() is monotone in the target); one mask,
+            // not a chain of branches
+            const bool keep = ((int)(rad > 0.0f) & (int)(R > 0.0f) &
+                               (int)(floorf(((bx + ext.y) + R) - 0.5f) >= fx0) &
+                               (int)(ceilf(((bx + ext.x) - R) - 0.5f) <= fx1) &
+                               (int)(floorf(((by + ext.w) + R) - 0.5f) >= fy0) &
+                               (int)(ceilf(((by + ext.z) - R) - 0.5f) <= fy1)) != 0;
+            const int cls = MODE == kLognormal ? (int)(R * (float)(2 * kGrainClassQ)) : 0;
+            listed = LISTS && keep && (MODE == kConstLists || (R < narrow_r && cls < a.gl_classes));
+            if (listed) {
+                // the list of the grain's class and of the cell of its centre
+                // fractions (grain_lists_kernel)
+                const float nx = 0.5f - bx, ny = 0.5f - by;
+                const float A = nx - floorf(nx), B = ny - floorf(ny);
+                const int gq = MODE == kLognormal ? kGrainClassQ : kGrainConstQ;
+                const int qa = min((int)(A * (float)gq), gq - 1), qb = min((int)(B * (float)gq), gq - 1);
+                const uint2 se = a.gl_cell[(uint32_t)(cls * gq + qb) * (uint32_t)gq + (uint32_t)qa];
+                p0 = (int)se.x;
+                len = (int)se.y;
+            } else if (RUNS && keep) {
+                // the run of samples whose box can hold a column
+                const float nc = R - (bx - 0.5f);
+                const float A = nc - floorf(nc);
+                const float lo = (A - (R + R)) - eps, hi = A + eps;
+                if (!(lo * Qf > -2.0f * Qf) || !(hi * Qf < 2.0f * Qf) ||
+                    (int)floorf(hi * Qf) + 1 - (int)floorf(lo * Qf) >= Q) {
+                    len = N;
+                } else {
+                    int lq = (int)floorf(lo * Qf), hq = (int)floorf(hi * Qf) + 1;
+                    if (lq < 0) {
+                        lq += Q;
+                        hq += Q;
                     }
+                    lq = min(max(lq, 0), Q - 1);
+                    hq = min(max(hq, lq + 1), 2 * Q);
+                    p0 = sq[lq];
+                    const int end = hq <= Q ? (int)sq[hq] : N + (int)sq[hq - Q];
+                    len = end - p0;
                 }
             }
+        }
+        if (LISTS) {
+            const bool walks = listed && len > 0;
+            const unsigned long long lmask = __ballot(walks);
+            if (lmask) {
+                const uint32_t fl = walks ? (uint32_t)len : 0u;
+                const uint32_t incl = wave_inclusive_sum(fl);
+                const int total = __builtin_amdgcn_readlane((int)incl, 63);
+                const int bias = total + 64 * STAGE;
+                const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(lmask >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)lmask, 0u));
+                float4 *rec = reinterpret_cast<float4 *>(s_wave[wid]);
+                if (walks) rec[rank] = make_float4(bx, by, R, __int_as_float(p0 - (int)(incl - fl) + bias));
+                const unsigned char *recb = reinterpret_cast<const unsigned char *>(rec);
+                const int my_end = walks && (int)incl != total ? (int)incl - 1 : -1;
+                const unsigned char *list = reinterpret_cast<const unsigned char *>(a.gl_list);
+                // A narrow grain's disk reaches only the pixel whose square
+                // holds the target, x = floor(t): a pixel whose centre is
+                // within R < 1/2 of t is that one.  It passes the reference's
+                // disk test and lies in its bounds() box; where |dx| and |dy|
+                // are at most R - C 2^-21 the box follows from them (its two
+                // roundings and theirs are at most C 2^-24 each), and only
+                // nearer the rim is it evaluated.
+                auto narrow = [&](uint32_t own, uint32_t entry) {
+                    const float4 g = *reinterpret_cast<const float4 *>(recb + own);
+                    const float4 r = *reinterpret_cast<const float4 *>(lds + entry);
+                    asm volatile("" ::"v"(r.x), "v"(r.y), "v"(r.z), "v"(r.w));
+                    const float txp = g.x + r.x, typ = g.y + r.y;
+                    const float px = floorf(txp), py = floorf(typ);
+                    const int tx = (int)px - X0, ty = (int)py - Y0;
+                    if (((unsigned)tx < (unsigned)(X1 - X0)) & ((unsigned)ty < (unsigned)(Y1 - Y0))) {
+                        const float dx = (px + 0.5f) - txp, dy = (py + 0.5f) - typ;
+                        if (dx * dx + dy * dy <= g.z * g.z) {
+                            bool in = fmaxf(fabsf(dx), fabsf(dy)) <= g.z - edge;
+                            if (!in) {
+                                float xl, xh, yl, yh;
+                                bounds(txp, g.z, xl, xh);
+                                bounds(typ, g.z, yl, yh);
+                                in = (xl <= px) & (px <= xh) & (yl <= py) & (py <= yh);
+                            }
+                            if (in) hit(tx, ty, r);
+                        }
+                    }
+                };
+                // constant radii close to 1/2 of planes so large that eps is
+                // not small against it: every pixel of the box in the lane
+                auto general = [&](uint32_t own, uint32_t entry) {
+                    const float4 g = *reinterpret_cast<const float4 *>(recb + own);
+                    const float4 r = *reinterpret_cast<const float4 *>(lds + entry);
+                    const float txp = g.x + r.x, typ = g.y + r.y;
+                    float xl, xh, yl, yh;
+                    bounds(txp, g.z, xl, xh);
+                    bounds(typ, g.z, yl, yh);
+                    xl = fmaxf(xl, fx0);
+                    xh = fminf(xh, fx1);
+                    yl = fmaxf(yl, fy0);
+                    yh = fminf(yh, fy1);
+                    for (float y = yl; y <= yh; y += 1.0f)
+                        for (float x = xl; x <= xh; x += 1.0f) {
+                            const float dx = (x + 0.5f) - txp, dy = (y + 0.5f) - typ;
+                            if (dx * dx + dy * dy <= g.z * g.z) hit((int)(x - fx0), (int)(y - fy0), r);
+                        }
+                };
+                if (MODE == kConstLists && !(a.r_list < narrow_r)) {
+                    uint32_t before = 0;
+                    for (int sb = 0; sb < total; sb += 64)
+                        walk_batch<1>(sb, total, bias, my_end, s_ends[wid], recb, list, before, general);
+                } else {
+                    walk_lists<STAGE>(total, bias, my_end, s_ends[wid], recb, list, narrow);
+                }
+            }
+        }
+        if (RUNS && __any(!listed && len > 0)) {
             gbx = bx;
             gby = by;
             gR = R;
-            // One candidate per lane: sample p (sorted position) against the
-            // grain of lane gl, whose target origin and output radius are
-            // (ebx, eby) and eR; ok false: nothing to test.
-            auto visit = [&](bool ok, int p, int gl, float ebx, float eby, float eR) {
-                const float2 X = sxy[p];
-                const float txp = ebx + X.x, typ = eby + X.y;
-                // bounds() of src/grainwise.rs:126-142 before its clamp; the
-                // tile lies inside the image, so meeting the tile is the clamp
-                const float xl = ceilf((txp - eR) - 0.5f), xh = floorf((txp + eR) - 0.5f);
-                const float yl = ceilf((typ - eR) - 0.5f), yh = floorf((typ + eR) - 0.5f);
-                const bool cand = ok & (xl <= xh) & (yl <= yh) & (xl <= fx1) & (xh >= fx0) & (yl <= fy1) &
+            const int rlen = listed ? 0 : len;
+            for (int it = 0; __any(it < rlen); ++it) {
+                // the cyclic run position (lanes past their run read a valid
+                // sample and queue nothing)
+                const int pr = p0 + it;
+                const int p = (int)min(min((uint32_t)pr, (uint32_t)(pr - N)), (uint32_t)(N - 1));
+                const float4 r = srec[p];
+                const float txp = bx + r.x, typ = by + r.y;
+                float xl, xh, yl, yh;
+                bounds(txp, R, xl, xh);
+                bounds(typ, R, yl, yh);
+                const bool cand = (it < rlen) & (xl <= xh) & (yl <= yh) & (xl <= fx1) & (xh >= fx0) & (yl <= fy1) &
                                   (yh >= fy0);
                 // a candidate box of one pixel lies in the tile (it meets
                 // it); wider boxes queue their pixels inside the tile
@@ -549,14 +655,11 @@ __global__ __launch_bounds__(BLOCK, 8) void grainwise_sorted(GrainArgs a, Sample
                     // one pixel per candidate: the drain's test of it, run
                     // here in the lane (same f32 expression)
                     if (cand) {
-                        const int k = sk[p];
-                        const int tx = (int)(xl - fx0), ty = (int)(yl - fy0);
                         const float dx = (xl + 0.5f) - txp, dy = (yl + 0.5f) - typ;
-                        if (dx * dx + dy * dy <= eR * eR)
-                            atomicOr(&bits[(ty * a.tile_w + tx) * words + (k >> 5)], 1u << (k & 31));
+                        if (dx * dx + dy * dy <= R * R) hit((int)(xl - fx0), (int)(yl - fy0), r);
                     }
                 } else {
-                    const uint32_t base = (uint32_t)gl | ((uint32_t)p << 6);
+                    const uint32_t base = (uint32_t)lane | ((uint32_t)p << 6);
                     const float cxl = fmaxf(xl, fx0), cxh = fminf(xh, fx1);
                     const float cyl = fmaxf(yl, fy0), cyh = fminf(yh, fy1);
                     const int tx = (int)(cxl - fx0), ty = (int)(cyl - fy0);
@@ -567,57 +670,6 @@ __global__ __launch_bounds__(BLOCK, 8) void grainwise_sorted(GrainArgs a, Sample
                         const int jy = c ? j / bw : 0, jx = c ? j - jy * bw : 0;
                         push(c, base | ((uint32_t)(tx + jx) << 17) | ((uint32_t)(ty + jy) << 24));
                     }
-                }
-            };
-            if (a.cell_q > 0) {
-                // The lanes' candidate lists, concatenated in lane order, are
-                // walked 64 entries a step (the per-lane walk ran for the
-                // wave's longest list).  Entry e belongs to the first lane g
-                // whose running total incl_g exceeds e, i.e. g = the number
-                // of lanes with incl <= e (a binary search over the
-                // nondecreasing incl), and is its list entry p0 + e - excl.
-                const uint32_t incl = wave_inclusive_sum((uint32_t)len);
-                const int total = __builtin_amdgcn_readlane((int)incl, 63);
-                const int excl = (int)incl - len;
-                const int dl = p0 - excl;
-                // Rounds of at most kOwnerMap entries (nearly all: about two
-                // per grain at C3) write each entry's owner lane into the
-                // wave's map, so that a step reads it with one load; longer
-                // rounds search the running totals.  The wave's LDS accesses
-                // run in order, so no barrier is needed.
-                const bool mapped = total <= kOwnerMap;  // uniform
-                if (mapped) {
-                    for (int j = 0; j < len; ++j) s_owner[wid][excl + j] = (uint8_t)lane;
-                    for (int s0 = 0; s0 < total; s0 += 64) {
-                        const int e = s0 + lane;
-                        const int g = s_owner[wid][min(e, total - 1)];
-                        const bool ok = e < total;
-                        const int ga = g << 2;
-                        const uint32_t pos = (uint32_t)(from_lane_i(dl, ga) + e);
-                        const int p = ok ? list_at(a.cell_list, pos) : 0;
-                        visit(ok, p, g, from_lane_f(bx, ga), from_lane_f(by, ga), from_lane_f(R, ga));
-                    }
-                } else {
-                    for (int s0 = 0; s0 < total; s0 += 64) {
-                        const int e = s0 + lane;
-                        int g = 0;
-#pragma unroll
-                        for (int b = 32; b >= 1; b >>= 1)
-                            g += from_lane_i((int)incl, (g + b - 1) << 2) <= e ? b : 0;
-                        const bool ok = e < total;  // then g <= 63 and its list holds e
-                        const int ga = g << 2;
-                        const uint32_t pos = (uint32_t)(from_lane_i(dl, ga) + e);
-                        const int p = ok ? list_at(a.cell_list, pos) : 0;
-                        visit(ok, p, g, from_lane_f(bx, ga), from_lane_f(by, ga), from_lane_f(R, ga));
-                    }
-                }
-            } else {
-                for (int it = 0; __any(it < len); ++it) {
-                    // the cyclic run position (lanes past their run read a
-                    // valid sample and queue nothing)
-                    const int pr = p0 + it;
-                    visit(it < len, (int)min(min((uint32_t)pr, (uint32_t)(pr - N)), (uint32_t)(N - 1)), lane, bx, by,
-                          R);
                 }
             }
             // the queue refers to the lanes' current grains
@@ -639,98 +691,38 @@ __global__ __launch_bounds__(BLOCK, 8) void grainwise_sorted(GrainArgs a, Sample
     }
 }
 
-// Candidate lists for grains of one constant output radius R: cell (qa, qb)
-// of a Q x Q grid over the fractions (A, B) of a grain's x and y targets
-// lists, in sorted position order, every sample whose fractions lie in
-// [qa/Q - 2R - eps, (qa+1)/Q + eps] and [qb/Q - 2R - eps, (qb+1)/Q + eps]
-// (mod 1), each widened by 2^-12.  A grain in the cell needs at most the
-// samples whose fraction lies in [A - 2R - eps, A + eps] (its box then has a
-// column: the per-grain run's argument) and in [B - 2R - eps, B + eps] (a
-// row), so the list is a superset of the candidates and the exact tests
-// downstream decide.  eps is the kernel's: C * 2^-20 + 2^-16 with C =
-// c_base + the offsets' largest magnitude.  One workgroup, one cell per
-// thread and pass; start has Q * Q + 1 entries, list room for Q * Q * N.
-__global__ __launch_bounds__(1024) void cell_lists_kernel(SampleTable st, int N, int Q, float R, float c_base,
-                                                          uint32_t *start, uint16_t *list)
+size_t grainwise_sorted_static_lds(int block)
 {
-    __shared__ uint32_t s_count[1024];
-    const float4 ext = *st.ext;
-    const float C = c_base + fmaxf(fmaxf(fabsf(ext.x), fabsf(ext.y)), fmaxf(fabsf(ext.z), fabsf(ext.w)));
-    const float eps = C * 9.5367431640625e-07f + 1.52587890625e-05f;
-    const float m = 2.44140625e-4f;  // 2^-12
-    const float w = ((R + R) + (eps + eps)) + (1.0f / (float)Q + (m + m));
-    const int cells = Q * Q;
-    auto member = [&](int c, int p) {
-        const float2 X = st.xy[p];
-        const float fx = X.x - floorf(X.x), fy = X.y - floorf(X.y);
-        const float lx = ((float)(c % Q) / (float)Q - (R + R)) - (eps + m);
-        const float ly = ((float)(c / Q) / (float)Q - (R + R)) - (eps + m);
-        float dx = fx - lx, dy = fy - ly;
-        dx -= floorf(dx);
-        dy -= floorf(dy);
-        return dx <= w && dy <= w;
-    };
-    uint32_t base = 0;
-    for (int c0 = 0; c0 < cells; c0 += 1024) {
-        const int c = c0 + (int)threadIdx.x;
-        uint32_t n = 0;
-        if (c < cells)
-            for (int p = 0; p < N; ++p) n += member(c, p) ? 1u : 0u;
-        s_count[threadIdx.x] = n;
-        __syncthreads();
-        // inclusive scan of the pass's counts (Hillis-Steele)
-        for (int o = 1; o < 1024; o <<= 1) {
-            const uint32_t v = threadIdx.x >= (unsigned)o ? s_count[threadIdx.x - o] : 0u;
-            __syncthreads();
-            s_count[threadIdx.x] += v;
-            __syncthreads();
-        }
-        const uint32_t first = base + s_count[threadIdx.x] - n;
-        if (c < cells) {
-            start[c] = first;
-            uint32_t k = first;
-            for (int p = 0; p < N; ++p)
-                if (member(c, p)) list[k++] = (uint16_t)p;
-        }
-        base += s_count[1023];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) start[cells] = base;
+    return (size_t)block / 64 * (kGrainWaveWords * 4 + 2 * kGrainStageMax * 4) + 64;
 }
-
-hipError_t launch_cell_lists(const SampleTable &st, int n, int q, float r_out, float c_base, uint32_t *start,
-                             uint16_t *list, hipStream_t s)
-{
-    hipLaunchKernelGGL(cell_lists_kernel, dim3(1), dim3(1024), 0, s, st, n, q, r_out, c_base, start, list);
-    return hipGetLastError();
-}
-
-size_t grainwise_sorted_static_lds(int block) { return (size_t)block / 64 * (kQueueCap * 4 + kOwnerMap) + 64; }
 
 size_t grainwise_sorted_lds(int tile_w, int tile_h, int n_samples, int qbuckets)
 {
     const size_t words = ((size_t)n_samples + 31) / 32;
     auto a16 = [](size_t b) { return (b + 15) & ~(size_t)15; };
-    return a16((size_t)tile_w * tile_h * words * 4) + a16((size_t)n_samples * 8) + a16((size_t)n_samples * 2) +
-           a16((size_t)(qbuckets + 1) * 2);
+    return a16((size_t)tile_w * tile_h * words * 4) + (size_t)n_samples * 16 + a16((size_t)(qbuckets + 1) * 2);
+}
+
+template <int MODE>
+static void launch_sorted_mode(const GrainArgs &a, const SampleTable &st, int block, hipStream_t s)
+{
+    const dim3 grid(a.n_tiles);
+    const size_t lds = (size_t)a.lds_bytes;
+    if (block == 256)
+        hipLaunchKernelGGL((grainwise_sorted<MODE, 256>), grid, dim3(256), lds, s, a, st);
+    else
+        hipLaunchKernelGGL((grainwise_sorted<MODE, 512>), grid, dim3(512), lds, s, a, st);
 }
 
 hipError_t launch_grainwise_sorted(const GrainArgs &a, const SampleTable &st, int dist_kind, int block,
                                    hipStream_t s)
 {
-    const dim3 grid(a.n_tiles);
-    const size_t lds = (size_t)a.lds_bytes;
-    if (dist_kind == 0) {
-        if (block == 256)
-            hipLaunchKernelGGL((grainwise_sorted<0, 256>), grid, dim3(256), lds, s, a, st);
-        else
-            hipLaunchKernelGGL((grainwise_sorted<0, 512>), grid, dim3(512), lds, s, a, st);
-    } else {
-        if (block == 256)
-            hipLaunchKernelGGL((grainwise_sorted<1, 256>), grid, dim3(256), lds, s, a, st);
-        else
-            hipLaunchKernelGGL((grainwise_sorted<1, 512>), grid, dim3(512), lds, s, a, st);
-    }
+    if (dist_kind != 0)
+        launch_sorted_mode<kLognormal>(a, st, block, s);
+    else if (a.gl_classes > 0)
+        launch_sorted_mode<kConstLists>(a, st, block, s);
+    else
+        launch_sorted_mode<kConstRuns>(a, st, block, s);
     return hipGetLastError();
 }
 

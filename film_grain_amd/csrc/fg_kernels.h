@@ -68,6 +68,9 @@ struct PixelArgs {
     float cl_inv_dz;
 };
 
+// Cells per side of the grain-wise candidate lists.
+constexpr int kGrainConstQ = 64, kGrainClassQ = 32;
+
 // Grain-wise integrator launch (src/grainwise.rs:12-124).
 struct GrainArgs {
     const float *lambda;
@@ -89,13 +92,15 @@ struct GrainArgs {
     uint32_t *pix_q;
     ulonglong2 *pix_s01, *pix_s23;
     const int *tile_list;  // optional launch order of the tiles (sorted kernel)
-    // optional candidate lists of the sorted kernel (constant radius): cell
-    // qb * cell_q + qa of a cell_q x cell_q grid over the grain's fractional
-    // target (A, B) lists sorted positions cell_list[cell_start[c] ..
-    // cell_start[c + 1]); cell_q = 0: the per-grain run instead
-    const uint32_t *cell_start;
-    const uint16_t *cell_list;
-    int cell_q;
+    // optional candidate lists of the sorted kernel (gl_classes > 0): (start,
+    // length) in gl_list per (class, cell of the grain's centre fractions);
+    // constant radius: one class of radius r_list, kGrainConstQ^2 cells;
+    // lognormal: class k of radii below (k + 1) / (2 kGrainClassQ),
+    // kGrainClassQ^2 cells.  An entry is a sorted position times 16.
+    const uint2 *gl_cell;
+    const uint16_t *gl_list;
+    int gl_classes;
+    float r_list;
 };
 
 // Writes (min x, max x, min y, max y) of n (x, y) pairs to *range (one workgroup).

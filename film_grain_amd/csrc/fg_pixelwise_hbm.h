@@ -115,12 +115,14 @@ size_t grainwise_sorted_static_lds(int block);
 hipError_t launch_pixel_state(const GrainArgs &a, hipStream_t s);
 hipError_t launch_grainwise_sorted(const GrainArgs &a, const SampleTable &st, int dist_kind, int block,
                                    hipStream_t s);
-// Candidate lists of the sorted grain-wise kernel for one constant output
-// radius r_out (GrainArgs::cell_*): q x q cells, start (q * q + 1 entries),
-// list (room for q * q * n positions); c_base = max(out_w, out_h) + the
-// largest output radius + 8 (the kernel's widening bound without the offsets).
-hipError_t launch_cell_lists(const SampleTable &st, int n, int q, float r_out, float c_base, uint32_t *start,
-                             uint16_t *list, hipStream_t s);
+// Candidate lists of the sorted grain-wise kernel: for r_const > 0 one class of
+// that output radius, else `classes` classes of radius (k + 1) / (2 q); q x q
+// cells each.  cell: classes * q * q (start, length) pairs; list: room for
+// classes * q * q * n positions; fill: classes counters (cleared here).
+// c_base = max(out_w, out_h) + the largest output radius + 8 (the kernel's
+// widening bound without the offsets).  Needs st.n <= 2048.
+hipError_t launch_grain_lists(const SampleTable &st, int q, int classes, float r_const, float c_base, uint32_t *fill,
+                              uint2 *cell, uint16_t *list, int *status, hipStream_t s);
 
 // Heaviest-first tile order: w[t] = the work of tile t (grains of the bins
 // covering its region), ids[t] = t; sort_tiles orders ids by w, descending

@@ -816,9 +816,11 @@ struct ListsShared {
     bool fits;
 };
 
-__device__ __forceinline__ void splat_lists_body(const SampleTable &st, int q, int e, uint32_t *fill, uint2 *cell,
-                                                 uint16_t *yidx, uint16_t *list, int *status, int blk,
-                                                 ListsShared &sh)
+// Class k's radius is r_const if that is positive, else (k + 1) / (2 q); eps
+// widens the windows; yidx may be null (no row-bucket counts).
+__device__ __forceinline__ void splat_lists_body(const SampleTable &st, int q, int e, float eps, float r_const,
+                                                 uint32_t *fill, uint2 *cell, uint16_t *yidx, uint16_t *list,
+                                                 int *status, int blk, ListsShared &sh)
 {
     // 64 cells per block, each split over 4 adjacent threads that take the
     // four quarters of the (X.y, p) order: the scan over the block in thread
@@ -839,10 +841,10 @@ __device__ __forceinline__ void splat_lists_body(const SampleTable &st, int q, i
     if (threadIdx.x <= kRowBuckets) sh.jb[threadIdx.x] = st.ybk[threadIdx.x];
     __syncthreads();
     const float m = 2.44140625e-4f;  // 2^-12
-    const float R = (float)(k + 1) / (float)(2 * q);
-    const float w = ((R + R) + (st.eps + st.eps)) + (1.0f / (float)q + (m + m));
-    const float lx = ((float)(c % q) / (float)q - R) - (st.eps + m);
-    const float ly = ((float)(c / q) / (float)q - R) - (st.eps + m);
+    const float R = r_const > 0.0f ? r_const : (float)(k + 1) / (float)(2 * q);
+    const float w = ((R + R) + (eps + eps)) + (1.0f / (float)q + (m + m));
+    const float lx = ((float)(c % q) / (float)q - R) - (eps + m);
+    const float ly = ((float)(c / q) / (float)q - R) - (eps + m);
     auto member = [&](int p) {
         const float2 f = s_f[p];
         float dx = f.x - lx, dy = f.y - ly;
@@ -877,17 +879,17 @@ __device__ __forceinline__ void splat_lists_body(const SampleTable &st, int q, i
         // the cell's entries before this quarter
         const int t0 = (int)threadIdx.x - quarter;
         uint32_t rel = s_scan[threadIdx.x] - n - (t0 > 0 ? s_scan[t0 - 1] : 0u);
-        uint16_t *yx = yidx + ((size_t)k * cells + c) * kRowBuckets;
+        uint16_t *yx = yidx ? yidx + ((size_t)k * cells + c) * kRowBuckets : nullptr;
         if (quarter == 0) {
             const uint32_t len = s_scan[threadIdx.x + 3] - (s_scan[threadIdx.x] - n);
             cell[(size_t)k * cells + c] = make_uint2(pos, len);
             // buckets that start past the last sample hold no entry
-            for (int b = 1; b <= kRowBuckets; ++b)
+            for (int b = 1; yx && b <= kRowBuckets; ++b)
                 if (sh.jb[b] == N) yx[b - 1] = (uint16_t)len;
         }
         // each other bucket count is written by the quarter holding the
         // bucket's first index: the cell's entries before that index
-        int b = 1;
+        int b = yx ? 1 : kRowBuckets + 1;
         while (b <= kRowBuckets && sh.jb[b] < p_lo) ++b;
         for (int i = p_lo; i < p_hi; ++i) {
             while (b <= kRowBuckets && sh.jb[b] <= i) {
@@ -907,7 +909,33 @@ __global__ __launch_bounds__(256) void splat_lists_kernel(SampleTable st, int q,
                                                           uint16_t *yidx, uint16_t *list, int *status)
 {
     __shared__ ListsShared sh;
-    splat_lists_body(st, q, e, fill, cell, yidx, list, status, blockIdx.x, sh);
+    splat_lists_body(st, q, e, st.eps, 0.0f, fill, cell, yidx, list, status, blockIdx.x, sh);
+}
+
+// The grain-wise kernel's lists (launch_grain_lists).  A grain's target is b +
+// X + 1/2 with b = bx - 1/2, its bounds() box of the splat's form around b + X,
+// so the same windows around frac(-b) hold its samples; eps is that kernel's:
+// C * 2^-20 + 2^-16, which covers the box's five roundings of at most C * 2^-24.
+__global__ __launch_bounds__(256) void grain_lists_kernel(SampleTable st, int q, float r_const, float c_base,
+                                                          uint32_t *fill, uint2 *cell, uint16_t *list, int *status)
+{
+    __shared__ ListsShared sh;
+    const float4 ext = *st.ext;
+    const float C = c_base + fmaxf(fmaxf(fabsf(ext.x), fabsf(ext.y)), fmaxf(fabsf(ext.z), fabsf(ext.w)));
+    const float eps = C * 9.5367431640625e-07f + 1.52587890625e-05f;
+    // room for every sample in every cell: span q
+    splat_lists_body(st, q, q, eps, r_const, fill, cell, nullptr, list, status, blockIdx.x, sh);
+}
+
+hipError_t launch_grain_lists(const SampleTable &st, int q, int classes, float r_const, float c_base, uint32_t *fill,
+                              uint2 *cell, uint16_t *list, int *status, hipStream_t s)
+{
+    if (q < 1 || q * q > 65536 || classes < 1 || st.n > 2048) return hipErrorInvalidValue;
+    const hipError_t err = launch_fill_u32(fill, classes, 0u, s);
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL(grain_lists_kernel, dim3(classes * ((q * q + 63) / 64)), dim3(256), 0, s, st, q, r_const, c_base,
+                       fill, cell, list, status);
+    return hipGetLastError();
 }
 
 // Batch sample tables: workgroup (x, p) sorts samples x * kBlock.. of plane p.
@@ -939,7 +967,7 @@ __global__ __launch_bounds__(256) void batch_splat_lists_kernel(BatchGen bg)
     const int p = find_run(bg.list_off, bg.n, blk);
     const BatchPlane &bp = cplane(bg.planes, p);
     const int4 lp = cload(bg.list_plan + p);
-    splat_lists_body(bp.st, lp.x, lp.z, cload(bg.list_fill + p), const_cast<uint2 *>(bp.st.cl_cell),
+    splat_lists_body(bp.st, lp.x, lp.z, bp.st.eps, 0.0f, cload(bg.list_fill + p), const_cast<uint2 *>(bp.st.cl_cell),
                      const_cast<uint16_t *>(bp.st.cl_yidx), const_cast<uint16_t *>(bp.st.cl_list), bp.a.status,
                      (int)(blk - cload(bg.list_off + p)), sh);
 }
@@ -1055,27 +1083,6 @@ __device__ __forceinline__ float lane_f(float v, int l)
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 __device__ __forceinline__ int lane_i(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
-
-// LDS locations as 32-bit LDS addresses: a bitset word's address held in a
-// sample record is used as it is, with no workgroup base added per hit
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-__device__ __forceinline__ uint32_t lds_addr(uint32_t *p)
-{
-    return (uint32_t)(uintptr_t)(lds_u32 *)p;
-}
-__device__ __forceinline__ void lds_or(uint32_t addr, uint32_t v)
-{
-    __hip_atomic_fetch_or((lds_u32 *)(uintptr_t)addr, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-// a * b + c for a, b < 2^24 with one full-rate v_mad_u32_u24 (b uniform).
-// Written out because the compiler turns two such terms into two products
-// and a three-way add.
-__device__ __forceinline__ uint32_t mad_u24(uint32_t a, uint32_t b, uint32_t c)
-{
-    uint32_t d;
-    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(b), "v"(c));
-    return d;
-}
 
 // One output tile of one plane: the body of the single-plane kernel and of the
 // persistent batch kernel (which therefore give identical planes).  lds is the
@@ -1413,26 +1420,11 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
         const unsigned long long lmask = LISTS ? __ballot(walks) : 0ull;
         if (LISTS && lmask) {
             // The listed grains' candidate lists, concatenated in lane order,
-            // are walked 64 entries a step.  The grains are numbered by their
-            // place in that order (their rank), and the stream's entry e
-            // belongs to the grain whose rank is the number of lists that end
-            // before e: a set bit per list end (its last entry) in a bitset
-            // of the batch's entries, so that a step's owners are a count of
-            // the set bits below each lane (two v_mbcnt) on top of the count
-            // before the step.  (Taking the owners from a scalar loop over
-            // the grains that start within the step was half of the walk's
-            // scalar instructions: 13.6 -> 11.2 ms per 4K RGB frame.)
+            // are walked 64 entries a step (walk_lists).
             const uint32_t fl = walks ? (uint32_t)len : 0u;
             const uint32_t incl = wave_inclusive_sum(fl);
             const int total = lane_i((int)incl, 63);
             const int excl = (int)(incl - fl);
-            // Entry e of the stream is list entry dl + e of its owner grain,
-            // dl = p0 - excl >= -excl > -total.  A step from s loads entry
-            // s + min(lane, total - 1 - s), and the steps of a batch that
-            // start past the stream have s < total + 64 (kWalkStage - 1), so
-            // biased by bias = total + 64 kWalkStage, the lane's part
-            // dlb + min(lane, total - 1 - s) is positive: a valid unsigned
-            // 32-bit offset from the batch's base.
             const int bias = total + 64 * kWalkStage;
             // one record per listed grain, in rank order: centre, r^2, dlb
             // (the wave's LDS accesses run in order, so no barrier is needed)
@@ -1443,72 +1435,31 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
                 queue[rank] = pk;  // the cells, for the window checks (the queue is empty here)
             }
             const unsigned char *grec = reinterpret_cast<const unsigned char *>(&s_grec[wid][0]);
-            uint32_t *ends = s_ends[wid];
             // the last list's end is left out: lanes past the stream count as
             // its entries
             const int my_end = walks && (int)incl != total ? (int)incl - 1 : -1;
-            uint32_t before = 0;  // list ends before the step
-            // STAGE steps from entry sb: their owners first, then all their
-            // list loads in flight together, then their tests: one global
-            // latency per batch of steps instead of one per step.  Lanes past
-            // the stream read its last entry (the stream's last pair again:
-            // its bit is ORed twice, which changes nothing).  A load takes a
-            // base in SGPRs (the batch's first entry, less the bias), a
-            // 32-bit byte offset in one VGPR and the step's 128 bytes as its
-            // immediate offset: no 64-bit address arithmetic.
-            auto batch = [&](auto stage, auto checked, int sb) {
-                constexpr int STAGE = decltype(stage)::value;
-                constexpr bool CHECK = decltype(checked)::value;
-                if (lane < 2 * STAGE) ends[lane] = 0u;
-                __builtin_amdgcn_wave_barrier();
-                const int rel = my_end - sb;
-                if ((unsigned)rel < 64u * STAGE && my_end >= 0) lds_or(lds_addr(ends + (rel >> 5)), 1u << (rel & 31));
-                __builtin_amdgcn_wave_barrier();
-                const unsigned char *lbb =
-                    reinterpret_cast<const unsigned char *>(st.cl_list) + 2 * ((long long)sb - bias);
-                uint32_t own[STAGE], pn[STAGE];
-#pragma unroll
-                for (int i = 0; i < STAGE; ++i) {
-                    const uint2 e = *reinterpret_cast<const uint2 *>(ends + 2 * i);
-                    own[i] = __builtin_amdgcn_mbcnt_hi(e.y, __builtin_amdgcn_mbcnt_lo(e.x, before)) << 4;
-                    before += __popc(e.x) + __popc(e.y);
-                }
-#pragma unroll
-                for (int i = 0; i < STAGE; ++i) {
-                    const uint32_t pos = *reinterpret_cast<const uint32_t *>(grec + own[i] + 12) +
-                                         (uint32_t)min(lane, total - 1 - (sb + 64 * i));
-                    pn[i] = (uint32_t)*reinterpret_cast<const uint16_t *>(lbb + 128 * i + (pos << 1));
-                }
-#pragma unroll
-                for (int i = 0; i < STAGE; ++i) {
-                    if (sb + 64 * i >= total) break;
-                    // the owner grain's record and the sample's, which the
-                    // entry is the byte offset of
-                    const float4 gr = *reinterpret_cast<const float4 *>(grec + own[i]);
-                    const float4 r = rec_at(pn[i]);
-                    // both reads issue before the test's branches (as in the
-                    // per-grain walk)
-                    asm volatile("" ::"v"(r.x), "v"(r.y), "v"(r.z), "v"(r.w));
-                    // A passing point at most safe_r from the centre in both
-                    // axes has the grain's cell in its window (splat_bounds);
-                    // beyond, the reference's window test decides.
-                    test(true, r, gr.x, gr.y, gr.z, [&](float dx, float dy, float xg, float yg) -> bool {
-                        if (!CHECK || fmaxf(fabsf(dx), fabsf(dy)) <= safe_r) return true;
-                        return in_window_fast(queue[own[i] >> 4], xg, yg);
-                    });
-                }
-                __builtin_amdgcn_wave_barrier();
-            };
-            // whole batches, then a shorter one where it holds the rest: the
-            // lists of a small N are a few entries each
             auto walk = [&](auto checked) {
-                int sb = 0;
-                for (; total - sb > 64 * (kWalkStage / 2); sb += 64 * kWalkStage)
-                    batch(std::integral_constant<int, kWalkStage>(), checked, sb);
-                if (total - sb > 64 * (kWalkStage / 4))
-                    batch(std::integral_constant<int, kWalkStage / 2>(), checked, sb);
-                else if (total - sb > 0)
-                    batch(std::integral_constant<int, kWalkStage / 4>(), checked, sb);
+                constexpr bool CHECK = decltype(checked)::value;
+                walk_lists<kWalkStage>(total, bias, my_end, s_ends[wid], grec,
+                                       reinterpret_cast<const unsigned char *>(st.cl_list),
+                                       [&](uint32_t own, uint32_t entry) {
+                                           // the owner grain's record and the sample's, which the
+                                           // entry is the byte offset of
+                                           const float4 gr = *reinterpret_cast<const float4 *>(grec + own);
+                                           const float4 r = rec_at(entry);
+                                           // both reads issue before the test's branches (as in
+                                           // the per-grain walk)
+                                           asm volatile("" ::"v"(r.x), "v"(r.y), "v"(r.z), "v"(r.w));
+                                           // A passing point at most safe_r from the centre in
+                                           // both axes has the grain's cell in its window
+                                           // (splat_bounds); beyond, the reference's window test
+                                           // decides.
+                                           test(true, r, gr.x, gr.y, gr.z,
+                                                [&](float dx, float dy, float xg, float yg) -> bool {
+                                                    if (!CHECK || fmaxf(fabsf(dx), fabsf(dy)) <= safe_r) return true;
+                                                    return in_window_fast(queue[own >> 4], xg, yg);
+                                                });
+                                       });
             };
             if (check) walk(std::true_type());
             else walk(std::false_type());
@@ -1625,7 +1576,7 @@ __global__ __launch_bounds__(BLOCK, 6) void splat_hbm_kernel(PixelArgs a, PixGeo
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ uint32_t s_queue[BLOCK / 64][kQueueCap];
     __shared__ float4 s_grec[BLOCK / 64][64];
-    __shared__ uint32_t s_ends[BLOCK / 64][2 * kWalkStage];
+    __shared__ __align__(16) uint32_t s_ends[BLOCK / 64][2 * kWalkStage];
     const int tile = a.tile_list ? a.tile_list[blockIdx.x] : (int)blockIdx.x;
     splat_tile<BLOCK, true, true>(a, geo, st, bin_start, grains, tile, lds, s_queue, s_grec, s_ends);
 }
@@ -1640,7 +1591,7 @@ __global__ __launch_bounds__(BLOCK, 6) void splat_batch_kernel(const BatchPlane 
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ uint32_t s_queue[BLOCK / 64][kQueueCap];
     __shared__ float4 s_grec[BLOCK / 64][64];
-    __shared__ uint32_t s_ends[BLOCK / 64][2 * kWalkStage];
+    __shared__ __align__(16) uint32_t s_ends[BLOCK / 64][2 * kWalkStage];
     __shared__ int s_item;
     for (;;) {
         __syncthreads();

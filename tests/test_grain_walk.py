@@ -1,0 +1,116 @@
+"""The grain-wise kernel's candidate lists and its narrow test
+(fg_grainwise.hip, grain_lists_kernel), on the CPU in f32 and on the GPU
+against the oracle."""
+import numpy as np
+import pytest
+
+f32 = np.float32
+
+
+def members(fx, fy, qa, qb, q, R, eps):
+    """splat_lists_body's membership, in its order of operations."""
+    m = f32(2.0 ** -12)
+    w = f32(f32(f32(R + R) + f32(eps + eps)) + f32(f32(f32(1) / f32(q)) + f32(m + m)))
+    dx = (fx - f32(f32(f32(f32(qa) / f32(q)) - R) - f32(eps + m))).astype(f32)
+    dy = (fy - f32(f32(f32(f32(qb) / f32(q)) - R) - f32(eps + m))).astype(f32)
+    dx = (dx - np.floor(dx)).astype(f32)
+    dy = (dy - np.floor(dy)).astype(f32)
+    return (dx <= w) & (dy <= w)
+
+
+def box(t, R):
+    """bounds() of src/grainwise.rs:126-142 before its clamp."""
+    return (np.ceil(((t - R).astype(f32) - f32(0.5)).astype(f32)),
+            np.floor(((t + R).astype(f32) - f32(0.5)).astype(f32)))
+
+
+@pytest.mark.parametrize("side,N,sd,const", [(1280, 64, 0.8, False), (4096, 128, 0.8, True), (4096, 300, 2.0, False),
+                                             (16384, 100, 0.8, True), (64, 2048, 0.4, False)])
+def test_lists_and_narrow_test_find_every_hit(side, N, sd, const):
+    """Every (sample, pixel) that the reference tests (in its box) and that
+    passes its disk test is in the grain's list, is pixel floor(t), and the
+    box need not be looked at where |dx|, |dy| <= R - C 2^-21."""
+    rng = np.random.default_rng(side + N)
+    X = rng.normal(0, sd, size=(N, 2)).astype(f32)
+    fx, fy = ((X[:, i] - np.floor(X[:, i])).astype(f32) for i in (0, 1))
+    rmax = f32(0.45 if const else 0.6)
+    C = f32(f32(side) + np.abs(X).max() + rmax + f32(8))
+    eps = f32(f32(C * f32(2.0 ** -20)) + f32(2.0 ** -16))
+    edge = f32(C * f32(2.0 ** -21))
+    narrow_r = f32(f32(0.5) - f32(eps + eps))
+    hits = rim = 0
+    for i in range(2500):
+        R = rmax if const and i % 2 else f32(rng.uniform(0.002, float(rmax)))
+        if i % 5 == 0 and not const:
+            R = f32(int(rng.integers(1, 32)) / 64 + rng.choice([-1e-6, 0, 1e-6]))  # class edges
+        if not R < narrow_r:
+            continue
+        b = rng.uniform(-4, side + 4, size=2).astype(f32)
+        if i % 3 == 0:  # targets of sample 0 at the rim of a pixel's disk
+            b = (np.floor(b) + f32(0.5) + rng.choice([-1, 1], 2) * R - X[0] +
+                 rng.uniform(-2, 2, 2) * 2.0 ** -12).astype(f32)
+        q = 64 if const else 32
+        Rl = R if const else f32((int(R * f32(64)) + 1) / 64)
+        n = (f32(0.5) - b).astype(f32)
+        f = (n - np.floor(n)).astype(f32)
+        qa, qb = (min(int(f32(v * f32(q))), q - 1) for v in f)
+        sel = members(fx, fy, qa, qb, q, Rl, eps)
+        t = (b + X).astype(f32)
+        xl, xh = box(t[:, 0], R)
+        yl, yh = box(t[:, 1], R)
+        for ox in (-1, 0, 1):
+            for oy in (-1, 0, 1):
+                px, py = np.floor(t[:, 0]) + ox, np.floor(t[:, 1]) + oy
+                dx = ((px + f32(0.5)).astype(f32) - t[:, 0]).astype(f32)
+                dy = ((py + f32(0.5)).astype(f32) - t[:, 1]).astype(f32)
+                disk = ((dx * dx).astype(f32) + (dy * dy).astype(f32)).astype(f32) <= f32(R * R)
+                inbox = (xl <= px) & (px <= xh) & (yl <= py) & (py <= yh)
+                ref = disk & inbox
+                assert not np.any(ref & ~sel), (i, float(R))
+                if ox or oy:
+                    assert not np.any(disk)
+                    continue
+                inner = disk & (np.maximum(np.abs(dx), np.abs(dy)) <= f32(R - edge))
+                assert not np.any(inner & ~inbox)
+                hits += int(ref.sum())
+                rim += int((disk & ~inner).sum())
+    assert hits > 0 and rim > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("r_out,sd", [(0.01, 0.0), (0.2, 0.0), (0.449, 0.0), (0.4501, 0.0), (0.51, 0.0), (1.2, 0.0),
+                                      (0.05, 0.03), (0.2, 0.15), (0.45, 0.1), (0.9, 0.5)])
+def test_planes_across_the_list_limits(hip_ctx, oracle, r_out, sd):
+    """Constant output radii on both sides of the lists' limits and lognormal
+    laws with narrow, wide and mixed grains, for several zooms and sample
+    counts."""
+    from film_grain_amd import synth
+    from tests import fgcases
+    rng = np.random.default_rng(int(r_out * 1e4))
+    for zoom, n in [(0.5, 300), (1.0, 1), (2.0, 64), (3.0, 2048)]:
+        w, h = 27, 22
+        grains = w * h * 1.4 / (np.pi * (r_out / zoom) ** 2)
+        while n > 1 and (round(w * zoom) * round(h * zoom) * n > 2_000_000 or grains * n > 5e8):
+            n //= 2
+        u = synth.sinusoid_field(w, h, int(rng.integers(0, 1 << 30)), n_waves=3)
+        case = fgcases.build_case(oracle, f"gl_{r_out}_{zoom}", u, r_out / zoom, sd / zoom,
+                                  "lognorm" if sd else "const", zoom=zoom, n_samples=n,
+                                  seed=int(rng.integers(0, 1 << 40)))
+        want = oracle.render_grainwise(case.plane, case.lam, case.offsets)
+        got = hip_ctx.render_host("grain", case.desc, case.lam, case.offsets)
+        assert int(np.sum(got != want)) == 0, (zoom, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sd", [0.0, 0.02])
+def test_thin_long_plane(hip_ctx, oracle, sd):
+    """Coordinates up to 6000 output pixels: a widening of 6e-3 and a rim of
+    3e-3 around radii of 0.04 and up."""
+    from film_grain_amd import synth
+    from tests import fgcases
+    u = synth.sinusoid_field(3000, 3, 5, n_waves=3)
+    case = fgcases.build_case(oracle, "thin", u, 0.04, sd, "lognorm" if sd else "const", zoom=2.0, n_samples=24,
+                              seed=77)
+    want = oracle.render_grainwise(case.plane, case.lam, case.offsets)
+    got = hip_ctx.render_host("grain", case.desc, case.lam, case.offsets)
+    assert int(np.sum(got != want)) == 0
