@@ -70,9 +70,6 @@ struct fg_ctx {
     DevBuf cells;             // candidate lists: grain-wise constant radius, splat direct test
     DevBuf scale_state;       // budget scale search: bracket, flag, probe sums
     DevBuf frame_io;          // frames from host memory: RGB in, offsets, 8-bit RGB out, planes out
-    std::vector<int> level_n;
-    std::vector<fg::SampleTable> level_tables;
-
     hipEvent_t scratch_done = nullptr;  // recorded after the last kernel that reads the scratch
     bool scratch_pending = false;
     // optional kernel timing: start, generation done, test kernel start, end
@@ -594,17 +591,79 @@ ListPlan list_plan(const fg::PixelArgs &a, float eps)
     return lp;
 }
 
-// Builds table t's lists in `at` (lp.bytes(t.n) bytes) and points t at them.
-hipError_t build_lists(const ListPlan &lp, fg::SampleTable &t, unsigned char *at, int *status, hipStream_t s)
+// Points table t at its lists in `at` (lp.bytes(t.n) bytes); returns their
+// counters.
+uint32_t *place_lists(const ListPlan &lp, fg::SampleTable &t, unsigned char *at)
 {
-    uint32_t *fill = reinterpret_cast<uint32_t *>(at);
-    uint2 *cs = reinterpret_cast<uint2 *>(at + 256);
-    uint16_t *yx = reinterpret_cast<uint16_t *>(cs + (size_t)lp.classes * lp.q * lp.q);
-    uint16_t *cl = yx + (size_t)lp.classes * lp.q * lp.q * fg::kRowBuckets;
-    t.cl_cell = cs;
-    t.cl_yidx = yx;
-    t.cl_list = cl;
-    return fg::launch_splat_lists(t, lp.q, lp.classes, lp.ew, fill, cs, yx, cl, status, s);
+    const size_t cells = (size_t)lp.classes * lp.q * lp.q;
+    t.cl_cell = reinterpret_cast<uint2 *>(at + 256);
+    t.cl_yidx = reinterpret_cast<uint16_t *>(at + 256 + cells * sizeof(uint2));
+    t.cl_list = t.cl_yidx + cells * fg::kRowBuckets;
+    return reinterpret_cast<uint32_t *>(at);
+}
+
+// The sample tables of one render and their lists: the levels' sample counts,
+// and the set's device launches after its buffers are placed.
+struct Tables {
+    fg::LevelSet set{};
+    ListPlan lp;
+    size_t list_bytes = 0;   // all levels' lists; 0: no lists
+    size_t level_bytes = 0;  // records and the tables of all levels but the last
+    bool lists() const { return list_bytes > 0 && list_bytes < ((size_t)1 << 32); }
+};
+
+Tables plan_tables(const fg::PixelArgs &a, float eps, float safe_r, bool levels)
+{
+    Tables t;
+    fg::LevelSet &set = t.set;
+    if (levels)
+        for (int l = 16; l < a.n_samples; l *= 2) set.level_n[set.n++] = l;
+    set.level_n[set.n++] = a.n_samples;
+    t.lp = list_plan(a, eps);
+    set.classes = t.lp.classes;
+    t.level_bytes = (sizeof(fg::SampleTable) * set.n + 255) & ~(size_t)255;
+    for (int l = 0; l < set.n; ++l) {
+        const int n = set.level_n[l];
+        t.list_bytes += t.lp.bytes(n);
+        if (l + 1 < set.n) t.level_bytes += (fg::sample_table_bytes(n, sample_buckets((uint32_t)n)) + 255) & ~(size_t)255;
+    }
+    set.full.eps = eps;
+    set.full.safe_r = safe_r;
+    return t;
+}
+
+// Places the tables: the full one in `samples`, the records and the smaller
+// ones in `levels` (t.level_bytes), the lists in `lists` (t.list_bytes; null:
+// none).
+void place_tables(Tables &t, void *samples, void *levels, void *lists)
+{
+    fg::LevelSet &set = t.set;
+    const int N = set.level_n[set.n - 1];
+    fg::sample_table_layout(samples, N, sample_buckets((uint32_t)N), &set.full);
+    unsigned char *lv = static_cast<unsigned char *>(levels), *ls = static_cast<unsigned char *>(lists);
+    set.store = reinterpret_cast<fg::SampleTable *>(lv);
+    lv += (sizeof(fg::SampleTable) * set.n + 255) & ~(size_t)255;
+    for (int l = 0; l < set.n; ++l) {
+        const int n = set.level_n[l], q = sample_buckets((uint32_t)n);
+        fg::SampleTable &st = set.t[l];
+        st = set.full;  // bounds of the whole offset set hold for every prefix
+        if (l + 1 < set.n) {
+            fg::sample_table_layout(lv, n, q, &st);
+            lv += (fg::sample_table_bytes(n, q) + 255) & ~(size_t)255;
+        }
+        if (ls && t.lp.bytes(n) > 0) {
+            set.fill[l] = place_lists(t.lp, st, ls);
+            ls += t.lp.bytes(n);
+        }
+    }
+}
+
+// Every table (full is ranked before) and its lists.
+hipError_t launch_tables(const Tables &t, bool lists, int *status, hipStream_t s)
+{
+    hipError_t e = fg::launch_sample_levels(t.set, s);
+    if (e == hipSuccess && lists) e = fg::launch_splat_lists(t.set, t.lp.q, t.lp.ew, status, s);
+    return e;
 }
 
 // Where a render's scratch comes from: the context's grow-only buffers
@@ -732,12 +791,25 @@ int run_pixel_hbm(fg_ctx *ctx, fg::PixelArgs &a, const fg::PixGeom &g, const flo
     // the context's buffers are shared by its calls: wait for the previous
     // user (an arena's callers are told that overlapping calls race)
     if (!src.arena && (rc = scratch_acquire(ctx, what)) != FG_OK) return rc;
-    const int q = sample_buckets((uint32_t)a.n_samples);
-    void *samples_p;
-    if ((rc = scratch_get(ctx, src, ctx->samples, fg::sample_table_bytes(a.n_samples, q), &samples_p, what)) != FG_OK)
+    float eps, safe_r;
+    splat_bounds(a, g, range, &eps, &safe_r);
+    Tables tab = plan_tables(a, eps, safe_r, a.budget != nullptr);
+    void *samples_p, *levels_p, *lists_p = nullptr;
+    const size_t tile_level_b = a.budget ? (size_t)a.n_tiles : 0;
+    if ((rc = scratch_get(ctx, src, ctx->samples,
+                          fg::sample_table_bytes(a.n_samples, sample_buckets((uint32_t)a.n_samples)), &samples_p,
+                          what)) != FG_OK)
         return rc;
-    fg::SampleTable st{};
-    splat_bounds(a, g, range, &st.eps, &st.safe_r);
+    if ((rc = scratch_get(ctx, src, ctx->levels, tab.level_bytes + tile_level_b, &levels_p, what)) != FG_OK) return rc;
+    if (tab.lists()) {
+        if ((rc = scratch_get(ctx, src, ctx->cells, tab.list_bytes, &lists_p, what)) != FG_OK) return rc;
+        a.cl_q = tab.lp.q;
+        a.cl_classes = tab.lp.classes;
+        a.cl_inv_dz = (float)(2 * tab.lp.q);
+    }
+    place_tables(tab, samples_p, levels_p, lists_p);
+    const fg::SampleTable &st = tab.set.t[tab.set.n - 1];
+    a.level_tables = tab.set.store;
     mark(ctx, 0, s);
     HbmGen gen;
     if ((rc = hbm_generate(ctx, src, a, g, dist_kind, s, &gen, pre)) != FG_OK) return rc;
@@ -758,82 +830,15 @@ int run_pixel_hbm(fg_ctx *ctx, fg::PixelArgs &a, const fg::PixGeom &g, const flo
         order.ids = reinterpret_cast<int *>(p + (size_t)a.n_tiles * 8);
         order.order = reinterpret_cast<int *>(p + (size_t)a.n_tiles * 12);
     }
-    e = fg::launch_sample_table(a.offs, a.n_samples, a.zoom, q, samples_p, &st, s);
-    // candidate lists for the direct test, one set per sample table
-    const ListPlan lp = list_plan(a, st.eps);
-    // (a fixed-N render touches no host container: the allocation-free
-    // entry point takes this path)
-    std::vector<int> &ln = ctx->level_n;
-    size_t lists_total = lp.bytes(a.n_samples);
-    if (a.budget) {
-        ln.clear();
-        for (int l = 16; l < a.n_samples; l *= 2) ln.push_back(l);
-        ln.push_back(a.n_samples);
-        lists_total = 0;
-        for (int l : ln) lists_total += lp.bytes(l);
-    }
-    unsigned char *lists_at = nullptr;
-    if (lists_total > 0 && lists_total < ((size_t)1 << 32)) {
-        void *cells_p;
-        if ((rc = scratch_get(ctx, src, ctx->cells, lists_total, &cells_p, what)) != FG_OK) return rc;
-        lists_at = static_cast<unsigned char *>(cells_p);
-        a.cl_q = lp.q;
-        a.cl_classes = lp.classes;
-        a.cl_inv_dz = (float)(2 * lp.q);
-    }
-    auto build_lists_for = [&](fg::SampleTable &t) -> hipError_t {
-        const size_t b = lp.bytes(t.n);
-        if (a.cl_q == 0 || b == 0) return hipSuccess;
-        const hipError_t err = build_lists(lp, t, lists_at, a.status, s);
-        lists_at += b;
-        return err;
-    };
-    if (e == hipSuccess && !a.budget) {
-        // the splat kernel reads its one table from device memory
-        void *levels_p;
-        if ((rc = scratch_get(ctx, src, ctx->levels, 256, &levels_p, what)) != FG_OK) return rc;
-        fg::SampleTable *d_table = static_cast<fg::SampleTable *>(levels_p);
-        e = build_lists_for(st);
-        if (e == hipSuccess) e = fg::launch_store_table(st, d_table, s);
-        a.level_tables = d_table;
-    }
+    // one sample table per level (the first 16, 32, ... samples, then all;
+    // all alone without budgets), their lists, and with budgets each tile's
+    // level
+    e = fg::launch_sample_rank(a.offs, a.zoom, tab.set.full, s);
+    if (e == hipSuccess) e = launch_tables(tab, lists_p != nullptr, a.status, s);
     if (e == hipSuccess && a.budget) {
-        // adaptive sampling: one sample table per level (the first 16, 32,
-        // ... samples, then all), and each tile's level
-        const int nl = (int)ln.size();
-        size_t bytes = 0;
-        for (int l : ln) bytes += (fg::sample_table_bytes(l, sample_buckets((uint32_t)l)) + 255) & ~(size_t)255;
-        const size_t head = 256 + (((size_t)nl * sizeof(fg::SampleTable) + 255) & ~(size_t)255);
-        void *levels_p;
-        if ((rc = scratch_get(ctx, src, ctx->levels, head + bytes + (size_t)a.n_tiles, &levels_p, what)) != FG_OK)
-            return rc;
-        unsigned char *base = static_cast<unsigned char *>(levels_p);
-        int *d_level_n = reinterpret_cast<int *>(base);
-        fg::SampleTable *d_tables = reinterpret_cast<fg::SampleTable *>(base + 256);
-        unsigned char *p = base + head;
-        ctx->level_tables.assign(nl, fg::SampleTable{});
-        for (int i = 0; i < nl && e == hipSuccess; ++i) {
-            fg::SampleTable &lt = ctx->level_tables[i];
-            if (ln[i] == a.n_samples) {
-                lt = st;  // the last level is the full table
-            } else {
-                e = fg::launch_sample_prefix(st, ln[i], sample_buckets((uint32_t)ln[i]), p, &lt, s);
-                lt.eps = st.eps;  // bounds of the whole offset set hold for every prefix
-                lt.safe_r = st.safe_r;
-            }
-            if (e == hipSuccess) e = build_lists_for(lt);
-            p += (fg::sample_table_bytes(ln[i], sample_buckets((uint32_t)ln[i])) + 255) & ~(size_t)255;
-        }
-        uint8_t *d_tile_level = p;
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(d_tables, ctx->level_tables.data(), sizeof(fg::SampleTable) * nl,
-                               hipMemcpyHostToDevice, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(d_level_n, ln.data(), sizeof(int) * nl, hipMemcpyHostToDevice, s);
-        a.level_tables = d_tables;
-        a.tile_level = d_tile_level;
-        if (e == hipSuccess) e = fg::launch_tile_levels(a, d_level_n, nl, d_tile_level, s);
-        // the host arrays above must outlive the copies
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        uint8_t *tile_level = static_cast<uint8_t *>(levels_p) + tab.level_bytes;
+        a.tile_level = tile_level;
+        e = fg::launch_tile_levels(a, tab.set, tile_level, s);
     }
     if (e == hipSuccess) e = fg::launch_pixel_tile_weights(a, g, start, order.w, order.ids, s);
     if (e == hipSuccess)
@@ -1020,11 +1025,10 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
     hipError_t e = fg::scan_bins(nullptr, &scan_bytes, nullptr, nullptr, (int)(nbins + 1), s);
     if (e != hipSuccess) return hip_error(ctx, e, what);
     const int q = sample_buckets((uint32_t)d->n_samples);
-    fg::SampleTable st{};
-    splat_bounds(a[0], geom, range, &st.eps, &st.safe_r);
-    const ListPlan lp = list_plan(a[0], st.eps);
-    const size_t lists_total = lp.bytes((int)d->n_samples);
-    const bool lists = lists_total > 0 && lists_total < ((size_t)1 << 32);
+    float eps, safe_r;
+    splat_bounds(a[0], geom, range, &eps, &safe_r);
+    Tables tab = plan_tables(a[0], eps, safe_r, false);
+    const bool lists = tab.lists();
     // the persistent splat's plane records, (plane, tile) items, their
     // weights and the item counter
     const int n_items = n * a[0].n_tiles;
@@ -1033,8 +1037,9 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
     if ((rc = ensure_bytes(ctx, ctx->scan_temp, scan_bytes, what)) != FG_OK) return rc;
     if ((rc = ensure_bytes(ctx, ctx->tiles, rec_b + items_b + w_b + 256, what)) != FG_OK) return rc;
     if ((rc = ensure_bytes(ctx, ctx->samples, fg::sample_table_bytes((int)d->n_samples, q), what)) != FG_OK) return rc;
-    if ((rc = ensure_bytes(ctx, ctx->levels, 256, what)) != FG_OK) return rc;
-    if (lists && (rc = ensure_bytes(ctx, ctx->cells, lists_total, what)) != FG_OK) return rc;
+    if ((rc = ensure_bytes(ctx, ctx->levels, tab.level_bytes, what)) != FG_OK) return rc;
+    if (lists && (rc = ensure_bytes(ctx, ctx->cells, tab.list_bytes, what)) != FG_OK) return rc;
+    place_tables(tab, ctx->samples.p, ctx->levels.p, lists ? ctx->cells.p : nullptr);
     mark(ctx, 0, s);
     for (int i = 0; i < n && e == hipSuccess; ++i) e = fg::launch_threshold(a[i], pre[i].T, s);
     if (e == hipSuccess) e = fg::launch_bin_count_planes(a[0], geom, fp, n, s);
@@ -1059,24 +1064,21 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
     }
     if ((rc = ensure_bytes(ctx, ctx->grains, std::max<size_t>(gsum, 1) * sizeof(float4), what)) != FG_OK) return rc;
     float4 *grains = static_cast<float4 *>(ctx->grains.p);
-    // one sample table and its candidate lists, which the splat reads from
-    // device memory
-    e = fg::launch_sample_table(a[0].offs, a[0].n_samples, a[0].zoom, q, ctx->samples.p, &st, s);
-    if (e == hipSuccess && lists) e = build_lists(lp, st, static_cast<unsigned char *>(ctx->cells.p), a[0].status, s);
-    fg::SampleTable *d_table = static_cast<fg::SampleTable *>(ctx->levels.p);
-    if (e == hipSuccess) e = fg::launch_store_table(st, d_table, s);
+    // one sample table and its candidate lists
+    e = fg::launch_sample_rank(a[0].offs, a[0].zoom, tab.set.full, s);
+    if (e == hipSuccess) e = launch_tables(tab, lists, a[0].status, s);
     fg::FramePlaneRecords rec{};
     for (int i = 0; i < n && e == hipSuccess; ++i) {
         e = fg::launch_bin_grains(a[i], geom, kind, pre[i].T, start[i], pre[i].mask, grains + goff[i], s);
         if (lists) {
-            a[i].cl_q = lp.q;
-            a[i].cl_classes = lp.classes;
-            a[i].cl_inv_dz = (float)(2 * lp.q);
+            a[i].cl_q = tab.lp.q;
+            a[i].cl_classes = tab.lp.classes;
+            a[i].cl_inv_dz = (float)(2 * tab.lp.q);
         }
         fg::BatchPlane &bp = rec.p[i];
         bp.a = a[i];
         bp.geo = geom;
-        bp.st = st;
+        bp.st = tab.set.t[0];
         bp.bin_start = start[i];
         bp.grains = grains + goff[i];
         bp.item_base = (long long)i * a[i].n_tiles;
@@ -1210,9 +1212,14 @@ int do_grainwise(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lambda, con
         a.pix_q = reinterpret_cast<uint32_t *>(ps + npx * 32);
         TileOrder order;
         if ((rc = tile_order_prepare(ctx, a.n_tiles, &order, s, what)) != FG_OK) return rc;
-        fg::SampleTable st{};
+        fg::LevelSet set{};
+        fg::sample_table_layout(ctx->samples.p, a.n_samples, q, &set.full);
+        const fg::SampleTable &st = set.full;
+        set.t[0] = set.full;
+        set.level_n[0] = a.n_samples;
+        set.n = 1;
         mark(ctx, 0, s);
-        hipError_t e = fg::launch_sample_table(a.offs, a.n_samples, 1.0f, q, ctx->samples.p, &st, s);
+        hipError_t e = fg::launch_sample_rank(a.offs, 1.0f, st, s);
         // Candidate lists for narrow grains, about N (2R + 1/Q)^2 samples each
         // instead of a run of N (2R + 1/Q): one class for a constant radius
         // below 0.45 output pixels (the kernel's narrow limit is 1/2 less its
@@ -1232,13 +1239,18 @@ int do_grainwise(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lambda, con
             uint2 *cell = reinterpret_cast<uint2 *>(cb + 256);
             uint16_t *list = reinterpret_cast<uint16_t *>(cell + cells);
             const float c_base = (float)std::max(a.out_w, a.out_h) + a.r_out_max + 8.0f;
+            set.fill[0] = reinterpret_cast<uint32_t *>(cb);
+            set.classes = classes;
+            if (e == hipSuccess) e = fg::launch_sample_levels(set, s);
             if (e == hipSuccess)
-                e = fg::launch_grain_lists(st, cq, classes, lognorm ? 0.0f : r_out, c_base,
-                                           reinterpret_cast<uint32_t *>(cb), cell, list, a.status, s);
+                e = fg::launch_grain_lists(st, cq, classes, lognorm ? 0.0f : r_out, c_base, set.fill[0], cell, list,
+                                           a.status, s);
             a.gl_cell = cell;
             a.gl_list = list;
             a.gl_classes = classes;
             a.r_list = r_out;
+        } else if (e == hipSuccess) {
+            e = fg::launch_sample_levels(set, s);
         }
         if (e == hipSuccess) e = fg::launch_pixel_state(a, s);
         if (e == hipSuccess) e = fg::launch_grain_tile_weights(a, st, order.w, order.ids, s);
@@ -1619,7 +1631,7 @@ int batch_gen_setup(fg_batch *b, const char *what, hipStream_t s)
     g.total_bins = bins[n];
     g.draw_chunk = fg::draw_chunk(g.total_bins);
     g.list_blocks = lists[n];
-    g.sort_blocks = (max_samples + fg::kBlock - 1) / fg::kBlock;
+    g.rank_blocks = fg::rank_blocks(max_samples);
     if (g.thr_blocks > 0x7fffffffLL || g.list_blocks > 0x7fffffffLL) return set_error(b->ctx, FG_EINVAL, "batch too large");
     // planes by radius distribution, each with the first draw chunk of its
     // bins in that sequence

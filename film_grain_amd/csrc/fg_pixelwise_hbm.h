@@ -60,26 +60,35 @@ constexpr int kRowBuckets = 16;
 
 // Bytes of the device buffer behind a SampleTable for n samples.
 size_t sample_table_bytes(int n, int qbuckets);
-// Builds the table in `buf` (sample_table_bytes bytes) and points *t at it.
-hipError_t launch_sample_table(const float2 *offs, int n, float zoom, int qbuckets, void *buf, SampleTable *t,
-                               hipStream_t s);
-// The table of the first n samples of `full` (full.n <= 2048), built by
-// filtering full's order instead of sorting again.
-hipError_t launch_sample_prefix(const SampleTable &full, int n, int qbuckets, void *buf, SampleTable *t,
-                                hipStream_t s);
+// The sample tables of one offset set: `full`, of all its samples, and the
+// tables of its first samples that an adaptive render's levels use (t[n - 1]
+// is full, the only one of a fixed-N render), with the counters of their
+// candidate lists (cleared with the tables; nullptr: no lists) and where the
+// table records go in device memory (nullptr: nowhere).
+constexpr int kMaxLevels = 8;  // 16, 32, ..., 1024 samples and all (at most 2048)
+struct LevelSet {
+    SampleTable full;
+    SampleTable t[kMaxLevels];
+    uint32_t *fill[kMaxLevels];
+    SampleTable *store;
+    int n, classes;
+    int level_n[kMaxLevels];  // samples per level, ascending
+};
+// Ranks t.n <= 2048 samples into t (laid out by sample_table_layout): its
+// sorted arrays and its y order.
+hipError_t launch_sample_rank(const float2 *offs, float zoom, const SampleTable &t, hipStream_t s);
+// The rest of every table of the set (full ranked before), in one launch.
+hipError_t launch_sample_levels(const LevelSet &set, hipStream_t s);
 
-// Candidate lists of the HBM splat (PixelArgs::cl_*): q * q cells per class,
-// class k of radius (k + 1) / (2 q).  e is an integer >= (2 st.eps + 2^-11)
-// q; list needs splat_lists_entries(q, classes, e, st.n) entries, cell
-// classes * q * q (start, length) pairs, yidx classes * q * q * kRowBuckets
-// counts, fill classes counters (cleared here).
-// A class beyond its room sets kStatusCapacity in *status.
+// Candidate lists of the HBM splat (PixelArgs::cl_*) for every level of a set,
+// in one launch: q * q cells per class, class k of radius (k + 1) / (2 q).  e
+// is an integer >= (2 t.eps + 2^-11) q; a table's cl_list needs
+// splat_lists_entries(q, classes, e, t.n) entries, cl_cell classes * q * q
+// (start, length) pairs, cl_yidx classes * q * q * kRowBuckets counts, its
+// fill classes counters.  A class beyond its room sets kStatusCapacity in
+// *status.
 size_t splat_lists_entries(int q, int classes, int e, int n);
-// Writes t to device memory at dst (the single-plane splat reads its table
-// from PixelArgs::level_tables).
-hipError_t launch_store_table(const SampleTable &t, SampleTable *dst, hipStream_t s);
-hipError_t launch_splat_lists(const SampleTable &st, int q, int classes, int e, uint32_t *fill, uint2 *cell,
-                              uint16_t *yidx, uint16_t *list, int *status, hipStream_t s);
+hipError_t launch_splat_lists(const LevelSet &set, int q, int e, int *status, hipStream_t s);
 
 // Also sets kStatusLambda in *a.status for lambda values outside the accepted range.
 hipError_t launch_threshold(const PixelArgs &a, double *T, hipStream_t s);
@@ -118,7 +127,7 @@ hipError_t launch_grainwise_sorted(const GrainArgs &a, const SampleTable &st, in
 // Candidate lists of the sorted grain-wise kernel: for r_const > 0 one class of
 // that output radius, else `classes` classes of radius (k + 1) / (2 q); q x q
 // cells each.  cell: classes * q * q (start, length) pairs; list: room for
-// classes * q * q * n positions; fill: classes counters (cleared here).
+// classes * q * q * n positions; fill: classes counters (cleared by the caller).
 // c_base = max(out_w, out_h) + the largest output radius + 8 (the kernel's
 // widening bound without the offsets).  Needs st.n <= 2048.
 hipError_t launch_grain_lists(const SampleTable &st, int q, int classes, float r_const, float c_base, uint32_t *fill,
@@ -176,7 +185,7 @@ struct BatchGen {
     uint32_t *const *list_fill;
     const long long *list_off;
     long long list_blocks;
-    int sort_blocks;              // workgroups per plane of the sample sort: ceil(max n_samples / kBlock)
+    int rank_blocks;              // workgroups per plane of the sample ranks: rank_blocks(max n_samples)
 };
 // Thresholds of every plane (sets kStatusLambda as launch_threshold does).
 hipError_t launch_batch_threshold(const BatchGen &bg, hipStream_t s);
@@ -185,11 +194,11 @@ hipError_t launch_batch_bin_grains(const BatchGen &bg, hipStream_t s);
 // Every plane's sample table and candidate lists.
 hipError_t launch_batch_sample_tables(const BatchGen &bg, hipStream_t s);
 
-// Adaptive sampling: tile_level[t] = first level (level_n ascending) covering
+// Adaptive sampling: tile_level[t] = first level (set.level_n) covering
 // the largest budget in tile t (a.budget).
-hipError_t launch_tile_levels(const PixelArgs &a, const int *level_n, int n_levels, uint8_t *tile_level,
-                              hipStream_t s);
-// Pointers of a sample table laid out in buf (as launch_sample_table does).
+hipError_t launch_tile_levels(const PixelArgs &a, const LevelSet &set, uint8_t *tile_level, hipStream_t s);
+int rank_blocks(int n);
+// Pointers of a sample table laid out in buf (sample_table_bytes bytes).
 void sample_table_layout(void *buf, int n, int qbuckets, SampleTable *t);
 // The plane records of one frame, written to device memory by a kernel
 // (they travel as its argument: no host buffer has to outlive a copy).

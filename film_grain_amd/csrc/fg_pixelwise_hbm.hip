@@ -544,50 +544,72 @@ __device__ __forceinline__ float sample_frac(float X)
     return f < 1.0f ? f : 0.0f;
 }
 
-// Rank sort of the samples by (fraction, index): thread i writes sample i to
-// its rank.  O(N^2) compares, N <= 65535, run once per render.
-__device__ __forceinline__ void sample_sort_body(const float2 *offs, int n, float zoom, const SampleTable &t,
-                                                 int blk, float *s_key)
+// Ranks of a table's samples (n <= 2048) by (fraction of X.x, index) and by
+// (X.y, index): workgroup blk takes kRankSamples samples, four adjacent
+// threads each, which count the smaller keys of every fourth group of four.
+// The keys are staged in LDS and read four at a time, so that the reads'
+// latency is shared (one key a read, 256 samples a workgroup and the y order
+// ranked by one workgroup on its own took 75 + 113 us for 1024 samples, this
+// and sample_levels_kernel take 15 + 10).  Sample i goes to its x rank; the y order
+// holds x ranks.  A NaN offset ranks last.
+constexpr int kRankSamples = 64;
+struct RankShared {
+    float x[2048], y[2048];
+};
+
+__device__ __forceinline__ void sample_rank_body(const float2 *offs, int n, float zoom, const SampleTable &t, int blk,
+                                                 RankShared &sh)
 {
-    const int i = blk * kBlock + threadIdx.x;
-    float2 oi = make_float2(0.0f, 0.0f);
-    float f = 0.0f;
-    if (i < n) {
-        oi = offs[i];
-        f = sample_frac(oi.x * zoom);
-    }
-    int rank = 0;
-    for (int base = 0; base < n; base += kBlock) {
-        const int j = base + (int)threadIdx.x;
-        __syncthreads();
-        s_key[threadIdx.x] = j < n ? sample_frac(offs[j].x * zoom) : 0.0f;
-        __syncthreads();
-        const int m = min(kBlock, n - base);
-        for (int jj = 0; jj < m; ++jj) {
-            const float fj = s_key[jj];
-            rank += (fj < f || (fj == f && base + jj < i)) ? 1 : 0;
+    const int padded = (n + 15) & ~15;
+    for (int j = threadIdx.x; j < padded; j += kBlock) {
+        // past the samples: keys above every sample's
+        float fx = INFINITY, y = INFINITY;
+        if (j < n) {
+            const float2 o = offs[j];
+            fx = sample_frac(o.x * zoom);
+            y = o.y * zoom;
         }
+        sh.x[j] = fx;
+        sh.y[j] = y == y ? y : INFINITY;
     }
-    if (i < n) {
-        const_cast<float2 *>(t.xy)[rank] = make_float2(oi.x * zoom, oi.y * zoom);
-        const_cast<float2 *>(t.o)[rank] = oi;
-        const_cast<uint16_t *>(t.k)[rank] = (uint16_t)i;
-        const_cast<float *>(t.key)[rank] = f;
+    __syncthreads();
+    const int i = blk * kRankSamples + ((int)threadIdx.x >> 2), part = threadIdx.x & 3;
+    const float xi = i < n ? sh.x[i] : 0.0f, yi = i < n ? sh.y[i] : 0.0f;
+    int rx = 0, ry = 0;
+    for (int g = part; 4 * g < padded; g += 4) {
+        const float4 kx = *reinterpret_cast<const float4 *>(&sh.x[4 * g]);
+        const float4 ky = *reinterpret_cast<const float4 *>(&sh.y[4 * g]);
+        auto below = [&](float k, float v, int j) { return (int)(k < v) | ((int)(k == v) & (int)(j < i)); };
+        rx += below(kx.x, xi, 4 * g) + below(kx.y, xi, 4 * g + 1) + below(kx.z, xi, 4 * g + 2) +
+              below(kx.w, xi, 4 * g + 3);
+        ry += below(ky.x, yi, 4 * g) + below(ky.y, yi, 4 * g + 1) + below(ky.z, yi, 4 * g + 2) +
+              below(ky.w, yi, 4 * g + 3);
+    }
+    rx += __shfl_xor(rx, 1, 64);
+    ry += __shfl_xor(ry, 1, 64);
+    rx += __shfl_xor(rx, 2, 64);
+    ry += __shfl_xor(ry, 2, 64);
+    if (i < n && part == 0) {
+        const float2 o = offs[i];
+        const_cast<float2 *>(t.xy)[rx] = make_float2(o.x * zoom, o.y * zoom);
+        const_cast<float2 *>(t.o)[rx] = o;
+        const_cast<uint16_t *>(t.k)[rx] = (uint16_t)i;
+        const_cast<float *>(t.key)[rx] = xi;
+        const_cast<uint16_t *>(t.yord)[ry] = (uint16_t)rx;
     }
 }
 
-__global__ __launch_bounds__(kBlock) void sample_sort_kernel(const float2 *offs, int n, float zoom,
-                                                             SampleTable t)
+__global__ __launch_bounds__(kBlock) void sample_rank_kernel(const float2 *offs, int n, float zoom, SampleTable t)
 {
-    __shared__ float s_key[kBlock];
-    sample_sort_body(offs, n, zoom, t, blockIdx.x, s_key);
+    __shared__ __align__(16) RankShared sh;
+    sample_rank_body(offs, n, zoom, t, blockIdx.x, sh);
 }
 
 // kRowBuckets intervals over a table's scaled y offsets [ext.z, ext.w]:
 // bucket(y) = floor((y - ext.z) * inv_w) clamped to [0, kRowBuckets - 1].
 // It is monotone in y, so the samples with y in [lo, hi] lie in buckets
-// bucket(lo)..bucket(hi).  sample_index (which orders the table) and the
-// splat compute it with the same code from the same extent; the splat's
+// bucket(lo)..bucket(hi).  sample_level_body (which builds the table) and
+// the splat compute it with the same code from the same extent; the splat's
 // bounds are widened by 2^-4 besides, far more than a last-bit difference.
 struct RowBuckets {
     float y0, inv_w;
@@ -604,25 +626,81 @@ __device__ __forceinline__ int row_bucket(const RowBuckets &r, float y)
     return min(max((int)floorf((y - r.y0) * r.inv_w), 0), kRowBuckets - 1);
 }
 
-// Bucket index (first sorted position with fraction >= q / Q, by binary
-// search), the extents of the scaled offsets, and the (X.y, position) order
-// with its row-bucket starts; one workgroup.
-struct IndexShared {
-    float4 r[kBlock];
-    float y[2048];
-    uint16_t ord[2048];
+// Completes a table (one workgroup of kLevelThreads): with filter set, t's
+// orders first, by filtering those of full, of which t holds the samples with
+// index < t.n (both stay sorted); without, t is ranked already; then the bucket index (first
+// position with fraction >= q / Q, by binary search), the extents of the
+// scaled offsets and the row-bucket starts of the y order.
+constexpr int kLevelThreads = 1024;
+struct LevelShared {
+    float key[2048], y[2048];
+    uint16_t ord[2048], pos[2048];
+    float4 r[kLevelThreads / 64];
+    uint32_t sum[kLevelThreads / 64];
 };
 
-__device__ __forceinline__ void sample_index_body(int n, const SampleTable &t, IndexShared &sh)
+// Exclusive prefix over the workgroup of v (0..2 per thread).
+__device__ __forceinline__ uint32_t level_prefix(uint32_t v, LevelShared &sh)
 {
-    float4 *s_r = sh.r;
+    const int wid = threadIdx.x >> 6;
+    const uint32_t incl = wave_inclusive_sum(v);
+    if ((threadIdx.x & 63) == 63) sh.sum[wid] = incl;
+    __syncthreads();
+    uint32_t before = 0;
+    for (int w = 0; w < wid; ++w) before += sh.sum[w];
+    __syncthreads();
+    return before + incl - v;
+}
+
+__device__ __forceinline__ void sample_level_body(bool filter, const SampleTable full, const SampleTable t,
+                                                  LevelShared &sh)
+{
+    const int n = t.n, tid = threadIdx.x;
+    uint16_t *yord = const_cast<uint16_t *>(t.yord), *ybk = const_cast<uint16_t *>(t.ybk);
+    if (filter) {
+        const int N = full.n, i0 = 2 * tid;
+        bool f[2];
+        for (int j = 0; j < 2; ++j) f[j] = i0 + j < N && full.k[i0 + j] < n;
+        uint32_t at = level_prefix((uint32_t)f[0] + (uint32_t)f[1], sh);
+        for (int j = 0; j < 2; ++j) {
+            const int i = i0 + j;
+            if (i < N) sh.pos[i] = f[j] ? (uint16_t)at : (uint16_t)0xFFFF;
+            if (f[j]) {
+                const float2 X = full.xy[i];
+                const_cast<float2 *>(t.xy)[at] = X;
+                const_cast<float2 *>(t.o)[at] = full.o[i];
+                const_cast<uint16_t *>(t.k)[at] = full.k[i];
+                const_cast<float *>(t.key)[at] = full.key[i];
+                sh.key[at] = full.key[i];
+                sh.y[at] = X.y;
+                ++at;
+            }
+        }
+        __syncthreads();
+        uint16_t p[2];
+        for (int j = 0; j < 2; ++j) p[j] = i0 + j < N ? sh.pos[full.yord[i0 + j]] : (uint16_t)0xFFFF;
+        at = level_prefix((uint32_t)(p[0] != 0xFFFF) + (uint32_t)(p[1] != 0xFFFF), sh);
+        for (int j = 0; j < 2; ++j)
+            if (p[j] != 0xFFFF) {
+                sh.ord[at] = p[j];
+                yord[at] = p[j];
+                ++at;
+            }
+    } else {
+        for (int i = tid; i < n; i += kLevelThreads) {
+            sh.key[i] = t.key[i];
+            sh.y[i] = t.xy[i].y;
+            sh.ord[i] = t.yord[i];
+        }
+    }
+    __syncthreads();
     const int Q = t.qbuckets;
-    for (int q = threadIdx.x; q <= Q; q += kBlock) {
+    for (int q = tid; q <= Q; q += kLevelThreads) {
         const float v = (float)q / (float)Q;  // exact: Q is a power of two
         int lo = 0, hi = n;
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
-            if (t.key[mid] < v)
+            if (sh.key[mid] < v)
                 lo = mid + 1;
             else
                 hi = mid;
@@ -630,92 +708,50 @@ __device__ __forceinline__ void sample_index_body(int n, const SampleTable &t, I
         const_cast<uint16_t *>(t.qidx)[q] = (uint16_t)lo;
     }
     float4 r = make_float4(INFINITY, -INFINITY, INFINITY, -INFINITY);
-    for (int k = threadIdx.x; k < n; k += kBlock) {
-        const float2 X = t.xy[k];
-        r.x = fminf(r.x, X.x);
-        r.y = fmaxf(r.y, X.x);
-        r.z = fminf(r.z, X.y);
-        r.w = fmaxf(r.w, X.y);
+    auto fold = [&](const float4 &b) {
+        r.x = fminf(r.x, b.x);
+        r.y = fmaxf(r.y, b.y);
+        r.z = fminf(r.z, b.z);
+        r.w = fmaxf(r.w, b.w);
+    };
+    // this thread wrote or can see every entry it reads: the filtered table's
+    // are read from full
+    const float2 *xy = filter ? full.xy : t.xy;
+    const uint16_t *k = filter ? full.k : t.k;
+    for (int i = tid; i < (filter ? full.n : n); i += kLevelThreads) {
+        if (k[i] >= n) continue;
+        const float2 X = xy[i];
+        fold(make_float4(X.x, X.x, X.y, X.y));
     }
-    s_r[threadIdx.x] = r;
+    for (int o = 32; o > 0; o >>= 1)
+        fold(make_float4(__shfl_xor(r.x, o, 64), __shfl_xor(r.y, o, 64), __shfl_xor(r.z, o, 64), __shfl_xor(r.w, o, 64)));
+    if ((tid & 63) == 0) sh.r[tid >> 6] = r;
     __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            const float4 b = s_r[threadIdx.x + w];
-            float4 c = s_r[threadIdx.x];
-            c.x = fminf(c.x, b.x);
-            c.y = fmaxf(c.y, b.y);
-            c.z = fminf(c.z, b.z);
-            c.w = fmaxf(c.w, b.w);
-            s_r[threadIdx.x] = c;
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *const_cast<float4 *>(t.ext) = s_r[0];
-    // the (X.y, position) order by rank (n <= 2048 for these; larger tables
-    // have no row order and leave it unused)
-    if (n > 2048) return;
-    const RowBuckets rb = row_buckets(s_r[0]);
-    for (int k = threadIdx.x; k < n; k += kBlock) sh.y[k] = t.xy[k].y;
-    __syncthreads();
-    for (int k = threadIdx.x; k < n; k += kBlock) {
-        const float y = sh.y[k];
-        int r = 0;
-        for (int j = 0; j < n; ++j) {
-            const float yj = sh.y[j];
-            r += (yj < y || (yj == y && j < k)) ? 1 : 0;
-        }
-        sh.ord[r] = (uint16_t)k;
-    }
-    __syncthreads();
-    uint16_t *yord = const_cast<uint16_t *>(t.yord), *ybk = const_cast<uint16_t *>(t.ybk);
-    for (int i = threadIdx.x; i < n; i += kBlock) yord[i] = sh.ord[i];
-    // the row buckets of the order are non-decreasing; index i starts
+    for (int w = 0; w < kLevelThreads / 64; ++w) fold(sh.r[w]);
+    if (tid == 0) *const_cast<float4 *>(t.ext) = r;
+    // the row buckets of the y order are non-decreasing; index i starts
     // buckets (bucket(i - 1), bucket(i)], with bucket(-1) = 0 and
     // bucket(n) = kRowBuckets
-    if (threadIdx.x == 0) ybk[0] = 0;
-    for (int i = threadIdx.x; i <= n; i += kBlock) {
+    const RowBuckets rb = row_buckets(r);
+    if (tid == 0) ybk[0] = 0;
+    for (int i = tid; i <= n; i += kLevelThreads) {
         const int prev = i == 0 ? 0 : row_bucket(rb, sh.y[sh.ord[i - 1]]);
         const int cur = i == n ? kRowBuckets : row_bucket(rb, sh.y[sh.ord[i]]);
         for (int b = prev + 1; b <= cur; ++b) ybk[b] = (uint16_t)i;
     }
 }
 
-__global__ __launch_bounds__(kBlock) void sample_index_kernel(int n, SampleTable t)
+// One workgroup per level of a set: the level's table, its list counters
+// cleared and its record stored.
+__global__ __launch_bounds__(kLevelThreads) void sample_levels_kernel(LevelSet set)
 {
-    __shared__ IndexShared sh;
-    sample_index_body(n, t, sh);
-}
-
-// The table of the first n samples from the table of all of them: the full
-// order is sorted by (fraction, index), so keeping the entries with index < n
-// in that order sorts the prefix by the same key.  One workgroup of 1024
-// threads, full.n <= 2048.
-__global__ __launch_bounds__(1024) void sample_prefix_kernel(SampleTable full, int n, SampleTable t)
-{
-    __shared__ uint32_t s_scan[1024];
-    const int i0 = 2 * (int)threadIdx.x, N = full.n;
-    const uint32_t f0 = (i0 < N && full.k[i0] < n) ? 1u : 0u;
-    const uint32_t f1 = (i0 + 1 < N && full.k[i0 + 1] < n) ? 1u : 0u;
-    s_scan[threadIdx.x] = f0 + f1;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const uint32_t v = (int)threadIdx.x >= o ? s_scan[threadIdx.x - o] : 0u;
-        __syncthreads();
-        s_scan[threadIdx.x] += v;
-        __syncthreads();
-    }
-    uint32_t pos = s_scan[threadIdx.x] - (f0 + f1);
-    for (int j = 0; j < 2; ++j) {
-        const int i = i0 + j;
-        if (j == 0 ? f0 : f1) {
-            const_cast<float2 *>(t.xy)[pos] = full.xy[i];
-            const_cast<float2 *>(t.o)[pos] = full.o[i];
-            const_cast<uint16_t *>(t.k)[pos] = full.k[i];
-            const_cast<float *>(t.key)[pos] = full.key[i];
-            ++pos;
-        }
-    }
+    __shared__ LevelShared sh;
+    const int l = blockIdx.x;
+    const SampleTable t = set.t[l];
+    sample_level_body(t.n < set.full.n, set.full, t, sh);
+    if (set.fill[l])
+        for (int k = threadIdx.x; k < set.classes; k += kLevelThreads) set.fill[l][k] = 0u;
+    if (set.store && threadIdx.x == 0) set.store[l] = t;
 }
 
 __host__ __device__ static inline size_t align16(size_t b) { return (b + 15) & ~(size_t)15; }
@@ -726,27 +762,20 @@ size_t sample_table_bytes(int n, int qbuckets)
            align16((size_t)(qbuckets + 1) * 2) + align16((size_t)(kRowBuckets + 1) * 2);
 }
 
-hipError_t launch_sample_table(const float2 *offs, int n, float zoom, int qbuckets, void *buf, SampleTable *t,
-                               hipStream_t s)
+int rank_blocks(int n) { return (n + kRankSamples - 1) / kRankSamples; }
+
+hipError_t launch_sample_rank(const float2 *offs, float zoom, const SampleTable &t, hipStream_t s)
 {
-    sample_table_layout(buf, n, qbuckets, t);
-    hipLaunchKernelGGL(sample_sort_kernel, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, offs,
-                       n, zoom, *t);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(sample_index_kernel, dim3(1), dim3(kBlock), 0, s, n, *t);
+    if (t.n < 1 || t.n > 2048) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(sample_rank_kernel, dim3((unsigned)rank_blocks(t.n)), dim3(kBlock), 0, s,
+                       offs, t.n, zoom, t);
     return hipGetLastError();
 }
 
-hipError_t launch_sample_prefix(const SampleTable &full, int n, int qbuckets, void *buf, SampleTable *t,
-                                hipStream_t s)
+hipError_t launch_sample_levels(const LevelSet &set, hipStream_t s)
 {
-    if (full.n > 2048 || n > full.n) return hipErrorInvalidValue;
-    sample_table_layout(buf, n, qbuckets, t);
-    hipLaunchKernelGGL(sample_prefix_kernel, dim3(1), dim3(1024), 0, s, full, n, *t);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(sample_index_kernel, dim3(1), dim3(kBlock), 0, s, n, *t);
+    if (set.n < 1 || set.n > kMaxLevels || set.full.n > 2048) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(sample_levels_kernel, dim3((unsigned)set.n), dim3(kLevelThreads), 0, s, set);
     return hipGetLastError();
 }
 
@@ -905,11 +934,15 @@ __device__ __forceinline__ void splat_lists_body(const SampleTable &st, int q, i
     }
 }
 
-__global__ __launch_bounds__(256) void splat_lists_kernel(SampleTable st, int q, int e, uint32_t *fill, uint2 *cell,
-                                                          uint16_t *yidx, uint16_t *list, int *status)
+// The lists of every level of a set, one after another.
+__global__ __launch_bounds__(256) void splat_lists_kernel(LevelSet set, int q, int e, int *status)
 {
     __shared__ ListsShared sh;
-    splat_lists_body(st, q, e, st.eps, 0.0f, fill, cell, yidx, list, status, blockIdx.x, sh);
+    const int per = set.classes * ((q * q + 63) / 64);
+    const int l = blockIdx.x / per;
+    const SampleTable &t = set.t[l];
+    splat_lists_body(t, q, e, t.eps, 0.0f, set.fill[l], const_cast<uint2 *>(t.cl_cell), const_cast<uint16_t *>(t.cl_yidx),
+                     const_cast<uint16_t *>(t.cl_list), status, blockIdx.x - l * per, sh);
 }
 
 // The grain-wise kernel's lists (launch_grain_lists).  A grain's target is b +
@@ -931,33 +964,32 @@ hipError_t launch_grain_lists(const SampleTable &st, int q, int classes, float r
                               uint2 *cell, uint16_t *list, int *status, hipStream_t s)
 {
     if (q < 1 || q * q > 65536 || classes < 1 || st.n > 2048) return hipErrorInvalidValue;
-    const hipError_t err = launch_fill_u32(fill, classes, 0u, s);
-    if (err != hipSuccess) return err;
     hipLaunchKernelGGL(grain_lists_kernel, dim3(classes * ((q * q + 63) / 64)), dim3(256), 0, s, st, q, r_const, c_base,
                        fill, cell, list, status);
     return hipGetLastError();
 }
 
-// Batch sample tables: workgroup (x, p) sorts samples x * kBlock.. of plane p.
-__global__ __launch_bounds__(kBlock) void batch_sample_sort_kernel(BatchGen bg)
+// Batch sample tables: workgroup (x, p) ranks samples x * kRankSamples.. of
+// plane p.
+__global__ __launch_bounds__(kBlock) void batch_sample_rank_kernel(BatchGen bg)
 {
-    __shared__ float s_key[kBlock];
+    __shared__ __align__(16) RankShared sh;
     const BatchPlane &bp = cplane(bg.planes, blockIdx.y);
-    if ((int)blockIdx.x * kBlock >= bp.a.n_samples) return;
-    sample_sort_body(bp.a.offs, bp.a.n_samples, bp.a.zoom, bp.st, blockIdx.x, s_key);
+    if ((int)blockIdx.x * kRankSamples >= bp.a.n_samples) return;
+    sample_rank_body(bp.a.offs, bp.a.n_samples, bp.a.zoom, bp.st, blockIdx.x, sh);
 }
 
-// One workgroup per plane: the table's index, and the candidate lists'
+// One workgroup per plane: the rest of its table, and the candidate lists'
 // counters cleared for batch_splat_lists_kernel.
-__global__ __launch_bounds__(kBlock) void batch_sample_index_kernel(BatchGen bg)
+__global__ __launch_bounds__(kLevelThreads) void batch_sample_level_kernel(BatchGen bg)
 {
-    __shared__ IndexShared sh;
+    __shared__ LevelShared sh;
     const int p = blockIdx.x;
     const BatchPlane &bp = cplane(bg.planes, p);
-    sample_index_body(bp.a.n_samples, bp.st, sh);
+    sample_level_body(false, bp.st, bp.st, sh);
     const int classes = cload(bg.list_plan + p).y;
     uint32_t *fill = cload(bg.list_fill + p);
-    for (int k = threadIdx.x; k < classes; k += kBlock) fill[k] = 0u;
+    for (int k = threadIdx.x; k < classes; k += kLevelThreads) fill[k] = 0u;
 }
 
 __global__ __launch_bounds__(256) void batch_splat_lists_kernel(BatchGen bg)
@@ -972,32 +1004,17 @@ __global__ __launch_bounds__(256) void batch_splat_lists_kernel(BatchGen bg)
                      (int)(blk - cload(bg.list_off + p)), sh);
 }
 
-__global__ void store_table_kernel(SampleTable t, SampleTable *dst)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) *dst = t;
-}
-
-hipError_t launch_store_table(const SampleTable &t, SampleTable *dst, hipStream_t s)
-{
-    hipLaunchKernelGGL(store_table_kernel, dim3(1), dim3(64), 0, s, t, dst);
-    return hipGetLastError();
-}
-
 size_t splat_lists_entries(int q, int classes, int e, int n)
 {
     return splat_list_base(classes, q, e, n);
 }
 
-hipError_t launch_splat_lists(const SampleTable &st, int q, int classes, int e, uint32_t *fill, uint2 *cell,
-                              uint16_t *yidx, uint16_t *list, int *status, hipStream_t s)
+hipError_t launch_splat_lists(const LevelSet &set, int q, int e, int *status, hipStream_t s)
 {
-    if (q < 1 || q * q > 65536 || classes < 1 || st.n > 2048) return hipErrorInvalidValue;
-    // a kernel, not hipMemsetAsync: batches capture this into a graph
-    hipError_t err = launch_fill_u32(fill, classes, 0u, s);
-    if (err != hipSuccess) return err;
-    const int parts = (q * q + 63) / 64;
-    hipLaunchKernelGGL(splat_lists_kernel, dim3(classes * parts), dim3(256), 0, s, st, q, e, fill, cell, yidx,
-                       list, status);
+    if (q < 1 || q * q > 65536 || set.classes < 1 || set.n < 1 || set.n > kMaxLevels || set.full.n > 2048)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(splat_lists_kernel, dim3(set.n * set.classes * ((q * q + 63) / 64)), dim3(256), 0, s, set, q, e,
+                       status);
     return hipGetLastError();
 }
 
@@ -1039,8 +1056,7 @@ __global__ __launch_bounds__(kBlock) void pixel_tile_weights_kernel(PixelArgs a,
 
 // Adaptive sampling: per tile, the first level whose sample count covers the
 // largest budget among its pixels (levels ascending, the last = n_samples).
-__global__ __launch_bounds__(kBlock) void tile_levels_kernel(PixelArgs a, const int *level_n, int n_levels,
-                                                             uint8_t *tile_level)
+__global__ __launch_bounds__(kBlock) void tile_levels_kernel(PixelArgs a, LevelSet set, uint8_t *tile_level)
 {
     const int tile = blockIdx.x * kBlock + threadIdx.x;
     if (tile >= a.n_tiles) return;
@@ -1051,15 +1067,14 @@ __global__ __launch_bounds__(kBlock) void tile_levels_kernel(PixelArgs a, const 
     for (int y = Y0; y < Y1; ++y)
         for (int x = X0; x < X1; ++x) m = max(m, (int)a.budget[(size_t)y * a.out_w + x]);
     int l = 0;
-    while (l + 1 < n_levels && level_n[l] < m) ++l;
+    while (l + 1 < set.n && set.level_n[l] < m) ++l;
     tile_level[tile] = (uint8_t)l;
 }
 
-hipError_t launch_tile_levels(const PixelArgs &a, const int *level_n, int n_levels, uint8_t *tile_level,
-                              hipStream_t s)
+hipError_t launch_tile_levels(const PixelArgs &a, const LevelSet &set, uint8_t *tile_level, hipStream_t s)
 {
     hipLaunchKernelGGL(tile_levels_kernel, dim3((unsigned)((a.n_tiles + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
-                       a, level_n, n_levels, tile_level);
+                       a, set, tile_level);
     return hipGetLastError();
 }
 
@@ -1747,12 +1762,12 @@ hipError_t launch_batch_bin_grains(const BatchGen &bg, hipStream_t s)
 
 hipError_t launch_batch_sample_tables(const BatchGen &bg, hipStream_t s)
 {
-    if (bg.n <= 0 || bg.n > 65535 || bg.sort_blocks <= 0 || bg.list_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(batch_sample_sort_kernel, dim3((unsigned)bg.sort_blocks, (unsigned)bg.n), dim3(kBlock), 0, s,
+    if (bg.n <= 0 || bg.n > 65535 || bg.rank_blocks <= 0 || bg.list_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(batch_sample_rank_kernel, dim3((unsigned)bg.rank_blocks, (unsigned)bg.n), dim3(kBlock), 0, s,
                        bg);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(batch_sample_index_kernel, dim3((unsigned)bg.n), dim3(kBlock), 0, s, bg);
+    hipLaunchKernelGGL(batch_sample_level_kernel, dim3((unsigned)bg.n), dim3(kLevelThreads), 0, s, bg);
     e = hipGetLastError();
     if (e != hipSuccess || bg.list_blocks == 0) return e;
     hipLaunchKernelGGL(batch_splat_lists_kernel, dim3((unsigned)bg.list_blocks), dim3(256), 0, s, bg);

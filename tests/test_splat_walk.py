@@ -151,3 +151,39 @@ def test_constant_radius_planes_equal_the_oracle(hip_ctx, oracle, w, h, r, zoom,
     want = oracle.render_pixelwise(case.plane, case.lam, case.offsets_input)
     got = hip_ctx.render_host("pixel", case.desc, case.lam, case.offsets_input)
     assert int(np.sum(got != want)) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 33, 63, 64, 65, 129, 1000, 1024, 2047, 2048])
+def test_tables_of_every_level(hip_ctx, oracle, n):
+    """Sample counts around the ranks' groups of four, a workgroup's 64
+    samples and the levels (16, 32, ..., n), with offsets that tie in x, in y
+    and in both: the fixed render and an adaptive one with budgets in every
+    level, against the oracle at each pixel's own sample count."""
+    import torch
+    from film_grain_amd import synth
+    from tests import fgcases
+    w, h = 24, 16
+    u = synth.sinusoid_field(w, h, n, n_waves=3)
+    case = fgcases.build_case(oracle, f"tab_{n}", u, 0.12, 0.04, "lognorm", n_samples=n, seed=n + 5)
+    offs = np.array(case.offsets_input)
+    offs[n // 2:, 0] = offs[:n - n // 2, 0]
+    offs[n // 3:, 1] = np.round(offs[n // 3:, 1] * 4) / 4
+    case.offsets_input[:] = offs
+    want = oracle.render_pixelwise(case.plane, case.lam, case.offsets_input)
+    got = hip_ctx.render_host("pixel", case.desc, case.lam, case.offsets_input)
+    assert int(np.sum(got != want)) == 0
+    rng = np.random.default_rng(n)
+    sizes = sorted({max(1, min(n, v)) for v in (1, 15, 16, 17, 32, 100, 128, 500, 1024, n)})
+    blocks = rng.choice(sizes, size=(h // 4, w // 4))
+    budget = np.kron(blocks, np.ones((4, 4), dtype=np.int64)).astype(np.uint16)
+    out = torch.empty((h, w), dtype=torch.float32, device="cuda:0")
+    hip_ctx.render_adaptive_device(case.desc, torch.from_numpy(case.lam).to("cuda:0"),
+                                   torch.from_numpy(case.offsets_input).to("cuda:0"),
+                                   torch.from_numpy(budget.view(np.int16)).to("cuda:0"), out)
+    hip_ctx.stream_status()
+    out = out.cpu().numpy()
+    for b in np.unique(budget):
+        p = oracle.plane(case.derived, int(b), case.seed, case.zoom, case.dist, case.radius)
+        fixed = oracle.render_pixelwise(p, case.lam, np.ascontiguousarray(case.offsets_input[:b]))
+        assert np.array_equal(out[budget == b], fixed[budget == b]), int(b)
