@@ -87,6 +87,145 @@ hipError_t launch_scan_u32(const uint32_t *in, uint32_t *out, long long n, uint3
     return hipGetLastError();
 }
 
+// ---- the bins of a plane, or of a frame's planes, in one set of launches ----
+// As above with 64-bit sums (a plane's total may reach 2^32: the host refuses
+// it then), the starts truncated to 32 bits, and each plane's total published
+// to the host.  A workgroup takes kBinScanTile bins; up to kBinScanSmall bins
+// one workgroup a plane does everything.
+constexpr int kBinScanThreads = 1024;
+constexpr int kBinScanItems = 4;
+constexpr int kBinScanTile = kBinScanThreads * kBinScanItems;
+constexpr long long kBinScanSmall = 4 * kBinScanTile;
+
+size_t bin_scan_partials(long long n) { return (size_t)((n + kBinScanTile - 1) / kBinScanTile) + 1; }
+
+// Exclusive prefix of v over the workgroup, and its total, in 64 bits (values
+// below 2^26 by the 32-bit wave sum).
+__device__ __forceinline__ unsigned long long bin_scan_prefix(unsigned long long v, unsigned long long *s_wave,
+                                                              unsigned long long &total)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    unsigned long long x = v;
+    if (__ballot(v >= (1ull << 26)) == 0ull) {
+        x = wave_inclusive_sum((uint32_t)v);
+    } else {
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned long long y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+    }
+    if (lane == 63) s_wave[wid] = x;
+    __syncthreads();
+    unsigned long long before = 0;
+    total = 0;
+    for (int w = 0; w < kBinScanThreads / 64; ++w) {
+        const unsigned long long t = s_wave[w];
+        before += w < wid ? t : 0ull;
+        total += t;
+    }
+    __syncthreads();
+    return before + x - v;
+}
+
+// A plane's total to the host (one thread), then its flag.
+__device__ __forceinline__ void publish_total(HostPublish *pub, uint32_t seq, int plane, unsigned long long total)
+{
+    __hip_atomic_store(&pub->total[plane], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&pub->total_seq[plane], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__device__ __forceinline__ unsigned long long bin_scan_load(const uint32_t *in, long long base, long long n,
+                                                            uint32_t v[kBinScanItems])
+{
+    unsigned long long sum = 0;
+    for (int i = 0; i < kBinScanItems; ++i) {
+        v[i] = base + i < n ? in[base + i] : 0u;
+        sum += v[i];
+    }
+    return sum;
+}
+
+__global__ __launch_bounds__(kBinScanThreads) void bin_scan_sums_kernel(BinScan b)
+{
+    __shared__ unsigned long long s_wave[kBinScanThreads / 64];
+    const int p = blockIdx.y;
+    uint32_t v[kBinScanItems];
+    unsigned long long total;
+    const long long base = (long long)blockIdx.x * kBinScanTile + (long long)threadIdx.x * kBinScanItems;
+    (void)bin_scan_prefix(bin_scan_load(b.in[p], base, b.n, v), s_wave, total);
+    if (threadIdx.x == 0) b.partials[p][blockIdx.x] = total;
+}
+
+__global__ __launch_bounds__(kBinScanThreads) void bin_scan_prefix_kernel(BinScan b, long long m)
+{
+    __shared__ unsigned long long s_wave[kBinScanThreads / 64];
+    const int p = blockIdx.x;
+    unsigned long long carry = 0;
+    for (long long i0 = 0; i0 < m; i0 += kBinScanThreads) {
+        const long long i = i0 + threadIdx.x;
+        const unsigned long long v = i < m ? b.partials[p][i] : 0ull;
+        unsigned long long total;
+        const unsigned long long ex = bin_scan_prefix(v, s_wave, total);
+        if (i < m) b.partials[p][i] = carry + ex;
+        carry += total;
+    }
+    if (threadIdx.x == 0) {
+        b.out[p][b.n] = (uint32_t)carry;
+        publish_total(b.pub, b.seq, p, carry);
+    }
+}
+
+__global__ __launch_bounds__(kBinScanThreads) void bin_scan_apply_kernel(BinScan b)
+{
+    __shared__ unsigned long long s_wave[kBinScanThreads / 64];
+    const int p = blockIdx.y;
+    uint32_t v[kBinScanItems];
+    unsigned long long total;
+    const long long base = (long long)blockIdx.x * kBinScanTile + (long long)threadIdx.x * kBinScanItems;
+    uint32_t run = (uint32_t)(b.partials[p][blockIdx.x] +
+                              bin_scan_prefix(bin_scan_load(b.in[p], base, b.n, v), s_wave, total));
+    for (int i = 0; i < kBinScanItems; ++i) {
+        if (base + i < b.n) b.out[p][base + i] = run;
+        run += v[i];
+    }
+}
+
+__global__ __launch_bounds__(kBinScanThreads) void bin_scan_small_kernel(BinScan b)
+{
+    __shared__ unsigned long long s_wave[kBinScanThreads / 64];
+    const int p = blockIdx.x;
+    unsigned long long carry = 0;
+    for (long long i0 = 0; i0 < b.n; i0 += kBinScanTile) {
+        uint32_t v[kBinScanItems];
+        unsigned long long total;
+        const long long base = i0 + (long long)threadIdx.x * kBinScanItems;
+        uint32_t run = (uint32_t)(carry + bin_scan_prefix(bin_scan_load(b.in[p], base, b.n, v), s_wave, total));
+        for (int i = 0; i < kBinScanItems; ++i) {
+            if (base + i < b.n) b.out[p][base + i] = run;
+            run += v[i];
+        }
+        carry += total;
+    }
+    if (threadIdx.x == 0) {
+        b.out[p][b.n] = (uint32_t)carry;
+        publish_total(b.pub, b.seq, p, carry);
+    }
+}
+
+hipError_t launch_bin_scan(const BinScan &b, hipStream_t s)
+{
+    if (b.planes < 1 || b.planes > kFramePlanes || b.n < 1) return hipErrorInvalidValue;
+    if (b.n <= kBinScanSmall) {
+        hipLaunchKernelGGL(bin_scan_small_kernel, dim3((unsigned)b.planes), dim3(kBinScanThreads), 0, s, b);
+        return hipGetLastError();
+    }
+    const long long m = (b.n + kBinScanTile - 1) / kBinScanTile;
+    hipLaunchKernelGGL(bin_scan_sums_kernel, dim3((unsigned)m, (unsigned)b.planes), dim3(kBinScanThreads), 0, s, b);
+    hipLaunchKernelGGL(bin_scan_prefix_kernel, dim3((unsigned)b.planes), dim3(kBinScanThreads), 0, s, b, m);
+    hipLaunchKernelGGL(bin_scan_apply_kernel, dim3((unsigned)m, (unsigned)b.planes), dim3(kBinScanThreads), 0, s, b);
+    return hipGetLastError();
+}
+
 __global__ __launch_bounds__(kBlock) void fill_u32_kernel(uint32_t *p, long long n, uint32_t v)
 {
     for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long long)gridDim.x * kBlock)
@@ -114,26 +253,13 @@ __device__ __forceinline__ int plane_of(const BatchPlane *planes, int n_planes, 
     return lo;
 }
 
-__device__ __forceinline__ uint32_t item_weight(const BatchPlane &p, int tile)
-{
-    const PixelArgs &a = p.a;
-    const int tyi = tile / a.tiles_x, txi = tile - tyi * a.tiles_x;
-    const int X0 = txi * a.tile_w, Y0 = tyi * a.tile_h;
-    const TileRegion r = tile_region(a, p.geo, X0, Y0, min(X0 + a.tile_w, a.out_w), min(Y0 + a.tile_h, a.out_h));
-    uint32_t sum = 0;
-    if (r.bx0 <= r.bx1)
-        for (int by = r.by0; by <= r.by1; ++by)
-            sum += p.bin_start[by * p.geo.nbx + r.bx1 + 1] - p.bin_start[by * p.geo.nbx + r.bx0];
-    return sum;
-}
-
 __global__ __launch_bounds__(kBlock) void batch_weights_kernel(const BatchPlane *planes, int n_planes, uint32_t *w,
                                                                int n_items)
 {
     const int item = blockIdx.x * kBlock + threadIdx.x;
     if (item >= n_items) return;
     const int pl = plane_of(planes, n_planes, item);
-    w[item] = item_weight(planes[pl], (int)(item - planes[pl].item_base));
+    w[item] = tile_weight(planes[pl].a, planes[pl].geo, planes[pl].bin_start, (int)(item - planes[pl].item_base));
 }
 
 hipError_t launch_batch_weights(const BatchPlane *planes, int n_planes, uint32_t *w, int n_items, hipStream_t s)
@@ -181,6 +307,48 @@ hipError_t launch_batch_order(const BatchPlane *planes, int n_planes, const uint
     (void)scratch;
     if (n_items <= 0) return hipSuccess;
     hipLaunchKernelGGL(batch_order_kernel, dim3(1), dim3(1024), 0, s, planes, n_planes, w, n_items, items);
+    return hipGetLastError();
+}
+
+// Weights and heaviest-first order of one plane's tiles in one workgroup, for
+// planes of at most kOrderTiles tiles: a counting sort by quarter octaves of
+// the weight.  (The weights' launch and a radix sort's one to four took 13 to
+// 25 us of a small plane; this takes 5 to 8.)
+__global__ __launch_bounds__(1024) void tile_order_kernel(PixelArgs a, PixGeom geo, const uint32_t *bin_start, int *order)
+{
+    __shared__ uint32_t s_count[128], s_pos[128];
+    constexpr int kPer = kOrderTiles / 1024;
+    if (threadIdx.x < 128) s_count[threadIdx.x] = 0;
+    __syncthreads();
+    uint8_t bucket[kPer];
+    for (int j = 0; j < kPer; ++j) {
+        const int tile = j * 1024 + (int)threadIdx.x;
+        bucket[j] = 0;
+        if (tile >= a.n_tiles) continue;
+        const uint32_t w = tile_weight(a, geo, bin_start, tile);
+        // 4 log2(w + 1) by the float's exponent and two mantissa bits
+        bucket[j] = (uint8_t)min(127u, (__float_as_uint((float)w + 1.0f) >> 21) - (127u << 2));
+        atomicAdd(&s_count[bucket[j]], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {  // first position of each bucket, heaviest first
+        const int b = 127 - 2 * (int)threadIdx.x;
+        const uint32_t c0 = s_count[b], c1 = s_count[b - 1];
+        const uint32_t before = wave_inclusive_sum(c0 + c1) - (c0 + c1);
+        s_pos[b] = before;
+        s_pos[b - 1] = before + c0;
+    }
+    __syncthreads();
+    for (int j = 0; j < kPer; ++j) {
+        const int tile = j * 1024 + (int)threadIdx.x;
+        if (tile < a.n_tiles) order[atomicAdd(&s_pos[bucket[j]], 1u)] = tile;
+    }
+}
+
+hipError_t launch_tile_order(const PixelArgs &a, const PixGeom &g, const uint32_t *bin_start, int *order, hipStream_t s)
+{
+    if (a.n_tiles > kOrderTiles) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, s, a, g, bin_start, order);
     return hipGetLastError();
 }
 

@@ -48,7 +48,10 @@ struct fg_ctx {
     // per-context device scratch: status word, stats counters, offsets range
     int *d_status = nullptr;
     unsigned long long *d_stats = nullptr;
-    unsigned long long *d_sum64 = nullptr;  // a plane's 64-bit grain total (bin_count)
+    // what kernels publish to the host (host and device addresses) and the
+    // last sequence number handed out
+    fg::HostPublish *h_pub = nullptr, *d_pub = nullptr;
+    uint32_t pub_seq = 0;
     // device address of this device's copy of the allocation-free entry
     // point's static scratch array (hipGetSymbolAddress at creation)
     unsigned char *noalloc_scratch = nullptr;
@@ -146,6 +149,12 @@ void free_buffers(fg_ctx *ctx)
 int ensure_bytes(fg_ctx *ctx, DevBuf &b, size_t bytes, const char *what)
 {
     if (b.cap >= bytes) return FG_OK;
+    if (ctx->scratch_pending) {
+        // the previous call's kernels may still read the buffer
+        const hipError_t e = hipEventSynchronize(ctx->scratch_done);
+        if (e != hipSuccess) return hip_error(ctx, e, what);
+        ctx->scratch_pending = false;
+    }
     free_buf(b);
     const size_t want = std::max<size_t>(bytes + bytes / 8, 256);  // headroom for the next plane
     const hipError_t e = hipMalloc(&b.p, want);
@@ -169,6 +178,73 @@ int scratch_acquire(fg_ctx *ctx, const char *what)
     return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
 }
 
+// True while s records into a graph of the caller's.
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+// The same order without the host waiting: work enqueued on s from here on runs
+// after the previous user's last kernel.  (The call waits for s itself before
+// it reads what its first kernels publish.)  A capture takes no event from
+// outside, so there the host waits.
+int scratch_acquire_on(fg_ctx *ctx, hipStream_t s, const char *what)
+{
+    if (!ctx->scratch_pending) return FG_OK;
+    if (capturing(s)) return scratch_acquire(ctx, what);
+    const hipError_t e = hipStreamWaitEvent(s, ctx->scratch_done, 0);
+    return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
+}
+
+// Waits until a kernel on s has published under seq (the flag holds it).  The
+// host polls the flag for up to 5 ms (a copy to host memory and a
+// stream wait cost 20 to 30 us more, twice in every small render), then waits
+// for the stream; a stream that ends without publishing is an error.
+hipError_t wait_published(const uint32_t *flag, uint32_t seq, hipStream_t s)
+{
+    const auto there = [&] { return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq; };
+    struct timespec t0, t;
+    (void)clock_gettime(CLOCK_MONOTONIC, &t0);
+    for (int i = 0;; ++i) {
+        if (there()) return hipSuccess;
+        if ((i & 255) != 255) continue;
+        (void)clock_gettime(CLOCK_MONOTONIC, &t);
+        if ((t.tv_sec - t0.tv_sec) * 1000000000LL + (t.tv_nsec - t0.tv_nsec) > 5000000LL) break;
+    }
+    const hipError_t e = hipStreamSynchronize(s);
+    if (e != hipSuccess) return e;
+    return there() ? hipSuccess : hipErrorUnknown;
+}
+
+// The offsets' range of a pixel-wise render: computed on s, published to the
+// host.  read_range waits for it.
+hipError_t enqueue_range(fg_ctx *ctx, const float *d_offs, int n, hipStream_t s, uint32_t *seq)
+{
+    *seq = ++ctx->pub_seq;
+    return fg::launch_offsets_range(reinterpret_cast<const float2 *>(d_offs), n, ctx->d_range, s, ctx->d_pub, *seq);
+}
+
+hipError_t read_range(fg_ctx *ctx, uint32_t seq, hipStream_t s, float4 *range)
+{
+    const hipError_t e = wait_published(&ctx->h_pub->range_seq, seq, s);
+    const float *r = ctx->h_pub->range;
+    if (e == hipSuccess) *range = make_float4(r[0], r[1], r[2], r[3]);
+    return e;
+}
+
+// Marks the scratch as in use by s when a call that has enqueued kernels on it
+// returns early.
+struct ScratchGuard {
+    fg_ctx *ctx;
+    hipStream_t s;
+    bool armed = true;
+    ~ScratchGuard()
+    {
+        if (armed && !capturing(s) && hipEventRecord(ctx->scratch_done, s) == hipSuccess) ctx->scratch_pending = true;
+    }
+};
+
 void mark(fg_ctx *ctx, int i, hipStream_t s)
 {
     if (!ctx->timing) return;
@@ -179,6 +255,7 @@ void mark(fg_ctx *ctx, int i, hipStream_t s)
 
 int scratch_release(fg_ctx *ctx, hipStream_t s, const char *what)
 {
+    if (capturing(s)) return FG_OK;  // nothing runs yet, and a recorded event would belong to the graph
     const hipError_t e = hipEventRecord(ctx->scratch_done, s);
     if (e != hipSuccess) return hip_error(ctx, e, what);
     ctx->scratch_pending = true;
@@ -539,6 +616,14 @@ void splat_bounds(const fg::PixelArgs &a, const fg::PixGeom &g, const float4 &r,
 struct TileOrder {
     uint32_t *w = nullptr, *w_sorted = nullptr;
     int *ids = nullptr, *order = nullptr;
+    void place(void *p, int n)  // 16 n bytes
+    {
+        unsigned char *b = static_cast<unsigned char *>(p);
+        w = reinterpret_cast<uint32_t *>(b);
+        w_sorted = reinterpret_cast<uint32_t *>(b + (size_t)n * 4);
+        ids = reinterpret_cast<int *>(b + (size_t)n * 8);
+        order = reinterpret_cast<int *>(b + (size_t)n * 12);
+    }
 };
 
 int tile_order_prepare(fg_ctx *ctx, int n, TileOrder *t, hipStream_t s, const char *what)
@@ -549,11 +634,7 @@ int tile_order_prepare(fg_ctx *ctx, int n, TileOrder *t, hipStream_t s, const ch
     hipError_t e = fg::sort_tiles(nullptr, &temp, nullptr, nullptr, nullptr, nullptr, n, s);
     if (e != hipSuccess) return hip_error(ctx, e, what);
     if ((rc = ensure_bytes(ctx, ctx->tile_temp, temp, what)) != FG_OK) return rc;
-    unsigned char *p = static_cast<unsigned char *>(ctx->tiles.p);
-    t->w = reinterpret_cast<uint32_t *>(p);
-    t->w_sorted = reinterpret_cast<uint32_t *>(p + (size_t)n * 4);
-    t->ids = reinterpret_cast<int *>(p + (size_t)n * 8);
-    t->order = reinterpret_cast<int *>(p + (size_t)n * 12);
+    t->place(ctx->tiles.p, n);
     return FG_OK;
 }
 
@@ -694,22 +775,15 @@ int scratch_get(fg_ctx *ctx, ScratchSource &src, DevBuf &b, size_t bytes, void *
 }
 
 // The per-plane generation of the HBM path: Poisson thresholds, per-bin
-// counts and nonempty masks, their scan, and every cell's grains written
-// contiguously per bin.
-// A plane's thresholds, bin counts (nbins + 1 entries) and nonempty masks,
-// computed beforehand with the other planes of its frame.
-struct PreCounts {
-    double *T = nullptr;
-    uint32_t *cnt = nullptr;
-    unsigned long long *mask = nullptr;
-};
-
+// counts and nonempty masks and their scan (hbm_count), and every cell's
+// grains written contiguously per bin (hbm_draw, after a wait for the total).
 struct HbmGen {
     double *T = nullptr;
     uint32_t *start = nullptr;
     unsigned long long *mask = nullptr;
     float4 *grains = nullptr;
     unsigned long long total = 0;
+    uint32_t seq = 0;  // the total is published under it
 };
 
 // The plane's grain total, refused when bin starts (u32 offsets) cannot
@@ -726,80 +800,82 @@ int check_total(fg_ctx *ctx, unsigned long long total, const char *what)
     return FG_OK;
 }
 
-int hbm_generate(fg_ctx *ctx, ScratchSource &src, fg::PixelArgs &a, const fg::PixGeom &g, int dist_kind,
-                 hipStream_t s, HbmGen *out, const PreCounts *pre = nullptr)
+int hbm_count(fg_ctx *ctx, ScratchSource &src, fg::PixelArgs &a, const fg::PixGeom &g, hipStream_t s, HbmGen *out)
 {
     const char *what = "Pixel renderer";
     int rc;
     const long long nbins = (long long)g.nbx * g.nby;
     const size_t npx = (size_t)a.in_w * a.in_h;
-    void *T_p, *cnt_p, *start_p, *mask_p, *temp_p, *grains_p;
-    if (pre) {
-        T_p = pre->T;
-        cnt_p = pre->cnt;
-        mask_p = pre->mask;
-    } else {
-        if ((rc = scratch_get(ctx, src, ctx->thresholds, npx * sizeof(double), &T_p, what)) != FG_OK) return rc;
-        if ((rc = scratch_get(ctx, src, ctx->bin_count, (size_t)(nbins + 1) * 4, &cnt_p, what)) != FG_OK) return rc;
-        if ((rc = scratch_get(ctx, src, ctx->bin_mask, (size_t)nbins * 32, &mask_p, what)) != FG_OK) return rc;
-    }
+    void *T_p, *cnt_p, *start_p, *mask_p, *temp_p;
+    if ((rc = scratch_get(ctx, src, ctx->thresholds, npx * sizeof(double), &T_p, what)) != FG_OK) return rc;
+    if ((rc = scratch_get(ctx, src, ctx->bin_count, (size_t)(nbins + 1) * 4, &cnt_p, what)) != FG_OK) return rc;
+    if ((rc = scratch_get(ctx, src, ctx->bin_mask, (size_t)nbins * 32, &mask_p, what)) != FG_OK) return rc;
     if ((rc = scratch_get(ctx, src, ctx->bin_start, (size_t)(nbins + 1) * 4, &start_p, what)) != FG_OK) return rc;
-    size_t temp_bytes = 0;
-    hipError_t e = fg::scan_bins(nullptr, &temp_bytes, nullptr, nullptr, (int)(nbins + 1), s);
-    if (e != hipSuccess) return hip_error(ctx, e, what);
-    if ((rc = scratch_get(ctx, src, ctx->scan_temp, temp_bytes, &temp_p, what)) != FG_OK) return rc;
-    double *T = static_cast<double *>(T_p);
+    if ((rc = scratch_get(ctx, src, ctx->scan_temp, fg::bin_scan_partials(nbins) * 8, &temp_p, what)) != FG_OK) return rc;
+    out->T = static_cast<double *>(T_p);
+    out->start = static_cast<uint32_t *>(start_p);
+    out->mask = static_cast<unsigned long long *>(mask_p);
+    out->seq = ++ctx->pub_seq;
     uint32_t *cnt = static_cast<uint32_t *>(cnt_p);
-    uint32_t *start = static_cast<uint32_t *>(start_p);
-    unsigned long long *mask = static_cast<unsigned long long *>(mask_p);
-    // the plane's grain total: the bin counts summed in 64 bits (cleared by
-    // a kernel: the caller may capture this into a graph)
-    e = fg::launch_fill_u32(reinterpret_cast<uint32_t *>(ctx->d_sum64), 2, 0u, s);
-    if (e == hipSuccess) e = fg::launch_fill_u32(cnt + nbins, 1, 0u, s);
-    if (!pre) {
-        if (e == hipSuccess) e = fg::launch_threshold(a, T, s);
-        if (e == hipSuccess) e = fg::launch_bin_count(a, g, T, cnt, mask, s);
-    }
-    if (e == hipSuccess) e = fg::launch_sum_u64(cnt, nbins, ctx->d_sum64, s);
-    if (e == hipSuccess) e = fg::scan_bins(temp_p, &temp_bytes, cnt, start, (int)(nbins + 1), s);
-    unsigned long long total = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&total, ctx->d_sum64, 8, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    hipError_t e = fg::launch_threshold(a, out->T, s);
+    if (e == hipSuccess) e = fg::launch_bin_count(a, g, out->T, cnt, out->mask, s);
+    fg::BinScan scan{};
+    scan.in[0] = cnt;
+    scan.out[0] = out->start;
+    scan.partials[0] = static_cast<unsigned long long *>(temp_p);
+    scan.n = nbins;
+    scan.pub = ctx->d_pub;
+    scan.seq = out->seq;
+    scan.planes = 1;
+    if (e == hipSuccess) e = fg::launch_bin_scan(scan, s);
+    return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
+}
+
+int hbm_draw(fg_ctx *ctx, ScratchSource &src, fg::PixelArgs &a, const fg::PixGeom &g, int dist_kind, hipStream_t s,
+             HbmGen *out)
+{
+    const char *what = "Pixel renderer";
+    int rc;
+    void *grains_p;
+    hipError_t e = wait_published(&ctx->h_pub->total_seq[0], out->seq, s);
     if (e != hipSuccess) return hip_error(ctx, e, what);
-    if ((rc = check_total(ctx, total, what)) != FG_OK) return rc;
-    if ((rc = scratch_get(ctx, src, ctx->grains, std::max<size_t>((size_t)total, 1) * sizeof(float4), &grains_p,
+    out->total = ctx->h_pub->total[0];
+    if ((rc = check_total(ctx, out->total, what)) != FG_OK) return rc;
+    if ((rc = scratch_get(ctx, src, ctx->grains, std::max<size_t>((size_t)out->total, 1) * sizeof(float4), &grains_p,
                           what)) != FG_OK)
         return rc;
-    float4 *grains = static_cast<float4 *>(grains_p);
-    e = fg::launch_bin_grains(a, g, dist_kind, T, start, mask, grains, s);
-    if (e != hipSuccess) return hip_error(ctx, e, what);
-    out->T = T;
-    out->start = start;
-    out->mask = mask;
-    out->grains = grains;
-    out->total = total;
-    return FG_OK;
+    out->grains = static_cast<float4 *>(grains_p);
+    e = fg::launch_bin_grains(a, g, dist_kind, out->T, out->start, out->mask, out->grains, s);
+    return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
+}
+
+// The sample table of a render's whole offset set, ranked before the call
+// waits for the offsets' range (the rank needs neither).
+int rank_samples(fg_ctx *ctx, ScratchSource &src, const fg_plane_desc *d, const float *d_offs, hipStream_t s,
+                 void **samples, const char *what)
+{
+    const int q = sample_buckets(d->n_samples);
+    const int rc = scratch_get(ctx, src, ctx->samples, fg::sample_table_bytes((int)d->n_samples, q), samples, what);
+    if (rc != FG_OK) return rc;
+    fg::SampleTable t{};
+    fg::sample_table_layout(*samples, (int)d->n_samples, q, &t);
+    const hipError_t e = fg::launch_sample_rank(reinterpret_cast<const float2 *>(d_offs), d->zoom, t, s);
+    return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
 }
 
 // Per-plane generation into HBM, then the splat-from-HBM kernel.  With an
 // arena, every scratch buffer comes from it and nothing is allocated.
+// samples: the table rank_samples filled.
 int run_pixel_hbm(fg_ctx *ctx, fg::PixelArgs &a, const fg::PixGeom &g, const float4 &range, int dist_kind,
-                  int block, hipStream_t s, ScratchSource src = ScratchSource(), const PreCounts *pre = nullptr)
+                  int block, void *samples_p, hipStream_t s, ScratchSource src)
 {
     const char *what = "Pixel renderer";
     int rc = FG_OK;
-    // the context's buffers are shared by its calls: wait for the previous
-    // user (an arena's callers are told that overlapping calls race)
-    if (!src.arena && (rc = scratch_acquire(ctx, what)) != FG_OK) return rc;
     float eps, safe_r;
     splat_bounds(a, g, range, &eps, &safe_r);
     Tables tab = plan_tables(a, eps, safe_r, a.budget != nullptr);
-    void *samples_p, *levels_p, *lists_p = nullptr;
+    void *levels_p, *lists_p = nullptr;
     const size_t tile_level_b = a.budget ? (size_t)a.n_tiles : 0;
-    if ((rc = scratch_get(ctx, src, ctx->samples,
-                          fg::sample_table_bytes(a.n_samples, sample_buckets((uint32_t)a.n_samples)), &samples_p,
-                          what)) != FG_OK)
-        return rc;
     if ((rc = scratch_get(ctx, src, ctx->levels, tab.level_bytes + tile_level_b, &levels_p, what)) != FG_OK) return rc;
     if (tab.lists()) {
         if ((rc = scratch_get(ctx, src, ctx->cells, tab.list_bytes, &lists_p, what)) != FG_OK) return rc;
@@ -812,37 +888,37 @@ int run_pixel_hbm(fg_ctx *ctx, fg::PixelArgs &a, const fg::PixGeom &g, const flo
     a.level_tables = tab.set.store;
     mark(ctx, 0, s);
     HbmGen gen;
-    if ((rc = hbm_generate(ctx, src, a, g, dist_kind, s, &gen, pre)) != FG_OK) return rc;
-    uint32_t *start = gen.start;
-    const float4 *grains = gen.grains;
-    // heaviest-first tile order: weights and ids (in, out), sort workspace
-    TileOrder order;
-    void *tiles_p, *tile_temp_p;
-    size_t sort_temp = 0;
-    hipError_t e = fg::sort_tiles(nullptr, &sort_temp, nullptr, nullptr, nullptr, nullptr, a.n_tiles, s);
-    if (e != hipSuccess) return hip_error(ctx, e, what);
-    if ((rc = scratch_get(ctx, src, ctx->tiles, (size_t)a.n_tiles * 16, &tiles_p, what)) != FG_OK) return rc;
-    if ((rc = scratch_get(ctx, src, ctx->tile_temp, sort_temp, &tile_temp_p, what)) != FG_OK) return rc;
-    {
-        unsigned char *p = static_cast<unsigned char *>(tiles_p);
-        order.w = reinterpret_cast<uint32_t *>(p);
-        order.w_sorted = reinterpret_cast<uint32_t *>(p + (size_t)a.n_tiles * 4);
-        order.ids = reinterpret_cast<int *>(p + (size_t)a.n_tiles * 8);
-        order.order = reinterpret_cast<int *>(p + (size_t)a.n_tiles * 12);
-    }
-    // one sample table per level (the first 16, 32, ... samples, then all;
-    // all alone without budgets), their lists, and with budgets each tile's
-    // level
-    e = fg::launch_sample_rank(a.offs, a.zoom, tab.set.full, s);
-    if (e == hipSuccess) e = launch_tables(tab, lists_p != nullptr, a.status, s);
+    if ((rc = hbm_count(ctx, src, a, g, s, &gen)) != FG_OK) return rc;
+    // The sample tables while the host waits for the total: one per level (the
+    // first 16, 32, ... samples, then all; all alone without budgets), their
+    // lists, and with budgets each tile's level.
+    hipError_t e = launch_tables(tab, lists_p != nullptr, a.status, s);
     if (e == hipSuccess && a.budget) {
         uint8_t *tile_level = static_cast<uint8_t *>(levels_p) + tab.level_bytes;
         a.tile_level = tile_level;
         e = fg::launch_tile_levels(a, tab.set, tile_level, s);
     }
-    if (e == hipSuccess) e = fg::launch_pixel_tile_weights(a, g, start, order.w, order.ids, s);
-    if (e == hipSuccess)
-        e = fg::sort_tiles(tile_temp_p, &sort_temp, order.w, order.w_sorted, order.ids, order.order, a.n_tiles, s);
+    if (e != hipSuccess) return hip_error(ctx, e, what);
+    if ((rc = hbm_draw(ctx, src, a, g, dist_kind, s, &gen)) != FG_OK) return rc;
+    const uint32_t *start = gen.start;
+    const float4 *grains = gen.grains;
+    // heaviest-first tile order
+    TileOrder order;
+    void *tiles_p;
+    if ((rc = scratch_get(ctx, src, ctx->tiles, (size_t)a.n_tiles * 16, &tiles_p, what)) != FG_OK) return rc;
+    order.place(tiles_p, a.n_tiles);
+    if (a.n_tiles <= fg::kOrderTiles) {
+        e = fg::launch_tile_order(a, g, start, order.order, s);
+    } else {
+        size_t sort_temp = 0;
+        void *tile_temp_p;
+        e = fg::sort_tiles(nullptr, &sort_temp, nullptr, nullptr, nullptr, nullptr, a.n_tiles, s);
+        if (e != hipSuccess) return hip_error(ctx, e, what);
+        if ((rc = scratch_get(ctx, src, ctx->tile_temp, sort_temp, &tile_temp_p, what)) != FG_OK) return rc;
+        e = fg::launch_pixel_tile_weights(a, g, start, order.w, order.ids, s);
+        if (e == hipSuccess)
+            e = fg::sort_tiles(tile_temp_p, &sort_temp, order.w, order.w_sorted, order.ids, order.order, a.n_tiles, s);
+    }
     a.tile_list = order.order;
     mark(ctx, 1, s);
     mark(ctx, 2, s);
@@ -908,15 +984,23 @@ int do_pixelwise_budget(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lamb
     int variant = stats ? 1 : pixel_variant(ctx, d);
     if (budget && variant != 3)
         return set_error(ctx, FG_EINVAL, "adaptive sampling needs the HBM splat formulation (n_samples <= 2048)");
+    const char *what = "Pixel renderer";
     fg::PixGeom geom{};
     float4 range{};
-    hipError_t e = fg::launch_offsets_range(reinterpret_cast<const float2 *>(d_offs), (int)d->n_samples,
-                                            ctx->d_range, s);
-    if (e != hipSuccess) return hip_error(ctx, e, "Pixel renderer");
+    void *samples_p = nullptr;
+    uint32_t seq = 0;
+    // the context's buffers are shared by its calls
+    int rc0 = scratch_acquire_on(ctx, s, what);
+    if (rc0 != FG_OK) return rc0;
+    ScratchGuard guard{ctx, s};
+    hipError_t e = enqueue_range(ctx, d_offs, (int)d->n_samples, s, &seq);
+    if (e != hipSuccess) return hip_error(ctx, e, what);
     if (variant == 3) {
-        e = hipMemcpyAsync(&range, ctx->d_range, sizeof range, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return hip_error(ctx, e, "Pixel renderer");
+        ScratchSource src;
+        if ((rc0 = rank_samples(ctx, src, d, d_offs, s, &samples_p, what)) != FG_OK) return rc0;
+        e = read_range(ctx, seq, s, &range);
+        if (e != hipSuccess) return hip_error(ctx, e, what);
+        ctx->scratch_pending = false;  // s waited for the previous user before the range
         if (!plane_geometry(d, range, &geom)) variant = 2;
     }
     int tw, th, lds;
@@ -925,7 +1009,7 @@ int do_pixelwise_budget(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lamb
         return set_error(ctx, FG_EINVAL, "adaptive sampling: the plane's cell grid does not fit the HBM splat path");
     if (variant != 3) pixel_config(ctx, d, variant, &tw, &th, &lds);
     fg::PixelArgs a{};
-    int rc0 = pixel_args(ctx, d, d_lambda, d_offs, d_out, tw, th, lds, ctx->d_range, ctx->d_status, &a);
+    rc0 = pixel_args(ctx, d, d_lambda, d_offs, d_out, tw, th, lds, ctx->d_range, ctx->d_status, &a);
     if (rc0 != FG_OK) return rc0;
     a.budget = budget;
     const size_t bits = (((size_t)tw * th * a.words * 4) + 15) & ~(size_t)15;
@@ -936,7 +1020,12 @@ int do_pixelwise_budget(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lamb
                      bits + (size_t)d->n_samples * 8 + min_grains * 32 <= (size_t)lds) ? 1 : 0;
     if (splat && bits + (a.offs_in_lds ? (size_t)d->n_samples * 8 : 0) + min_grains * 32 > (size_t)lds)
         return set_error(ctx, FG_EINVAL, "sample count too large for one pixel-wise tile");
-    if (variant == 3) return run_pixel_hbm(ctx, a, geom, range, (int)d->dist_kind, splat_hbm_block(ctx, d), s);
+    if (variant == 3) {
+        rc0 = run_pixel_hbm(ctx, a, geom, range, (int)d->dist_kind, splat_hbm_block(ctx, d), samples_p, s,
+                            ScratchSource());
+        guard.armed = rc0 != FG_OK;
+        return rc0;
+    }
     mark(ctx, 0, s);
     e = fg::launch_lambda_check(d_lambda, (long long)d->in_w * d->in_h, a.status, s);
     if (e != hipSuccess) return hip_error(ctx, e, "Pixel renderer");
@@ -969,12 +1058,21 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
     fg::PixGeom geom{};
     int tw = 0, th = 0, lds = 0;
     bool joint = n > 1 && n <= fg::kFramePlanes && variant == 3;
+    void *samples_p = nullptr;
+    ScratchGuard guard{ctx, s, false};
+    int rc;
     if (joint) {
-        hipError_t e = fg::launch_offsets_range(reinterpret_cast<const float2 *>(d_offs), (int)d->n_samples,
-                                                ctx->d_range, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(&range, ctx->d_range, sizeof range, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        // the previous call's kernels may still read the context's buffers
+        if ((rc = scratch_acquire_on(ctx, s, what)) != FG_OK) return rc;
+        guard.armed = true;
+        uint32_t seq = 0;
+        hipError_t e = enqueue_range(ctx, d_offs, (int)d->n_samples, s, &seq);
         if (e != hipSuccess) return hip_error(ctx, e, what);
+        ScratchSource src;
+        if ((rc = rank_samples(ctx, src, d, d_offs, s, &samples_p, what)) != FG_OK) return rc;
+        e = read_range(ctx, seq, s, &range);
+        if (e != hipSuccess) return hip_error(ctx, e, what);
+        ctx->scratch_pending = false;  // s waited for the previous user before the range
         joint = plane_geometry(d, range, &geom) && hbm_config(ctx, d, &tw, &th, &lds, 4LL * ctx->num_cus);
     }
     if (!joint) {
@@ -989,42 +1087,42 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
         const int rc = pixel_args(ctx, d, lams[i], d_offs, outs[i], tw, th, lds, ctx->d_range, ctx->d_status, &a[i]);
         if (rc != FG_OK) return rc;
     }
-    // The frame's pipeline: thresholds and the joint count, every plane's
-    // scan, one host read of all the grain totals (their sizes), then each
-    // plane's draws and tile order, one sample table and its candidate lists
-    // for all the planes (they share the offsets), and the splats.  Every
-    // plane has its own bin starts, grains and tile order, so nothing waits
-    // for a plane's splat; the previous call's kernels may still read the
-    // context's buffers, hence the one acquire.
-    int rc = scratch_acquire(ctx, what);
-    if (rc != FG_OK) return rc;
+    // The frame's pipeline: thresholds and the joint count, the planes' scans
+    // with one wait for all their grain totals (their sizes), during which one
+    // sample table and its candidate lists are built for all the planes (they
+    // share the offsets), then each plane's draws, and the splats.  Every
+    // plane has its own bin starts and grains, so nothing waits for a plane's
+    // splat.
     const int kind = (int)d->dist_kind, block = splat_hbm_block(ctx, d);
     const long long nbins = (long long)geom.nbx * geom.nby;
     const size_t t_b = align256((size_t)d->in_w * d->in_h * sizeof(double));
     const size_t c_b = align256((size_t)(nbins + 1) * 4), m_b = align256((size_t)nbins * 32);
-    const size_t per_plane = t_b + 2 * c_b + m_b;  // thresholds | counts | starts | masks
-    if ((rc = ensure_bytes(ctx, ctx->plane_counts, 256 + (size_t)n * per_plane, what)) != FG_OK) return rc;
+    const size_t s_b = align256(fg::bin_scan_partials(nbins) * 8);
+    const size_t per_plane = t_b + 2 * c_b + m_b + s_b;  // thresholds | counts | starts | masks | scan sums
+    if ((rc = ensure_bytes(ctx, ctx->plane_counts, (size_t)n * per_plane, what)) != FG_OK) return rc;
     unsigned char *base = static_cast<unsigned char *>(ctx->plane_counts.p);
-    unsigned long long *d_tot = reinterpret_cast<unsigned long long *>(base);  // the planes' grain totals
-    uint32_t *start[fg::kFramePlanes];
-    PreCounts pre[fg::kFramePlanes];
+    double *T[fg::kFramePlanes];
+    unsigned long long *mask[fg::kFramePlanes];
     fg::FramePlanes fp{};
+    fg::BinScan scan{};
+    scan.n = nbins;
+    scan.planes = n;
+    scan.pub = ctx->d_pub;
+    scan.seq = ++ctx->pub_seq;
     for (int i = 0; i < n; ++i) {
-        unsigned char *b = base + 256 + (size_t)i * per_plane;
-        pre[i].T = reinterpret_cast<double *>(b);
-        pre[i].cnt = reinterpret_cast<uint32_t *>(b + t_b);
-        start[i] = reinterpret_cast<uint32_t *>(b + t_b + c_b);
-        pre[i].mask = reinterpret_cast<unsigned long long *>(b + t_b + 2 * c_b);
-        fp.T[i] = pre[i].T;
-        fp.cnt[i] = pre[i].cnt;
-        fp.mask[i] = pre[i].mask;
+        unsigned char *b = base + (size_t)i * per_plane;
+        T[i] = reinterpret_cast<double *>(b);
+        uint32_t *cnt = reinterpret_cast<uint32_t *>(b + t_b);
+        mask[i] = reinterpret_cast<unsigned long long *>(b + t_b + 2 * c_b);
+        fp.T[i] = T[i];
+        fp.cnt[i] = cnt;
+        fp.mask[i] = mask[i];
+        scan.in[i] = cnt;
+        scan.out[i] = reinterpret_cast<uint32_t *>(b + t_b + c_b);
+        scan.partials[i] = reinterpret_cast<unsigned long long *>(b + t_b + 2 * c_b + m_b);
     }
-    // the rest of the scratch, sized before any kernel of this call runs
+    // the rest of the scratch, sized before any kernel of this call uses it
     // (growing a buffer frees the old one)
-    size_t scan_bytes = 0;
-    hipError_t e = fg::scan_bins(nullptr, &scan_bytes, nullptr, nullptr, (int)(nbins + 1), s);
-    if (e != hipSuccess) return hip_error(ctx, e, what);
-    const int q = sample_buckets((uint32_t)d->n_samples);
     float eps, safe_r;
     splat_bounds(a[0], geom, range, &eps, &safe_r);
     Tables tab = plan_tables(a[0], eps, safe_r, false);
@@ -1034,28 +1132,23 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
     const int n_items = n * a[0].n_tiles;
     const size_t rec_b = align256(sizeof(fg::BatchPlane) * fg::kFramePlanes);
     const size_t items_b = align256((size_t)n_items * sizeof(int2)), w_b = align256((size_t)n_items * 4);
-    if ((rc = ensure_bytes(ctx, ctx->scan_temp, scan_bytes, what)) != FG_OK) return rc;
     if ((rc = ensure_bytes(ctx, ctx->tiles, rec_b + items_b + w_b + 256, what)) != FG_OK) return rc;
-    if ((rc = ensure_bytes(ctx, ctx->samples, fg::sample_table_bytes((int)d->n_samples, q), what)) != FG_OK) return rc;
     if ((rc = ensure_bytes(ctx, ctx->levels, tab.level_bytes, what)) != FG_OK) return rc;
     if (lists && (rc = ensure_bytes(ctx, ctx->cells, tab.list_bytes, what)) != FG_OK) return rc;
-    place_tables(tab, ctx->samples.p, ctx->levels.p, lists ? ctx->cells.p : nullptr);
+    place_tables(tab, samples_p, ctx->levels.p, lists ? ctx->cells.p : nullptr);
     mark(ctx, 0, s);
-    for (int i = 0; i < n && e == hipSuccess; ++i) e = fg::launch_threshold(a[i], pre[i].T, s);
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < n && e == hipSuccess; ++i) e = fg::launch_threshold(a[i], T[i], s);
     if (e == hipSuccess) e = fg::launch_bin_count_planes(a[0], geom, fp, n, s);
-    // totals (cleared by a kernel, as the single-plane path does) and scans
-    if (e == hipSuccess) e = fg::launch_fill_u32(reinterpret_cast<uint32_t *>(d_tot), 2 * n, 0u, s);
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
-        e = fg::launch_fill_u32(pre[i].cnt + nbins, 1, 0u, s);
-        if (e == hipSuccess) e = fg::launch_sum_u64(pre[i].cnt, nbins, d_tot + i, s);
-        if (e == hipSuccess)
-            e = fg::scan_bins(ctx->scan_temp.p, &scan_bytes, pre[i].cnt, start[i], (int)(nbins + 1), s);
-    }
+    if (e == hipSuccess) e = fg::launch_bin_scan(scan, s);
+    if (e == hipSuccess) e = launch_tables(tab, lists, a[0].status, s);
     unsigned long long total[fg::kFramePlanes] = {};
-    if (e == hipSuccess) e = hipMemcpyAsync(total, d_tot, sizeof(unsigned long long) * n, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    for (int i = 0; i < n && e == hipSuccess; ++i) {
+        e = wait_published(&ctx->h_pub->total_seq[i], scan.seq, s);
+        total[i] = ctx->h_pub->total[i];
+    }
     if (e != hipSuccess) return hip_error(ctx, e, what);
-    // the grain array of all the planes (nothing of this call runs now)
+    // the grain array of all the planes (nothing of this call uses it yet)
     size_t goff[fg::kFramePlanes], gsum = 0;
     for (int i = 0; i < n; ++i) {
         if ((rc = check_total(ctx, total[i], what)) != FG_OK) return rc;
@@ -1064,12 +1157,9 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
     }
     if ((rc = ensure_bytes(ctx, ctx->grains, std::max<size_t>(gsum, 1) * sizeof(float4), what)) != FG_OK) return rc;
     float4 *grains = static_cast<float4 *>(ctx->grains.p);
-    // one sample table and its candidate lists
-    e = fg::launch_sample_rank(a[0].offs, a[0].zoom, tab.set.full, s);
-    if (e == hipSuccess) e = launch_tables(tab, lists, a[0].status, s);
     fg::FramePlaneRecords rec{};
     for (int i = 0; i < n && e == hipSuccess; ++i) {
-        e = fg::launch_bin_grains(a[i], geom, kind, pre[i].T, start[i], pre[i].mask, grains + goff[i], s);
+        e = fg::launch_bin_grains(a[i], geom, kind, T[i], scan.out[i], mask[i], grains + goff[i], s);
         if (lists) {
             a[i].cl_q = tab.lp.q;
             a[i].cl_classes = tab.lp.classes;
@@ -1079,7 +1169,7 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
         bp.a = a[i];
         bp.geo = geom;
         bp.st = tab.set.t[0];
-        bp.bin_start = start[i];
+        bp.bin_start = scan.out[i];
         bp.grains = grains + goff[i];
         bp.item_base = (long long)i * a[i].n_tiles;
     }
@@ -1101,6 +1191,7 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
     if (e == hipSuccess) e = fg::launch_splat_batch(d_planes, items, n_items, counter, grid, block, a[0].lds_bytes, s);
     mark(ctx, 3, s);
     if (e != hipSuccess) return hip_error(ctx, e, what);
+    guard.armed = false;
     return scratch_release(ctx, s, what);
 }
 
@@ -1199,8 +1290,9 @@ int do_grainwise(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lambda, con
     const char *what = "Grain renderer";
     if (variant == 2) {
         // the sample order lives in the context's scratch
-        int rc = scratch_acquire(ctx, what);
+        int rc = scratch_acquire_on(ctx, s, what);
         if (rc != FG_OK) return rc;
+        ScratchGuard guard{ctx, s};
         const int q = sample_buckets(d->n_samples);
         if ((rc = ensure_bytes(ctx, ctx->samples, fg::sample_table_bytes(a.n_samples, q), what)) != FG_OK)
             return rc;
@@ -1261,6 +1353,7 @@ int do_grainwise(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lambda, con
         if (e == hipSuccess) e = fg::launch_grainwise_sorted(a, st, (int)d->dist_kind, grain_block(ctx, d), s);
         mark(ctx, 3, s);
         if (e != hipSuccess) return hip_error(ctx, e, what);
+        guard.armed = false;
         return scratch_release(ctx, s, what);
     }
     hipError_t e = fg::launch_offsets_range(a.offs, a.n_samples, ctx->d_range, s);
@@ -1848,7 +1941,6 @@ int fg_ctx_create(int device_ordinal, fg_ctx **out)
     }
     if (e == hipSuccess) e = hipMalloc(&ctx->d_status, sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&ctx->d_stats, 4 * sizeof(unsigned long long));
-    if (e == hipSuccess) e = hipMalloc(&ctx->d_sum64, 2 * sizeof(unsigned long long));
     // this device's copy of the allocation-free entry point's scratch (the
     // device is current)
     if (e == hipSuccess) e = hipGetSymbolAddress(reinterpret_cast<void **>(&ctx->noalloc_scratch), HIP_SYMBOL(scratch));
@@ -1859,6 +1951,12 @@ int fg_ctx_create(int device_ordinal, fg_ctx **out)
     if (e == hipSuccess) {
         *ctx->h_cancel = 0;
         e = hipHostGetDevicePointer((void **)&ctx->d_cancel, ctx->h_cancel, 0);
+    }
+    if (e == hipSuccess)
+        e = hipHostMalloc((void **)&ctx->h_pub, sizeof(fg::HostPublish), hipHostMallocCoherent | hipHostMallocMapped);
+    if (e == hipSuccess) {
+        std::memset(ctx->h_pub, 0, sizeof(fg::HostPublish));
+        e = hipHostGetDevicePointer((void **)&ctx->d_pub, ctx->h_pub, 0);
     }
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) {
@@ -1877,9 +1975,9 @@ void fg_ctx_destroy(fg_ctx *ctx)
     free_buffers(ctx);
     (void)hipFree(ctx->d_status);
     (void)hipFree(ctx->d_stats);
-    (void)hipFree(ctx->d_sum64);
     (void)hipFree(ctx->d_range);
     if (ctx->h_cancel) (void)hipHostFree(ctx->h_cancel);
+    if (ctx->h_pub) (void)hipHostFree(ctx->h_pub);
     if (ctx->scratch_done) (void)hipEventDestroy(ctx->scratch_done);
     for (hipEvent_t ev : ctx->tev)
         if (ev) (void)hipEventDestroy(ev);
@@ -1955,11 +2053,16 @@ int fg_render_pixelwise_device_noalloc(fg_ctx *ctx, const fg_plane_desc *desc, c
     if (e != hipSuccess) return hip_error(ctx, e, what);
     if (!ctx->noalloc_scratch) return set_error(ctx, FG_EHIP, std::string(what) + ": no scratch address");
     hipStream_t s = reinterpret_cast<hipStream_t>(hip_stream);
+    ScratchSource src;
+    src.arena = ctx->noalloc_scratch;
+    src.cap = kNoAllocScratchBytes;
     float4 range{};
-    e = fg::launch_offsets_range(reinterpret_cast<const float2 *>(d_offsets_input_xy), (int)desc->n_samples,
-                                 ctx->d_range, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&range, ctx->d_range, sizeof range, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    void *samples_p = nullptr;
+    uint32_t seq = 0;
+    e = enqueue_range(ctx, d_offsets_input_xy, (int)desc->n_samples, s, &seq);
+    if (e != hipSuccess) return hip_error(ctx, e, what);
+    if ((rc = rank_samples(ctx, src, desc, d_offsets_input_xy, s, &samples_p, what)) != FG_OK) return rc;
+    e = read_range(ctx, seq, s, &range);
     if (e != hipSuccess) return hip_error(ctx, e, what);
     fg::PixGeom geom{};
     int tw, th, lds;
@@ -1969,10 +2072,7 @@ int fg_render_pixelwise_device_noalloc(fg_ctx *ctx, const fg_plane_desc *desc, c
     if ((rc = pixel_args(ctx, desc, d_lambda, d_offsets_input_xy, d_out, tw, th, lds, ctx->d_range, ctx->d_status,
                          &a)) != FG_OK)
         return rc;
-    ScratchSource src;
-    src.arena = ctx->noalloc_scratch;
-    src.cap = kNoAllocScratchBytes;
-    return run_pixel_hbm(ctx, a, geom, range, (int)desc->dist_kind, splat_hbm_block(ctx, desc), s, src);
+    return run_pixel_hbm(ctx, a, geom, range, (int)desc->dist_kind, splat_hbm_block(ctx, desc), samples_p, s, src);
 }
 
 int fg_render_pixelwise_adaptive_device(fg_ctx *ctx, const fg_plane_desc *desc, const float *d_lambda,
@@ -2441,11 +2541,11 @@ int fg_pixelwise_grains(fg_ctx *ctx, const fg_plane_desc *desc, const float *d_l
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_error(ctx, e, what);
     hipStream_t s = ctx->stream;
+    if ((rc = scratch_acquire(ctx, what)) != FG_OK) return rc;
     float4 range{};
-    e = fg::launch_offsets_range(reinterpret_cast<const float2 *>(d_offsets_input_xy), (int)desc->n_samples,
-                                 ctx->d_range, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&range, ctx->d_range, sizeof range, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    uint32_t seq = 0;
+    e = enqueue_range(ctx, d_offsets_input_xy, (int)desc->n_samples, s, &seq);
+    if (e == hipSuccess) e = read_range(ctx, seq, s, &range);
     if (e != hipSuccess) return hip_error(ctx, e, what);
     fg::PixGeom geom{};
     int tw, th, lds;
@@ -2455,10 +2555,10 @@ int fg_pixelwise_grains(fg_ctx *ctx, const fg_plane_desc *desc, const float *d_l
     if ((rc = pixel_args(ctx, desc, d_lambda, d_offsets_input_xy, nullptr, tw, th, lds, ctx->d_range, ctx->d_status,
                          &a)) != FG_OK)
         return rc;
-    if ((rc = scratch_acquire(ctx, what)) != FG_OK) return rc;
     ScratchSource src;
     HbmGen gen;
-    if ((rc = hbm_generate(ctx, src, a, geom, (int)desc->dist_kind, s, &gen)) != FG_OK) return rc;
+    if ((rc = hbm_count(ctx, src, a, geom, s, &gen)) != FG_OK) return rc;
+    if ((rc = hbm_draw(ctx, src, a, geom, (int)desc->dist_kind, s, &gen)) != FG_OK) return rc;
     *n_grains = gen.total;
     origin[0] = geom.Ix0;
     origin[1] = geom.Jy0;

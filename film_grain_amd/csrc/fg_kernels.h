@@ -103,8 +103,18 @@ struct GrainArgs {
     float r_list;
 };
 
-// Writes (min x, max x, min y, max y) of n (x, y) pairs to *range (one workgroup).
-hipError_t launch_offsets_range(const float2 *offs, int n, float4 *range, hipStream_t s);
+// Values kernels hand to the host without a copy: coherent pinned host memory
+// that a kernel writes, each value followed by its flag (the call's sequence
+// number, with release order), and the host polls.
+struct HostPublish {
+    float range[4];
+    unsigned long long total[4];
+    uint32_t range_seq, total_seq[4];
+};
+// Writes (min x, max x, min y, max y) of n (x, y) pairs to *range, and to pub
+// under seq if that is given (one workgroup).
+hipError_t launch_offsets_range(const float2 *offs, int n, float4 *range, hipStream_t s, HostPublish *pub = nullptr,
+                                uint32_t seq = 0);
 // variant: 0 splat (default), 1 gather.  Stats always use the gather kernel.
 hipError_t launch_pixelwise(const PixelArgs &a, int dist_kind, int variant, bool with_stats,
                             hipStream_t s);

@@ -424,7 +424,8 @@ __global__ __launch_bounds__(kBlock) void pixelwise_splat(PixelArgs a)
     }
 }
 
-__global__ __launch_bounds__(kBlock) void offsets_range_kernel(const float2 *offs, int n, float4 *range)
+__global__ __launch_bounds__(kBlock) void offsets_range_kernel(const float2 *offs, int n, float4 *range, HostPublish *pub,
+                                                               uint32_t seq)
 {
     __shared__ float4 s_r[kBlock];
     float4 r = make_float4(INFINITY, -INFINITY, INFINITY, -INFINITY);
@@ -449,12 +450,22 @@ __global__ __launch_bounds__(kBlock) void offsets_range_kernel(const float2 *off
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) *range = s_r[0];
+    if (threadIdx.x == 0) {
+        const float4 v = s_r[0];
+        *range = v;
+        if (pub) {
+            const float f[4] = {v.x, v.y, v.z, v.w};
+            for (int i = 0; i < 4; ++i)
+                __hip_atomic_store(&pub->range[i], f[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(&pub->range_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
 }
 
-hipError_t launch_offsets_range(const float2 *offs, int n, float4 *range, hipStream_t s)
+hipError_t launch_offsets_range(const float2 *offs, int n, float4 *range, hipStream_t s, HostPublish *pub,
+                                uint32_t seq)
 {
-    hipLaunchKernelGGL(offsets_range_kernel, dim3(1), dim3(kBlock), 0, s, offs, n, range);
+    hipLaunchKernelGGL(offsets_range_kernel, dim3(1), dim3(kBlock), 0, s, offs, n, range, pub, seq);
     return hipGetLastError();
 }
 

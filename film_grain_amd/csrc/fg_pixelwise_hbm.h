@@ -95,8 +95,6 @@ hipError_t launch_threshold(const PixelArgs &a, double *T, hipStream_t s);
 // bin_mask: four 64-bit words per bin, the nonempty cells (bin_grains reads them).
 hipError_t launch_bin_count(const PixelArgs &a, const PixGeom &g, const double *T, uint32_t *bin_count,
                             unsigned long long *bin_mask, hipStream_t s);
-// hipCUB exclusive sum; with temp == nullptr only sets *temp_bytes.
-hipError_t scan_bins(void *temp, size_t *temp_bytes, const uint32_t *in, uint32_t *out, int n, hipStream_t s);
 // The planes of one frame (same seed and geometry): their thresholds, and
 // where their bin counts and nonempty masks go.
 constexpr int kFramePlanes = 3;
@@ -105,6 +103,20 @@ struct FramePlanes {
     uint32_t *cnt[kFramePlanes];
     unsigned long long *mask[kFramePlanes];
 };
+// Exclusive scans of the planes' bin counts (n bins; out has n + 1 entries,
+// out[n] the total in 32 bits), with each plane's 64-bit total published to
+// pub under seq; partials: bin_scan_partials(n) words a plane.
+struct BinScan {
+    const uint32_t *in[kFramePlanes];
+    uint32_t *out[kFramePlanes];
+    unsigned long long *partials[kFramePlanes];
+    long long n;
+    HostPublish *pub;
+    uint32_t seq;
+    int planes;
+};
+size_t bin_scan_partials(long long n);
+hipError_t launch_bin_scan(const BinScan &b, hipStream_t s);
 // bin_count for n_planes (1..3) planes in one pass: each cell hashed once
 // (the planes' cell streams are the same), counted against every plane's
 // threshold.
@@ -140,6 +152,9 @@ hipError_t launch_pixel_tile_weights(const PixelArgs &a, const PixGeom &g, const
                                      int *ids, hipStream_t s);
 hipError_t sort_tiles(void *temp, size_t *temp_bytes, const uint32_t *w_in, uint32_t *w_out, const int *ids_in,
                       int *ids_out, int n, hipStream_t s);
+// Weights and order of at most kOrderTiles tiles in one launch.
+constexpr int kOrderTiles = 4096;
+hipError_t launch_tile_order(const PixelArgs &a, const PixGeom &g, const uint32_t *bin_start, int *order, hipStream_t s);
 // Grain-wise: w[t] = grains of the input pixels whose grains can reach tile t.
 hipError_t launch_grain_tile_weights(const GrainArgs &a, const SampleTable &st, uint32_t *w, int *ids,
                                      hipStream_t s);

@@ -8,7 +8,7 @@
 //   bin_count   cells of the plane's extended grid (every cell any window can
 //               reach) in 16x16-cell bins, one thread per cell: Poisson counts,
 //               summed per bin
-//   scan        exclusive scan of the bin counts (hipCUB) -> bin_start
+//   scan        exclusive scan of the bin counts -> bin_start
 //   bin_grains  each bin's grains written contiguously at bin_start[bin]: the
 //               non-empty cells' counts and streams first, then the draws,
 //               a lane taking the bin's next cell when its own is done
@@ -1039,18 +1039,7 @@ __global__ __launch_bounds__(kBlock) void pixel_tile_weights_kernel(PixelArgs a,
 {
     const int tile = blockIdx.x * kBlock + threadIdx.x;
     if (tile >= a.n_tiles) return;
-    const int tyi = tile / a.tiles_x, txi = tile - tyi * a.tiles_x;
-    const int X0 = txi * a.tile_w, Y0 = tyi * a.tile_h;
-    const TileRegion r = tile_region(a, geo, X0, Y0, min(X0 + a.tile_w, a.out_w), min(Y0 + a.tile_h, a.out_h));
-    uint32_t sum = 0;
-    if (r.bx0 <= r.bx1)
-        for (int by = r.by0; by <= r.by1; ++by)
-            sum += bin_start[by * geo.nbx + r.bx1 + 1] - bin_start[by * geo.nbx + r.bx0];
-    if (a.budget) {  // adaptive: the work also scales with the tile's samples
-        const int n = reinterpret_cast<const SampleTable *>(a.level_tables)[a.tile_level[tile]].n;
-        sum = (uint32_t)min((unsigned long long)sum * (unsigned long long)n / 16ull, 0xFFFFFFFFull);
-    }
-    w[tile] = sum;
+    w[tile] = tile_weight(a, geo, bin_start, tile);
     ids[tile] = tile;
 }
 
@@ -1721,11 +1710,6 @@ hipError_t launch_bin_count_planes(const PixelArgs &a, const PixGeom &g, const F
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
-}
-
-hipError_t scan_bins(void *temp, size_t *temp_bytes, const uint32_t *in, uint32_t *out, int n, hipStream_t s)
-{
-    return hipcub::DeviceScan::ExclusiveSum(temp, *temp_bytes, in, out, n, s);
 }
 
 hipError_t launch_bin_grains(const PixelArgs &a, const PixGeom &g, int dist_kind, const double *T,

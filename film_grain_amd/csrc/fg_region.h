@@ -39,6 +39,25 @@ __device__ __forceinline__ TileRegion tile_region(const PixelArgs &a, const PixG
     return r;
 }
 
+// Work of a splat tile: the grains of the bins covering its region, times its
+// samples with budgets.
+__device__ __forceinline__ uint32_t tile_weight(const PixelArgs &a, const PixGeom &geo, const uint32_t *bin_start,
+                                                int tile)
+{
+    const int tyi = tile / a.tiles_x, txi = tile - tyi * a.tiles_x;
+    const int X0 = txi * a.tile_w, Y0 = tyi * a.tile_h;
+    const TileRegion r = tile_region(a, geo, X0, Y0, min(X0 + a.tile_w, a.out_w), min(Y0 + a.tile_h, a.out_h));
+    uint32_t sum = 0;
+    if (r.bx0 <= r.bx1)
+        for (int by = r.by0; by <= r.by1; ++by)
+            sum += bin_start[by * geo.nbx + r.bx1 + 1] - bin_start[by * geo.nbx + r.bx0];
+    if (a.budget) {
+        const int n = reinterpret_cast<const SampleTable *>(a.level_tables)[a.tile_level[tile]].n;
+        sum = (uint32_t)min((unsigned long long)sum * (unsigned long long)n / 16ull, 0xFFFFFFFFull);
+    }
+    return sum;
+}
+
 }  // namespace fg
 
 #endif
