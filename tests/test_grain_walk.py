@@ -9,13 +9,14 @@ f32 = np.float32
 
 def members(fx, fy, qa, qb, q, R, eps):
     """splat_lists_body's membership, in its order of operations."""
-    m = f32(2.0 ** -12)
-    w = f32(f32(f32(R + R) + f32(eps + eps)) + f32(f32(f32(1) / f32(q)) + f32(m + m)))
-    dx = (fx - f32(f32(f32(f32(qa) / f32(q)) - R) - f32(eps + m))).astype(f32)
-    dy = (fy - f32(f32(f32(f32(qb) / f32(q)) - R) - f32(eps + m))).astype(f32)
-    dx = (dx - np.floor(dx)).astype(f32)
-    dy = (dy - np.floor(dy)).astype(f32)
-    return (dx <= w) & (dy <= w)
+    half = f32(f32(0.5) / f32(q))
+    reach = f32(R + f32(eps + f32(2.0 ** -12)))
+
+    def beyond(f, c):  # distance from the cell's interval on the unit circle
+        d = (f - f32(f32(f32(c) / f32(q)) + half)).astype(f32)
+        return np.maximum((np.abs((d - np.rint(d)).astype(f32)) - half).astype(f32), f32(0))
+    dx, dy = beyond(fx, qa), beyond(fy, qb)
+    return ((dx * dx).astype(f32) + (dy * dy).astype(f32)).astype(f32) <= f32(reach * reach)
 
 
 def box(t, R):

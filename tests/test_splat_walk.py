@@ -99,6 +99,45 @@ def test_target_from_the_centre_finds_every_passing_pixel(z, out_side):
     assert hits > 0
 
 
+@pytest.mark.parametrize("z,out_side,n", [(0.3, 512, 64), (1.0, 4096, 100), (2.0, 3840, 256), (4.0, 16384, 33)])
+def test_lists_hold_every_passing_sample(z, out_side, n):
+    """Every sample with a pixel that passes the f32 disk test of a narrow
+    grain is in the list of the grain's class and cell, in the kernels'
+    arithmetic."""
+    from tests.test_grain_walk import members
+    rng = np.random.default_rng(int(z * 10) + out_side + n)
+    zf, iz, q = f32(z), f32(f32(1) / f32(z)), 32
+    slack = f32(f32(4e-3) + f32(f32(2e-6) * f32(out_side)))
+    o = rng.normal(0, 0.8 / z, size=(n, 2)).astype(f32)
+    X = (o * zf).astype(f32)
+    fx, fy = ((X[:, i] - np.floor(X[:, i])).astype(f32) for i in (0, 1))
+    c_out = out_side + 4 * z + 8  # splat_bounds, less its margins
+    eps = f32(c_out * 2.0 ** -20 + 2.0 ** -16)
+    hits = 0
+    for i in range(2500):
+        rad = f32(rng.uniform(0.004, (0.5 - float(slack)) * (1 - 1e-6)) / z)
+        if i % 4 == 0:  # at the classes' edges
+            rad = f32((int(rng.integers(1, 31)) / 64 + rng.choice([-1e-6, 0, 1e-6])) / z)
+        g = rng.uniform(0, out_side / z, size=2).astype(f32)
+        if i % 3 == 0:  # sample 0's point at the rim, on a diagonal
+            px = np.floor(g * zf)
+            g = (((px + 0.5) / z) - o[0] + rng.choice([-1, 1], 2) * (rad / np.sqrt(2) * (1 - 1e-6))).astype(f32)
+        b = ((g * zf).astype(f32) - f32(0.5)).astype(f32)
+        rz = f32(f32(rad * zf) + slack)
+        if not rz + rz < 1:
+            continue
+        k = int(f32(rz * f32(2 * q)))
+        f = (-b - np.floor(-b)).astype(f32)
+        qa, qb = (min(int(f32(v * f32(q))), q - 1) for v in f)
+        sel = members(fx, fy, qa, qb, q, f32(f32(k + 1) / f32(2 * q)), eps)
+        near = np.rint(((o + g).astype(f32).astype(np.float64) * z - 0.5)).astype(f32)
+        dx = ((((near + f32(0.5)) * iz).astype(f32) - o).astype(f32) - g).astype(f32)
+        inside = ((dx * dx).astype(f32).sum(axis=1)).astype(f32) <= f32(rad * rad)
+        assert not np.any(inside & ~sel), (i, float(rad))
+        hits += int(inside.sum())
+    assert hits > 0
+
+
 @pytest.mark.parametrize("side,rm,delta", [(64, 0.1, 0.1), (4096, 0.05, 0.05), (4096, 0.3, 0.11), (1500, 0.012, 0.4),
                                            (16000, 0.1, 0.1)])
 def test_points_within_safe_r_have_the_cell_in_their_window(side, rm, delta):
