@@ -649,6 +649,8 @@ hipError_t tile_order_sort(fg_ctx *ctx, int n, const TileOrder &t, hipStream_t s
 // largest rz, 32 x 32 cells, each with its row-bucket counts.
 struct ListPlan {
     int q = 32, classes = 0, ew = 0;
+    float r = 0.0f;  // > 0: the one class's radius in output pixels
+    float inv_dz() const { return r > 0.0f ? 0.0f : (float)(2 * q); }
     // Lists for every table of at most 2048 samples (beyond, the room of
     // N * span^2 entries per class grows past 100 MB).  Short lists pay as
     // well: the splat packs the lists of consecutive grains into its 64-lane
@@ -663,12 +665,26 @@ struct ListPlan {
     }
 };
 
-ListPlan list_plan(const fg::PixelArgs &a, float eps)
+// A constant radius has one class of that radius; a lognormal law has classes
+// up to its clamp radius, or the largest narrow one.  A grain's class takes
+// its radius alone: the slack of its candidate box (4e-3 and more) is for the
+// box, not for the disk test, and a class of the radius with it was one too
+// wide for half of the grains.  (Classes by the widened radius, also for a
+// constant one: adaptive 1080p RGB 17.1 ms, now 16.3; 4K RGB at N = 256 14.3
+// and 14.0; 256x256 constant 280 and 269 us.  q = 64 instead of 32: 17.8, 14.0
+// and 274, the batch of 12 uneven planes 11.3 ms for 9.2.)
+ListPlan list_plan(const fg::PixelArgs &a, float eps, int dist_kind)
 {
     ListPlan lp;
-    const float slack = 4e-3f + 2e-6f * (float)std::max(a.out_w, a.out_h);
-    lp.classes = std::max(1, std::min(32, (int)std::ceil(std::min(a.rm * a.zoom + slack, 0.5f) * 64.0f)));
     lp.ew = (int)std::ceil((2.0 * (double)eps + std::ldexp(1.0, -11)) * lp.q + 0.01);
+    const float r = a.r_const * a.zoom;
+    if (dist_kind == 0 && r > 0.0f && r < 0.5f) {
+        lp.classes = 1;
+        lp.r = r;
+        lp.ew += (int)std::ceil(2.0 * (double)r * lp.q) - 1;
+    } else {
+        lp.classes = std::min(32, (int)(std::min(a.rm * a.zoom, 0.5f) * (float)(2 * lp.q)) + 1);
+    }
     return lp;
 }
 
@@ -693,15 +709,16 @@ struct Tables {
     bool lists() const { return list_bytes > 0 && list_bytes < ((size_t)1 << 32); }
 };
 
-Tables plan_tables(const fg::PixelArgs &a, float eps, float safe_r, bool levels)
+Tables plan_tables(const fg::PixelArgs &a, int dist_kind, float eps, float safe_r, bool levels)
 {
     Tables t;
     fg::LevelSet &set = t.set;
     if (levels)
         for (int l = 16; l < a.n_samples; l *= 2) set.level_n[set.n++] = l;
     set.level_n[set.n++] = a.n_samples;
-    t.lp = list_plan(a, eps);
+    t.lp = list_plan(a, eps, dist_kind);
     set.classes = t.lp.classes;
+    set.r_const = t.lp.r;
     t.level_bytes = (sizeof(fg::SampleTable) * set.n + 255) & ~(size_t)255;
     for (int l = 0; l < set.n; ++l) {
         const int n = set.level_n[l];
@@ -873,7 +890,7 @@ int run_pixel_hbm(fg_ctx *ctx, fg::PixelArgs &a, const fg::PixGeom &g, const flo
     int rc = FG_OK;
     float eps, safe_r;
     splat_bounds(a, g, range, &eps, &safe_r);
-    Tables tab = plan_tables(a, eps, safe_r, a.budget != nullptr);
+    Tables tab = plan_tables(a, dist_kind, eps, safe_r, a.budget != nullptr);
     void *levels_p, *lists_p = nullptr;
     const size_t tile_level_b = a.budget ? (size_t)a.n_tiles : 0;
     if ((rc = scratch_get(ctx, src, ctx->levels, tab.level_bytes + tile_level_b, &levels_p, what)) != FG_OK) return rc;
@@ -881,7 +898,7 @@ int run_pixel_hbm(fg_ctx *ctx, fg::PixelArgs &a, const fg::PixGeom &g, const flo
         if ((rc = scratch_get(ctx, src, ctx->cells, tab.list_bytes, &lists_p, what)) != FG_OK) return rc;
         a.cl_q = tab.lp.q;
         a.cl_classes = tab.lp.classes;
-        a.cl_inv_dz = (float)(2 * tab.lp.q);
+        a.cl_inv_dz = tab.lp.inv_dz();
     }
     place_tables(tab, samples_p, levels_p, lists_p);
     const fg::SampleTable &st = tab.set.t[tab.set.n - 1];
@@ -1125,7 +1142,7 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
     // (growing a buffer frees the old one)
     float eps, safe_r;
     splat_bounds(a[0], geom, range, &eps, &safe_r);
-    Tables tab = plan_tables(a[0], eps, safe_r, false);
+    Tables tab = plan_tables(a[0], kind, eps, safe_r, false);
     const bool lists = tab.lists();
     // the persistent splat's plane records, (plane, tile) items, their
     // weights and the item counter
@@ -1163,7 +1180,7 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
         if (lists) {
             a[i].cl_q = tab.lp.q;
             a[i].cl_classes = tab.lp.classes;
-            a[i].cl_inv_dz = (float)(2 * tab.lp.q);
+            a[i].cl_inv_dz = tab.lp.inv_dz();
         }
         fg::BatchPlane &bp = rec.p[i];
         bp.a = a[i];
@@ -1714,7 +1731,9 @@ int batch_gen_setup(fg_batch *b, const char *what, hipStream_t s)
         fill[p] = nullptr;
         if (b->list_mem[p]) {
             if (lp.q < 1 || lp.q * lp.q > 65536 || lp.classes < 1) return set_error(b->ctx, FG_EINVAL, "batch list plan");
-            plan[p] = make_int4(lp.q, lp.classes, lp.ew, 0);
+            int r_bits;
+            std::memcpy(&r_bits, &lp.r, sizeof r_bits);
+            plan[p] = make_int4(lp.q, lp.classes, lp.ew, r_bits);
             fill[p] = reinterpret_cast<uint32_t *>(b->list_mem[p]);
             lb = (long long)lp.classes * ((lp.q * lp.q + 63) / 64);
         }
@@ -1825,7 +1844,7 @@ int batch_create(fg_ctx *ctx, const fg_plane_desc *descs, int n, const float *co
             return rc;
         fg::sample_table_layout(b->samples[p], (int)d->n_samples, b->qb[p], &bp.st);
         // candidate lists, built with the plane's table on every run
-        b->list_plans[p] = list_plan(bp.a, bp.st.eps);
+        b->list_plans[p] = list_plan(bp.a, bp.st.eps, (int)d->dist_kind);
         b->list_mem[p] = nullptr;
         const size_t lb = b->list_plans[p].bytes((int)d->n_samples);
         if (lb > 0 && lb < ((size_t)1 << 32)) {
@@ -1836,7 +1855,7 @@ int batch_create(fg_ctx *ctx, const fg_plane_desc *descs, int n, const float *co
             bp.st.cl_list = bp.st.cl_yidx + (size_t)lp.classes * lp.q * lp.q * fg::kRowBuckets;
             bp.a.cl_q = lp.q;
             bp.a.cl_classes = lp.classes;
-            bp.a.cl_inv_dz = (float)(2 * lp.q);
+            bp.a.cl_inv_dz = lp.inv_dz();
         }
     }
     if (items > 0x7fffffffLL || b->total_bins >= 0xffffffffLL)

@@ -62,7 +62,7 @@ struct PixelArgs {
     // sample order per (radius class, cell of the grain's centre fractions),
     // for narrow grains that take the direct disk test; the lists of each
     // sample table are SampleTable::cl_cell / cl_list.  Class k holds grains
-    // with rz < (k + 1) / cl_inv_dz; list (k, c) is cl_cell[k * cl_q^2 + c]
+    // with rad * zoom < (k + 1) / cl_inv_dz (0: class 0 holds all); list (k, c) is cl_cell[k * cl_q^2 + c]
     // = (start, length) in cl_list.
     int cl_q, cl_classes;
     float cl_inv_dz;

@@ -73,6 +73,7 @@ struct LevelSet {
     SampleTable *store;
     int n, classes;
     int level_n[kMaxLevels];  // samples per level, ascending
+    float r_const;  // > 0: the lists' one class is of this radius
 };
 // Ranks t.n <= 2048 samples into t (laid out by sample_table_layout): its
 // sorted arrays and its y order.
@@ -81,8 +82,9 @@ hipError_t launch_sample_rank(const float2 *offs, float zoom, const SampleTable 
 hipError_t launch_sample_levels(const LevelSet &set, hipStream_t s);
 
 // Candidate lists of the HBM splat (PixelArgs::cl_*) for every level of a set,
-// in one launch: q * q cells per class, class k of radius (k + 1) / (2 q).  e
-// is an integer >= (2 t.eps + 2^-11) q; a table's cl_list needs
+// in one launch: q * q cells per class, class k of radius (k + 1) / (2 q), or
+// the one class of radius r_const.  e is an integer >= (2 t.eps + 2^-11) q,
+// plus 2 r_const q - 1 in the latter case; a table's cl_list needs
 // splat_lists_entries(q, classes, e, t.n) entries, cl_cell classes * q * q
 // (start, length) pairs, cl_yidx classes * q * q * kRowBuckets counts, its
 // fill classes counters.  A class beyond its room sets kStatusCapacity in
@@ -194,8 +196,9 @@ struct BatchGen {
     unsigned long long *mask;
     float4 *grains;
     // sample tables (each plane's st): the candidate lists' plan per plane,
-    // (q, classes, e, 0) with classes == 0 for a plane without lists, their
-    // counters, and the first splat-lists workgroup of each plane
+    // (q, classes, e, the bits of r_const) with classes == 0 for a plane
+    // without lists, their counters, and the first splat-lists workgroup of
+    // each plane
     const int4 *list_plan;
     uint32_t *const *list_fill;
     const long long *list_off;

@@ -805,12 +805,12 @@ void sample_table_layout(void *buf, int n, int qbuckets, SampleTable *t)
 // splat from HBM grains
 // ---------------------------------------------------------------------------
 // Candidate lists for the direct test.  A sample's point can pass a narrow
-// grain's disk test only if (frac(X), frac(Y)) lies within rz + eps of
+// grain's disk test only if (frac(X), frac(Y)) lies within rad * zoom + eps of
 // c = (frac(-bx), frac(-by)), bx = cx * zoom - 0.5, on the unit torus (c is
 // exact in f32, and so is its cell floor(c * q) for q a power of two): the
 // target bx + X and the point's distances take a few roundings of at most
-// C * 2^-24 each, which eps covers.  The list of class k (rz < R =
-// (k + 1) dz) and cell (qa, qb) holds every sample whose fractions are within
+// C * 2^-24 each, which eps covers.  The list of class k (rad * zoom < R =
+// (k + 1) dz; a constant radius is its own one class) and cell (qa, qb) holds every sample whose fractions are within
 // R + eps + 2^-12 of the cell's square (2^-12 for the rounding of this test
 // and of the class): the square with its corners rounded.  (With square
 // corners, the disk test's bounding box, a list at R = 0.2 is 23% longer: the
@@ -942,7 +942,7 @@ __global__ __launch_bounds__(256) void splat_lists_kernel(LevelSet set, int q, i
     const int per = set.classes * ((q * q + 63) / 64);
     const int l = blockIdx.x / per;
     const SampleTable &t = set.t[l];
-    splat_lists_body(t, q, e, t.eps, 0.0f, set.fill[l], const_cast<uint2 *>(t.cl_cell), const_cast<uint16_t *>(t.cl_yidx),
+    splat_lists_body(t, q, e, t.eps, set.r_const, set.fill[l], const_cast<uint2 *>(t.cl_cell), const_cast<uint16_t *>(t.cl_yidx),
                      const_cast<uint16_t *>(t.cl_list), status, blockIdx.x - l * per, sh);
 }
 
@@ -1000,7 +1000,7 @@ __global__ __launch_bounds__(256) void batch_splat_lists_kernel(BatchGen bg)
     const int p = find_run(bg.list_off, bg.n, blk);
     const BatchPlane &bp = cplane(bg.planes, p);
     const int4 lp = cload(bg.list_plan + p);
-    splat_lists_body(bp.st, lp.x, lp.z, bp.st.eps, 0.0f, cload(bg.list_fill + p), const_cast<uint2 *>(bp.st.cl_cell),
+    splat_lists_body(bp.st, lp.x, lp.z, bp.st.eps, __int_as_float(lp.w), cload(bg.list_fill + p), const_cast<uint2 *>(bp.st.cl_cell),
                      const_cast<uint16_t *>(bp.st.cl_yidx), const_cast<uint16_t *>(bp.st.cl_list), bp.a.status,
                      (int)(blk - cload(bg.list_off + p)), sh);
 }
@@ -1392,7 +1392,7 @@ __device__ __forceinline__ void splat_tile(const PixelArgs &a, const PixGeom &ge
         const unsigned long long unsafe_m = LISTS ? __ballot(in_class && rad > safe_r) : 0ull;
         const bool check = win_fast && (unsafe_m & (unsafe_m - 1ull)) != 0ull;  // two or more
         if (in_class && (check || rad <= safe_r)) {
-            const int k = (int)(rz * a.cl_inv_dz);
+            const int k = (int)(rad * z * a.cl_inv_dz);
             if (k < a.cl_classes) {
                 const float ncx = -bx, ncy = -by;
                 const float fx = ncx - floorf(ncx), fy = ncy - floorf(ncy);

@@ -126,10 +126,11 @@ def test_lists_hold_every_passing_sample(z, out_side, n):
         rz = f32(f32(rad * zf) + slack)
         if not rz + rz < 1:
             continue
-        k = int(f32(rz * f32(2 * q)))
+        # a constant radius is its own class
+        R = f32(rad * zf) if i % 2 else f32(f32(int(f32(f32(rad * zf) * f32(2 * q))) + 1) / f32(2 * q))
         f = (-b - np.floor(-b)).astype(f32)
         qa, qb = (min(int(f32(v * f32(q))), q - 1) for v in f)
-        sel = members(fx, fy, qa, qb, q, f32(f32(k + 1) / f32(2 * q)), eps)
+        sel = members(fx, fy, qa, qb, q, R, eps)
         near = np.rint(((o + g).astype(f32).astype(np.float64) * z - 0.5)).astype(f32)
         dx = ((((near + f32(0.5)) * iz).astype(f32) - o).astype(f32) - g).astype(f32)
         inside = ((dx * dx).astype(f32).sum(axis=1)).astype(f32) <= f32(rad * rad)
