@@ -198,24 +198,98 @@ __global__ __launch_bounds__(kBlock) void grainwise_tiles(GrainArgs a)
 // count draws are stored so that the splat kernel resumes each pixel's stream
 // where the reference does (keeps the large Poisson sampler out of the splat
 // kernel's registers).  Pixels with lambda <= 0 get q = 0.
+//
+// Bound by instruction issue (f64 logarithms, divisions and tangents).  A wave
+// takes 64 pixels at a time through the setup and one attempt of the rejection
+// sampler (lambda >= 12); the streams that were rejected, about half, wait in
+// the wave's LDS queue and are tried again 64 at a time as soon as there are
+// as many, the last ones at the wave's end.  (The wave's LDS accesses run in
+// order, so no barrier is needed.)  A 4096x4096 plane with about 90 grains a
+// pixel takes 1.05 ms; one pixel a lane until it was accepted took 1.83, with
+// 24 of 64 lanes busy.
+constexpr int kStateQueue = 128;  // entries: below 64 before a push of up to 64
+
+struct StateQueue {
+    uint64_t s[4][kStateQueue];
+    double c[3][kStateQueue];  // PoissonReject's log_lambda, sqrt_2lambda, magic
+    uint64_t pixel[kStateQueue];
+    float lambda[kStateQueue];
+};
+
+__device__ __forceinline__ void put_pixel_state(const GrainArgs &a, long long p, uint32_t q, const Xoshiro &rng)
+{
+    a.pix_q[p] = q;
+    a.pix_s01[p] = make_ulonglong2(rng.s0, rng.s1);
+    a.pix_s23[p] = make_ulonglong2(rng.s2, rng.s3);
+}
+
 __global__ __launch_bounds__(kBlock) void pixel_state_kernel(GrainArgs a)
 {
+    __shared__ StateQueue s_queue[kBlock / 64];
+    const int lane = threadIdx.x & 63;
+    StateQueue &sq = s_queue[threadIdx.x >> 6];
     const long long n = (long long)a.in_w * a.in_h;
-    for (long long p = (long long)blockIdx.x * kBlock + threadIdx.x; p < n; p += (long long)gridDim.x * kBlock) {
-        const int y = (int)(p / a.in_w), x = (int)(p - (long long)y * a.in_w);
-        const float lam = a.lambda[p];
+    const long long stride = (long long)gridDim.x * kBlock;
+    long long base = (long long)blockIdx.x * kBlock + (threadIdx.x & ~63);
+    int queued = 0;  // uniform
+    while (base < n || queued > 0) {
         Xoshiro rng;
         rng.s0 = rng.s1 = rng.s2 = rng.s3 = 0;
-        uint32_t q = 0;
-        // values outside the accepted range are skipped and flagged (once per wave)
-        if (__ballot(lambda_invalid(lam)) != 0ull && (threadIdx.x & 63) == 0) atomicOr(a.status, kStatusLambda);
-        if (lam > 0.0f && lam <= kMaxLambda) {
-            rng.seed(mix3(a.seed, kPixelStream, x, y));
-            q = poisson_u32(rng, (double)lam);
+        long long p;
+        bool on;  // the lane takes an attempt
+        PoissonReject pr(12.0, 0.0, 0.0, 0.0);
+        if (queued < 64 && base < n) {  // 64 new pixels
+            p = base + lane;
+            base += stride;
+            const bool in = p < n;
+            const float lam = in ? a.lambda[p] : 0.0f;
+            // values outside the accepted range are skipped and flagged (once per wave)
+            if (__ballot(lambda_invalid(lam)) != 0ull && lane == 0) atomicOr(a.status, kStatusLambda);
+            const bool drawn = lam > 0.0f && lam <= kMaxLambda;
+            on = drawn && (double)lam >= 12.0;
+            uint32_t q = 0;
+            if (drawn) {
+                const int y = (int)(p / a.in_w), x = (int)(p - (long long)y * a.in_w);
+                rng.seed(mix3(a.seed, kPixelStream, x, y));
+                if (!on) q = poisson_knuth(rng, (double)lam);
+            }
+            if (in && !on) put_pixel_state(a, p, q, rng);
+            if (on) pr = PoissonReject((double)lam);
+        } else {  // the queue's last ones again
+            const int m = min(queued, 64);
+            queued -= m;
+            on = lane < m;
+            const int slot = queued + (on ? lane : 0);
+            rng.s0 = sq.s[0][slot];
+            rng.s1 = sq.s[1][slot];
+            rng.s2 = sq.s[2][slot];
+            rng.s3 = sq.s[3][slot];
+            pr = PoissonReject((double)sq.lambda[slot], sq.c[0][slot], sq.c[1][slot], sq.c[2][slot]);
+            p = (long long)sq.pixel[slot];
+            __builtin_amdgcn_wave_barrier();
         }
-        a.pix_q[p] = q;
-        a.pix_s01[p] = make_ulonglong2(rng.s0, rng.s1);
-        a.pix_s23[p] = make_ulonglong2(rng.s2, rng.s3);
+        bool again = false;
+        if (on) {
+            double r = 0.0;
+            again = !pr.attempt(rng, &r);
+            if (!again) put_pixel_state(a, p, poisson_count(r), rng);
+        }
+        const unsigned long long m = __ballot(again);
+        const int slot = queued + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        if (again) {
+            sq.s[0][slot] = rng.s0;
+            sq.s[1][slot] = rng.s1;
+            sq.s[2][slot] = rng.s2;
+            sq.s[3][slot] = rng.s3;
+            sq.c[0][slot] = pr.log_lambda;
+            sq.c[1][slot] = pr.sqrt_2lambda;
+            sq.c[2][slot] = pr.magic;
+            sq.pixel[slot] = (uint64_t)p;
+            sq.lambda[slot] = (float)pr.lambda;
+        }
+        queued += __popcll(m);
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -264,7 +338,11 @@ hipError_t launch_grain_count(const GrainArgs &a, int dist_kind, hipStream_t s)
 hipError_t launch_pixel_state(const GrainArgs &a, hipStream_t s)
 {
     const long long n = (long long)a.in_w * a.in_h;
-    const long long blocks = std::min<long long>((n + kBlock - 1) / kBlock, 1LL << 20);
+    // A wave's last attempts run nearly empty, so waves take 128 pixels or
+    // more; 1024 workgroups are four a CU, as many as fit by LDS.  (64, 256 and
+    // 512 pixels at least: the same at 4096x4096, 0.3, 0.4 and 1% more for a
+    // 1280x720 RGB frame.)
+    const long long per = 2 * kBlock, blocks = std::max<long long>(1, std::min<long long>((n + per - 1) / per, 1024));
     hipLaunchKernelGGL(pixel_state_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, a);
     return hipGetLastError();
 }

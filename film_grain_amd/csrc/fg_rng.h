@@ -196,52 +196,70 @@ FG_HD double log_gamma(double x)
 }
 
 // Poisson<f64>::sample for lambda >= 12 (Cauchy comparison rejection), as f64.
-FG_HD double poisson_rejection(Xoshiro &rng, double lambda)
-{
-    const double log_lambda = log(lambda);
-    const double sqrt_2lambda = sqrt(2.0 * lambda);
-    const double magic = lambda * log_lambda - log_gamma(1.0 + lambda);
-    double result;
-    for (;;) {
-        double comp;
-        for (;;) {
-            comp = 0.0 + 1.0 * tan(3.14159265358979323846 * standard_f64(rng.next()));
-            result = sqrt_2lambda * comp + lambda;
-            if (result >= 0.0) break;
-        }
+struct PoissonReject {
+    double lambda, log_lambda, sqrt_2lambda, magic;
+    FG_HD explicit PoissonReject(double l)
+        : lambda(l), log_lambda(log(l)), sqrt_2lambda(sqrt(2.0 * l)), magic(l * log_lambda - log_gamma(1.0 + l))
+    {
+    }
+    FG_HD PoissonReject(double l, double ll, double s2l, double m) : lambda(l), log_lambda(ll), sqrt_2lambda(s2l), magic(m)
+    {
+    }
+    // One comparison deviate; true when it is accepted.  (The reference draws
+    // deviates until one is not negative, then accepts or starts again: a
+    // negative one is a rejection that takes no second uniform.)
+    FG_HD bool attempt(Xoshiro &rng, double *out) const
+    {
+        const double comp = 0.0 + 1.0 * tan(3.14159265358979323846 * standard_f64(rng.next()));
+        double result = sqrt_2lambda * comp + lambda;
+        if (!(result >= 0.0)) return false;
         result = floor(result);
+        *out = result;
         // check = 0.9 (1 + comp^2) exp(...), and the draw is accepted when
         // U <= check
-        if (cmp_exp(standard_f64(rng.next()), result * log_lambda - log_gamma(1.0 + result) - magic,
-                    0.9 * (1.0 + comp * comp), false))
-            break;
+        return cmp_exp(standard_f64(rng.next()), result * log_lambda - log_gamma(1.0 + result) - magic,
+                       0.9 * (1.0 + comp * comp), false);
+    }
+};
+
+FG_HD double poisson_rejection(Xoshiro &rng, double lambda)
+{
+    const PoissonReject pr(lambda);
+    double result;
+    while (!pr.attempt(rng, &result)) {
     }
     return result;
 }
 
-// Poisson<f64>::new(lambda).sample(rng) as u32.  Only exp(-lambda) is needed on
-// the Knuth branch; the other precomputed terms of Poisson::new feed the
-// rejection branch only.
-FG_HD uint32_t poisson_u32(Xoshiro &rng, double lambda)
+FG_HD uint32_t poisson_count(double r)
 {
-    if (lambda < 12.0) {
-#if defined(__HIP_DEVICE_COMPILE__)
-        const double e = exp_neg_glibc((float)lambda);  // lambda is an f32 value
-#else
-        const double e = exp(-lambda);
-#endif
-        double p = 1.0;
-        uint32_t n = 0;
-        while (p > e) {
-            p = p * standard_f64(rng.next());
-            ++n;
-        }
-        return n == 0 ? 0u : n - 1u;
-    }
-    const double r = poisson_rejection(rng, lambda);
     if (!(r > 0.0)) return 0u;
     if (r >= 4294967295.0) return 0xFFFFFFFFu;
     return (uint32_t)r;
+}
+
+// Poisson<f64>::new(lambda).sample(rng) as u32.  Only exp(-lambda) is needed on
+// the Knuth branch (lambda < 12); the other precomputed terms of Poisson::new
+// feed the rejection branch only.
+FG_HD uint32_t poisson_knuth(Xoshiro &rng, double lambda)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double e = exp_neg_glibc((float)lambda);  // lambda is an f32 value
+#else
+    const double e = exp(-lambda);
+#endif
+    double p = 1.0;
+    uint32_t n = 0;
+    while (p > e) {
+        p = p * standard_f64(rng.next());
+        ++n;
+    }
+    return n == 0 ? 0u : n - 1u;
+}
+
+FG_HD uint32_t poisson_u32(Xoshiro &rng, double lambda)
+{
+    return lambda < 12.0 ? poisson_knuth(rng, lambda) : poisson_count(poisson_rejection(rng, lambda));
 }
 
 // StandardNormal via the 256-layer ziggurat of rand_distr 0.4.3 (symmetric

@@ -115,3 +115,19 @@ def test_thin_long_plane(hip_ctx, oracle, sd):
     want = oracle.render_grainwise(case.plane, case.lam, case.offsets)
     got = hip_ctx.render_host("grain", case.desc, case.lam, case.offsets)
     assert int(np.sum(got != want)) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,h,r,sd", [(1, 1, 0.1, 0.0), (63, 1, 0.14, 0.0), (65, 3, 0.05, 0.02), (513, 2, 0.13, 0.0),
+                                      (129, 64, 0.3, 0.0), (811, 655, 0.13, 0.0), (700, 750, 0.06, 0.0)])
+def test_counts_of_every_pixel(hip_ctx, oracle, w, h, r, sd):
+    """Pixels below and above a mean of 12 grains (Knuth's product, the
+    rejection sampler with its queue), whole and partial waves, one round of
+    the grid's pixels and more; streams resume where the count left them."""
+    from film_grain_amd import synth
+    from tests import fgcases
+    plane = synth.sinusoid_field(w, h, w + h, n_waves=3)
+    c = fgcases.build_case(oracle, "count", plane, r, sd, "lognorm" if sd else "const", zoom=1.0, n_samples=2, seed=w)
+    want = oracle.render_grainwise(c.plane, c.lam, c.offsets)
+    got = hip_ctx.render_host("grain", c.desc, c.lam, c.offsets)
+    assert np.array_equal(got, want)
