@@ -310,45 +310,60 @@ hipError_t launch_batch_order(const BatchPlane *planes, int n_planes, const uint
     return hipGetLastError();
 }
 
-// Weights and heaviest-first order of one plane's tiles in one workgroup, for
-// planes of at most kOrderTiles tiles: a counting sort by quarter octaves of
-// the weight.  (The weights' launch and a radix sort's one to four took 13 to
-// 25 us of a small plane; this takes 5 to 8.)
-__global__ __launch_bounds__(1024) void tile_order_kernel(PixelArgs a, PixGeom geo, const uint32_t *bin_start, int *order)
+// Heaviest-first order of one plane's tiles in one workgroup: a counting sort
+// by sixteenth octaves of the weight.  Up to kOrderFused tiles compute their
+// weights here as well (w null): 5 to 8 us.  More have too many scattered
+// reads for one workgroup (4080 tiles: 63 us) and take a launch of their own
+// (10 us and 6 here).  A radix sort takes two to five launches, 13 to 28 us;
+// beyond kOrderTiles it is the shorter.
+__global__ __launch_bounds__(1024) void tile_order_kernel(PixelArgs a, PixGeom geo, const uint32_t *bin_start,
+                                                          const uint32_t *w, int n, int *order)
 {
-    __shared__ uint32_t s_count[128], s_pos[128];
-    constexpr int kPer = kOrderTiles / 1024;
-    if (threadIdx.x < 128) s_count[threadIdx.x] = 0;
+    constexpr int kPer = kOrderTiles / 1024, kBuckets = 512, kBucketsLane = kBuckets / 64;
+    __shared__ uint32_t s_count[kBuckets], s_pos[kBuckets];
+    if (threadIdx.x < kBuckets) s_count[threadIdx.x] = 0;
     __syncthreads();
-    uint8_t bucket[kPer];
+    uint32_t bucket[kPer];
+#pragma unroll
     for (int j = 0; j < kPer; ++j) {
         const int tile = j * 1024 + (int)threadIdx.x;
         bucket[j] = 0;
-        if (tile >= a.n_tiles) continue;
-        const uint32_t w = tile_weight(a, geo, bin_start, tile);
-        // 4 log2(w + 1) by the float's exponent and two mantissa bits
-        bucket[j] = (uint8_t)min(127u, (__float_as_uint((float)w + 1.0f) >> 21) - (127u << 2));
+        if (tile >= n) continue;
+        const uint32_t v = w ? w[tile] : tile_weight(a, geo, bin_start, tile);
+        // 16 log2(v + 1) by the float's exponent and four mantissa bits
+        bucket[j] = min(kBuckets - 1u, (__float_as_uint((float)v + 1.0f) >> 19) - (127u << 4));
         atomicAdd(&s_count[bucket[j]], 1u);
     }
     __syncthreads();
     if (threadIdx.x < 64) {  // first position of each bucket, heaviest first
-        const int b = 127 - 2 * (int)threadIdx.x;
-        const uint32_t c0 = s_count[b], c1 = s_count[b - 1];
-        const uint32_t before = wave_inclusive_sum(c0 + c1) - (c0 + c1);
-        s_pos[b] = before;
-        s_pos[b - 1] = before + c0;
+        const int b = kBuckets - 1 - kBucketsLane * (int)threadIdx.x;
+        uint32_t sum = 0;
+        for (int j = 0; j < kBucketsLane; ++j) sum += s_count[b - j];
+        uint32_t pos = wave_inclusive_sum(sum) - sum;
+        for (int j = 0; j < kBucketsLane; ++j) {
+            s_pos[b - j] = pos;
+            pos += s_count[b - j];
+        }
     }
     __syncthreads();
+#pragma unroll
     for (int j = 0; j < kPer; ++j) {
         const int tile = j * 1024 + (int)threadIdx.x;
-        if (tile < a.n_tiles) order[atomicAdd(&s_pos[bucket[j]], 1u)] = tile;
+        if (tile < n) order[atomicAdd(&s_pos[bucket[j]], 1u)] = tile;
     }
 }
 
 hipError_t launch_tile_order(const PixelArgs &a, const PixGeom &g, const uint32_t *bin_start, int *order, hipStream_t s)
 {
-    if (a.n_tiles > kOrderTiles) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, s, a, g, bin_start, order);
+    if (a.n_tiles > kOrderFused) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, s, a, g, bin_start, nullptr, a.n_tiles, order);
+    return hipGetLastError();
+}
+
+hipError_t launch_weight_order(const uint32_t *w, int n, int *order, hipStream_t s)
+{
+    if (n > kOrderTiles) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, s, PixelArgs{}, PixGeom{}, nullptr, w, n, order);
     return hipGetLastError();
 }
 

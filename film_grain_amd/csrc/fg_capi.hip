@@ -609,41 +609,6 @@ void splat_bounds(const fg::PixelArgs &a, const fg::PixGeom &g, const float4 &r,
     *safe_r = sr > 0.0f ? sr : -1.0f;
 }
 
-// Heaviest-first launch order of n tiles: the caller's weights kernel fills
-// TileOrder::w / ids, then sort() leaves the sorted ids in TileOrder::order.
-// Workgroups start in launch order, so the heavy tiles start first and the
-// light ones fill the tail.
-struct TileOrder {
-    uint32_t *w = nullptr, *w_sorted = nullptr;
-    int *ids = nullptr, *order = nullptr;
-    void place(void *p, int n)  // 16 n bytes
-    {
-        unsigned char *b = static_cast<unsigned char *>(p);
-        w = reinterpret_cast<uint32_t *>(b);
-        w_sorted = reinterpret_cast<uint32_t *>(b + (size_t)n * 4);
-        ids = reinterpret_cast<int *>(b + (size_t)n * 8);
-        order = reinterpret_cast<int *>(b + (size_t)n * 12);
-    }
-};
-
-int tile_order_prepare(fg_ctx *ctx, int n, TileOrder *t, hipStream_t s, const char *what)
-{
-    int rc = ensure_bytes(ctx, ctx->tiles, (size_t)n * 16, what);
-    if (rc != FG_OK) return rc;
-    size_t temp = 0;
-    hipError_t e = fg::sort_tiles(nullptr, &temp, nullptr, nullptr, nullptr, nullptr, n, s);
-    if (e != hipSuccess) return hip_error(ctx, e, what);
-    if ((rc = ensure_bytes(ctx, ctx->tile_temp, temp, what)) != FG_OK) return rc;
-    t->place(ctx->tiles.p, n);
-    return FG_OK;
-}
-
-hipError_t tile_order_sort(fg_ctx *ctx, int n, const TileOrder &t, hipStream_t s)
-{
-    size_t temp = ctx->tile_temp.cap;
-    return fg::sort_tiles(ctx->tile_temp.p, &temp, t.w, t.w_sorted, t.ids, t.order, n, s);
-}
-
 // Candidate lists of the splat's direct test for one sample table: classes
 // of 1/64 output pixel up to the narrow limit rz < 0.5 and the plane's
 // largest rz, 32 x 32 cells, each with its row-bucket counts.
@@ -791,6 +756,47 @@ int scratch_get(fg_ctx *ctx, ScratchSource &src, DevBuf &b, size_t bytes, void *
     return FG_OK;
 }
 
+// Heaviest-first launch order of n tiles: the caller's weights kernel fills
+// TileOrder::w / ids, then sort() leaves the sorted ids in TileOrder::order.
+// Workgroups start in launch order, so the heavy tiles start first and the
+// light ones fill the tail.
+struct TileOrder {
+    uint32_t *w = nullptr, *w_sorted = nullptr;
+    int *ids = nullptr, *order = nullptr;
+    void place(void *p, int n)  // 16 n bytes
+    {
+        unsigned char *b = static_cast<unsigned char *>(p);
+        w = reinterpret_cast<uint32_t *>(b);
+        w_sorted = reinterpret_cast<uint32_t *>(b + (size_t)n * 4);
+        ids = reinterpret_cast<int *>(b + (size_t)n * 8);
+        order = reinterpret_cast<int *>(b + (size_t)n * 12);
+    }
+};
+
+// Places the order in the tiles buffer, and the radix sort's scratch where the
+// plane has too many tiles for one workgroup (kOrderTiles).
+int tile_order_prepare(fg_ctx *ctx, ScratchSource &src, int n, TileOrder *t, size_t *temp, void **temp_p,
+                       hipStream_t s, const char *what)
+{
+    void *p;
+    int rc = scratch_get(ctx, src, ctx->tiles, (size_t)n * 16, &p, what);
+    if (rc != FG_OK) return rc;
+    t->place(p, n);
+    *temp = 0;
+    *temp_p = nullptr;
+    if (n <= fg::kOrderTiles) return FG_OK;
+    const hipError_t e = fg::sort_tiles(nullptr, temp, nullptr, nullptr, nullptr, nullptr, n, s);
+    if (e != hipSuccess) return hip_error(ctx, e, what);
+    return scratch_get(ctx, src, ctx->tile_temp, *temp, temp_p, what);
+}
+
+// Orders by the weights in t.w (and t.ids).
+hipError_t tile_order_sort(int n, const TileOrder &t, size_t temp, void *temp_p, hipStream_t s)
+{
+    if (n <= fg::kOrderTiles) return fg::launch_weight_order(t.w, n, t.order, s);
+    return fg::sort_tiles(temp_p, &temp, t.w, t.w_sorted, t.ids, t.order, n, s);
+}
+
 // The per-plane generation of the HBM path: Poisson thresholds, per-bin
 // counts and nonempty masks and their scan (hbm_count), and every cell's
 // grains written contiguously per bin (hbm_draw, after a wait for the total).
@@ -921,20 +927,14 @@ int run_pixel_hbm(fg_ctx *ctx, fg::PixelArgs &a, const fg::PixGeom &g, const flo
     const float4 *grains = gen.grains;
     // heaviest-first tile order
     TileOrder order;
-    void *tiles_p;
-    if ((rc = scratch_get(ctx, src, ctx->tiles, (size_t)a.n_tiles * 16, &tiles_p, what)) != FG_OK) return rc;
-    order.place(tiles_p, a.n_tiles);
-    if (a.n_tiles <= fg::kOrderTiles) {
+    size_t sort_temp;
+    void *sort_p;
+    if ((rc = tile_order_prepare(ctx, src, a.n_tiles, &order, &sort_temp, &sort_p, s, what)) != FG_OK) return rc;
+    if (a.n_tiles <= fg::kOrderFused) {
         e = fg::launch_tile_order(a, g, start, order.order, s);
     } else {
-        size_t sort_temp = 0;
-        void *tile_temp_p;
-        e = fg::sort_tiles(nullptr, &sort_temp, nullptr, nullptr, nullptr, nullptr, a.n_tiles, s);
-        if (e != hipSuccess) return hip_error(ctx, e, what);
-        if ((rc = scratch_get(ctx, src, ctx->tile_temp, sort_temp, &tile_temp_p, what)) != FG_OK) return rc;
         e = fg::launch_pixel_tile_weights(a, g, start, order.w, order.ids, s);
-        if (e == hipSuccess)
-            e = fg::sort_tiles(tile_temp_p, &sort_temp, order.w, order.w_sorted, order.ids, order.order, a.n_tiles, s);
+        if (e == hipSuccess) e = tile_order_sort(a.n_tiles, order, sort_temp, sort_p, s);
     }
     a.tile_list = order.order;
     mark(ctx, 1, s);
@@ -1320,7 +1320,10 @@ int do_grainwise(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lambda, con
         a.pix_s23 = reinterpret_cast<ulonglong2 *>(ps + npx * 16);
         a.pix_q = reinterpret_cast<uint32_t *>(ps + npx * 32);
         TileOrder order;
-        if ((rc = tile_order_prepare(ctx, a.n_tiles, &order, s, what)) != FG_OK) return rc;
+        ScratchSource src;
+        size_t sort_temp;
+        void *sort_p;
+        if ((rc = tile_order_prepare(ctx, src, a.n_tiles, &order, &sort_temp, &sort_p, s, what)) != FG_OK) return rc;
         fg::LevelSet set{};
         fg::sample_table_layout(ctx->samples.p, a.n_samples, q, &set.full);
         const fg::SampleTable &st = set.full;
@@ -1363,7 +1366,7 @@ int do_grainwise(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lambda, con
         }
         if (e == hipSuccess) e = fg::launch_pixel_state(a, s);
         if (e == hipSuccess) e = fg::launch_grain_tile_weights(a, st, order.w, order.ids, s);
-        if (e == hipSuccess) e = tile_order_sort(ctx, a.n_tiles, order, s);
+        if (e == hipSuccess) e = tile_order_sort(a.n_tiles, order, sort_temp, sort_p, s);
         a.tile_list = order.order;
         mark(ctx, 1, s);
         mark(ctx, 2, s);

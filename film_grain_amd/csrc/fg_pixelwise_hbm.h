@@ -154,8 +154,10 @@ hipError_t launch_pixel_tile_weights(const PixelArgs &a, const PixGeom &g, const
                                      int *ids, hipStream_t s);
 hipError_t sort_tiles(void *temp, size_t *temp_bytes, const uint32_t *w_in, uint32_t *w_out, const int *ids_in,
                       int *ids_out, int n, hipStream_t s);
-// Weights and order of at most kOrderTiles tiles in one launch.
-constexpr int kOrderTiles = 4096;
+// Weights and order of at most kOrderFused tiles in one launch; order of at
+// most kOrderTiles tiles by given weights.
+constexpr int kOrderFused = 2048, kOrderTiles = 8192;
+hipError_t launch_weight_order(const uint32_t *w, int n, int *order, hipStream_t s);
 hipError_t launch_tile_order(const PixelArgs &a, const PixGeom &g, const uint32_t *bin_start, int *order, hipStream_t s);
 // Grain-wise: w[t] = grains of the input pixels whose grains can reach tile t.
 hipError_t launch_grain_tile_weights(const GrainArgs &a, const SampleTable &st, uint32_t *w, int *ids,

@@ -126,7 +126,8 @@ def test_call_after_a_refused_one(oracle):
     (200, 200, 0.1, None),     # either side of 16384 bins: one workgroup, three launches
     (212, 212, 0.1, None),
     (64, 48, 0.1, 0.0),        # no grain at all
-    (2200, 2000, 1.0, 0.02),   # more than 4096 tiles: ordered by the radix sort
+    (2200, 2000, 1.0, 0.02),   # more than 2048 tiles: weights in their own launch
+    (3000, 2900, 1.0, 0.02),   # more than 8192: ordered by the radix sort
 ])
 def test_bin_starts_and_tile_order(oracle, w, h, radius, grey):
     plane = (np.full((h, w), grey, dtype=np.float32) if grey is not None
