@@ -14,7 +14,10 @@
 //   layer 1: Z1 = X W1 + b1      4 x v_mfma_f32_16x16x16_bf16 (one per 16 outputs)
 //   layer 2: Z2 = H1 W2 + b2     8 x v_mfma_f32_16x16x32_bf16, H1 = relu(Z1) in BF16
 //   layer 3: y = H2 . w3 + b3    FP32 dot products (a 64-vector), H2 = relu(Z2)
-// The biases are the accumulators' initial values.
+// The forward pass adds a bias after its layer's sum, and layer 3's columns one
+// after the other: its predictions decide integer budgets, so their bits are
+// part of its result.  In the gradient the biases are the accumulators' initial
+// values.
 // Backward of the loss per row (fused, per tile), either the squared error to
 // a target t, L = (y - t)^2, g = dL/dy = 2 (y - t), or the Gaussian negative
 // log-likelihood of a residual t under the predicted log std y,
@@ -134,12 +137,13 @@ __device__ __forceinline__ void load_weights(const MlpOperands &s, MlpWeights &w
     }
 }
 
-// Bounded by instruction issue: 12 matrix instructions and about 100 VALU per
-// 16 rows, which do not overlap fully.  2.07M rows (75 MB): 45 us with the
-// conversions in hardware, fused multiply-adds and the biases as initial
-// accumulators; 88 us with conversions in software.  More rows in flight (two
-// to eight tiles ahead, four at once) and two or four waves per SIMD instead
-// of three: no difference.
+// Bounded by instruction issue: 12 matrix instructions and about 130 VALU per
+// 16 rows, which do not overlap fully.  2.07M rows (75 MB): 44 us with the
+// conversions in hardware, 88 us with conversions in software.  (The biases as
+// initial accumulators and layer 3 in four fused chains are 4 us less, and move
+// one budget in about 1e5 by a sample.)  More rows in flight (two to eight tiles
+// ahead, four at once) and two or four waves per SIMD instead of three: no
+// difference.
 constexpr int kTiles = 2;  // 16-row tiles a wave works on at once
 __global__ __launch_bounds__(256, 3) void mlp_forward_kernel(const float *P, const uint16_t *X, long long n, float *out,
                                                           bool aligned)
@@ -162,6 +166,7 @@ __global__ __launch_bounds__(256, 3) void mlp_forward_kernel(const float *P, con
     const long long tiles = (n + 15) / 16;
     const long long stride = (long long)gridDim.x * 4 * kTiles;
     const v4bf zero = {};
+    const v4f zero4 = {};
     long long tt = ((long long)blockIdx.x * 4 + wid) * kTiles;
     v4bf x[kTiles], xn[kTiles];  // this step's rows, and the next one's, in flight meanwhile
     auto fetch = [&](v4bf *v, long long at) {
@@ -177,20 +182,19 @@ __global__ __launch_bounds__(256, 3) void mlp_forward_kernel(const float *P, con
         v8bf h0[kTiles], h1[kTiles];
         for (int u = 0; u < kTiles; ++u) {
             v4bf h[4];
-            for (int cb = 0; cb < 4; ++cb) h[cb] = relu_bf16(mfma16(w.w1[cb], x[u], b1[cb]));
+            for (int cb = 0; cb < 4; ++cb) h[cb] = relu_bf16(mfma16(w.w1[cb], x[u], zero4) + b1[cb]);
             h0[u] = join(h[0], h[1]);
             h1[u] = join(h[2], h[3]);
         }
         // layer 2 (transposed) and layer 3
         float y[kTiles];
         for (int u = 0; u < kTiles; ++u) {
-            float acc[4];
+            float acc = 0.0f;
             for (int cb = 0; cb < 4; ++cb) {
-                const v4f c = mfma32(w.w2[cb][1], h1[u], mfma32(w.w2[cb][0], h0[u], b2[cb]));
-                acc[cb] = fmaxf(c[0], 0.0f) * w3[cb][0];
-                for (int i = 1; i < 4; ++i) acc[cb] = __builtin_fmaf(fmaxf(c[i], 0.0f), w3[cb][i], acc[cb]);
+                const v4f c = mfma32(w.w2[cb][1], h1[u], mfma32(w.w2[cb][0], h0[u], zero4)) + b2[cb];
+                for (int i = 0; i < 4; ++i) acc += fmaxf(c[i], 0.0f) * w3[cb][i];
             }
-            y[u] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+            y[u] = acc;
         }
         for (int u = 0; u < kTiles; ++u) {
             y[u] += __shfl_xor(y[u], 16, 64);

@@ -6,7 +6,7 @@ on the oracle), so this is also the reference's own N = b render."""
 import numpy as np
 import pytest
 
-from film_grain_amd import synth
+from film_grain_amd import budget, synth
 from tests import fgcases
 
 pytestmark = pytest.mark.gpu
@@ -122,3 +122,24 @@ def test_budget_kernel(hip_ctx):
     want = np.clip(np.ceil(1000.0 * np.sqrt(Xb[:, 4].astype(np.float64))), 1, 2048).astype(np.int64)
     assert np.all(np.abs(got - want) <= 1)
     assert np.mean(got == want) > 0.999
+
+
+def test_learned_frame_equals_fixed_renders_at_its_budgets(hip_ctx):
+    """The frame budget.render_adaptive_frame returns, pixel by pixel: the
+    fixed render at the budget it returns for that pixel."""
+    import torch
+    model = budget.ErrorModel.load()
+    planes = [budget.upload(s) for s in budget.image_planes(50_003, 61, 45)]
+    bufs = budget.frame_buffers(planes)
+    outs, _ = budget.render_adaptive_frame(hip_ctx, model, planes, bufs, (12.0 / 255.0) ** 2, n_min=16, n_max=256)
+    torch.cuda.synchronize()
+    for dp, out, b in zip(planes, outs, bufs.budget):
+        b = (b.to(torch.int32) & 0xFFFF).view(dp.out_h, dp.out_w)
+        ns = torch.unique(b).tolist()
+        assert 16 <= ns[0] and ns[-1] <= 256 and len(ns) > 20
+        want = torch.empty_like(out)
+        fixed = torch.empty_like(out)
+        for n in ns:
+            hip_ctx.render_device("pixel", _desc_with_n(dp.desc, n), dp.lam, dp.offs[:n], fixed)
+            want = torch.where(b == n, fixed, want)
+        assert torch.equal(out, want)

@@ -74,3 +74,38 @@ def test_feature_rows_at_any_alignment(hip_ctx, shift):
     hip_ctx.mlp_features(u, 55, 34, 1.5, 0.1, 0.05, 0.8, 1, out=buf[shift:shift + 55 * 34 * 16])
     assert torch.equal(buf[shift:shift + 55 * 34 * 16].view(-1, 16), want)
     assert torch.all(buf[:shift] == 123) and torch.all(buf[shift + 55 * 34 * 16:] == 123)
+
+
+@pytest.mark.parametrize("n", [1, 31, 513])
+def test_forward_adds_in_a_fixed_order(hip_ctx, n):
+    """The sample budgets are a ceiling of the predictions, so the order of the
+    forward pass's additions is part of its result: the bias after the layer's
+    sum, layer 3 one column after the other, products and sums rounded apart.
+    Integer operands make every sum before the biases exact whatever its order
+    (|z2| <= 64 * 256 * 3 < 2^24), so the prediction is known to the bit."""
+    import torch
+    rng = np.random.default_rng(n)
+    P = np.zeros(mlp_ref.N_PARAMS, np.float32)
+    P[:12 * 64] = rng.integers(-3, 4, 12 * 64)
+    P[mlp_ref.P_B1:mlp_ref.P_W2] = rng.integers(-20, 21, 64)
+    P[mlp_ref.P_W2:mlp_ref.P_B2] = rng.integers(-3, 4, 64 * 64)
+    P[mlp_ref.P_B2:mlp_ref.P_W3] = rng.normal(0, 30, 64)
+    P[mlp_ref.P_W3:mlp_ref.P_B3] = rng.normal(0, 0.3, 64)
+    P[mlp_ref.P_B3] = 0.37
+    X = np.zeros((n, 16), np.float32)
+    X[:, :12] = rng.integers(-4, 5, (n, 12))
+    W1, b1, W2, b2, w3, b3 = mlp_ref.unpack(P)
+    h1 = np.maximum(X @ W1 + b1, 0)
+    assert h1.max() <= 256  # exact in BF16
+    h2 = np.maximum((h1 @ W2) + b2[None, :], np.float32(0))
+    assert h2.dtype == np.float32
+    # lane g of a row holds columns 16 cb + 4 g + i
+    prod = (h2 * mlp_ref.bf16(w3)[None, :]).reshape(n, 4, 4, 4)  # row, cb, g, i
+    acc = np.zeros((n, 4), np.float32)
+    for cb in range(4):
+        for i in range(4):
+            acc = acc + prod[:, cb, :, i]
+    want = ((acc[:, 0] + acc[:, 1]) + (acc[:, 2] + acc[:, 3])) + b3
+    bits = (X.view(np.uint32) >> 16).astype(np.uint16).view(np.int16)
+    got = hip_ctx.mlp_forward(torch.from_numpy(P).to("cuda:0"), torch.from_numpy(bits).to("cuda:0")).cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), want.astype(np.float32).view(np.uint32))
