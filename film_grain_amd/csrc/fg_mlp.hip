@@ -79,6 +79,18 @@ __device__ __forceinline__ v4bf load_x(const uint16_t *X, long long row, int g, 
     return x;
 }
 
+// Feature r of rows row0 + 4g..+3 (0 past n).
+__device__ __forceinline__ v4bf load_x_column(const uint16_t *X, long long row0, long long n, int r, int g)
+{
+    v4bf x = {};
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+        const long long row = row0 + 4 * g + i;
+        if (row < n) x[i] = __builtin_bit_cast(__bf16, X[row * 16 + r]);
+    }
+    return x;
+}
+
 // Forward pass for inference, without LDS: the layers are computed
 // transposed, Z1^T = W1^T X^T (16x16x16: A = a 16-output block of W1^T,
 // B = X^T) and Z2^T = W2^T H1^T (16x16x32), so that a lane's accumulator
@@ -217,7 +229,9 @@ __global__ __launch_bounds__(256, 3) void mlp_forward_kernel(const float *P, con
 // take as operands, the transposed form what the next product along the
 // layers takes, so nothing crosses lanes but y and its gradient, and LDS
 // holds only W2's backward operands and the T-layout vectors.  X in the plain
-// layout is X times the identity.
+// layout is X times the identity; a NaN or an infinity makes its whole row NaN
+// there (it meets the identity's zeros), and such a tile is read from memory
+// instead (every tile read so: 51 us for 46 at 400003 rows, 185 for 162 at 2M).
 // Bounded by instruction issue at many rows (2M rows: 0.17 ms, 650 us before);
 // at few by the set-up and the atomics on grad, kMlpParams a workgroup: one
 // workgroup per 256 rows up to one per CU (per 1024 rows: 34 us instead of 27
@@ -283,6 +297,10 @@ __global__ __launch_bounds__(kGradBlock, 2) void mlp_grad_kernel(const float *P,
             xnext = load_x(X, next, g, aligned);
             tnext = target[next];
         }
+        const v4f xf = mfma16(x, ident, zero4);
+        v4bf xn = __builtin_convertvector(xf, v4bf);
+        const float xs = (xf[0] + xf[1]) + (xf[2] + xf[3]);
+        if (__builtin_expect(__any(xs != xs), 0)) xn = load_x_column(X, tt * 16, n, r, g);
         // layer 1 transposed
         v4bf h[4];
         for (int cb = 0; cb < 4; ++cb) h[cb] = relu_bf16(mfma16(w.w1[cb], x, s_b1[cb * 4 + g]));
@@ -343,7 +361,6 @@ __global__ __launch_bounds__(kGradBlock, 2) void mlp_grad_kernel(const float *P,
             zn[cb] = __builtin_convertvector(d, v4bf);
         }
         // layer 1 and dZ1 plain, and the products over the rows
-        const v4bf xn = __builtin_convertvector(mfma16(x, ident, zero4), v4bf);
         for (int cb = 0; cb < 4; ++cb) {
             const v4f a1 = mfma16(x, w.w1[cb], (v4f){b1n[cb], b1n[cb], b1n[cb], b1n[cb]});
             const v4bf hn = relu_bf16(a1);

@@ -65,6 +65,40 @@ def test_nan_features_act_as_before_the_first_relu(hip_ctx):
     assert abs(y[20] - want) <= 1e-4 * max(1.0, abs(want))
 
 
+@pytest.mark.parametrize("bits", [0x7FC0, 0x7F80])
+@pytest.mark.parametrize("n,row", [(48, 20), (1025, 1024)])
+def test_a_bad_feature_stays_in_its_row_of_the_gradient(hip_ctx, bits, n, row):
+    """A NaN feature, or an infinite one whose weights are negative, makes its
+    row's first layer NaN or -inf, which relu turns to 0: the row acts as one of
+    zero hidden values, and of the gradient only the bad feature's own row of
+    dW1 (NaN or infinity times 0) is NaN."""
+    import torch
+    rng = np.random.default_rng(n)
+    P, X, Xd = _case(rng, n, 0)
+    P[3 * 64:4 * 64] = -np.abs(P[3 * 64:4 * 64]) - 0.01
+    t = rng.normal(0, 1, n).astype(np.float32)
+    Xd = Xd.clone()
+    Xd[row, 3] = bits
+    grad = torch.zeros(mlp_ref.N_PARAMS, dtype=torch.float32, device="cuda:0")
+    loss = torch.zeros(1, dtype=torch.float32, device="cuda:0")
+    hip_ctx.mlp_grad(torch.from_numpy(P).to("cuda:0"), Xd, torch.from_numpy(t).to("cuda:0"), grad, loss)
+    got = grad.cpu().numpy()
+    others = np.arange(n) != row
+    want, l_ref = mlp_ref.grad(P, X[others], t[others], n_total=n)
+    P0 = P.copy()  # the row's hidden values are 0
+    P0[mlp_ref.P_W1:mlp_ref.P_B1] = 0.0
+    P0[mlp_ref.P_B1:mlp_ref.P_W2] = -1.0
+    g0, l0 = mlp_ref.grad(P0, X[:1], t[row:row + 1], n_total=n)
+    want = want + g0
+    bad = np.zeros(mlp_ref.N_PARAMS, bool)
+    bad[3 * 64:4 * 64] = True
+    assert np.array_equal(np.isnan(got), bad)
+    d = np.linalg.norm((got - want)[~bad]) / np.linalg.norm(want[~bad])
+    print(f"[bad feature] n {n}: {d:.2e}", flush=True)
+    assert d <= 2.0 ** -8
+    assert abs(float(loss.item()) - (l_ref + l0)) <= 1e-4 * (l_ref + l0)
+
+
 @pytest.mark.parametrize("shift", [0, 1, 4])
 def test_feature_rows_at_any_alignment(hip_ctx, shift):
     import torch
