@@ -2529,11 +2529,13 @@ int fg_budget_scale_device(fg_ctx *ctx, const float *d_pred_log_s, int64_t n, fl
         !(target_mse >= 0.0))
         return set_error(ctx, FG_EINVAL, "invalid budget scale arguments");
     const char *what = "budget scale";
+    std::lock_guard<std::mutex> lock(ctx->mu);
+    hipError_t e = hipSetDevice(ctx->device);
+    if (e != hipSuccess) return hip_error(ctx, e, what);
     const int rc = ensure_bytes(ctx, ctx->scale_state, fg::budget_scale_state_bytes(), what);
     if (rc != FG_OK) return rc;
-    const hipError_t e = fg::launch_budget_scale(d_pred_log_s, n, s_mult, target_mse, n_min, n_max, n_ref, 3,
-                                                 (long long)1 << 18, ctx->scale_state.p, d_scale,
-                                                 reinterpret_cast<hipStream_t>(hip_stream));
+    e = fg::launch_budget_scale(d_pred_log_s, n, s_mult, target_mse, n_min, n_max, n_ref, 3, (long long)1 << 18,
+                                ctx->scale_state.p, d_scale, reinterpret_cast<hipStream_t>(hip_stream));
     return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
 }
 
