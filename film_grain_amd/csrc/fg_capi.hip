@@ -29,6 +29,7 @@
 struct DevBuf {
     void *p = nullptr;
     size_t cap = 0;
+    bool in_graph = false;  // a graph of the caller's has its address
 };
 
 struct fg_ctx {
@@ -75,6 +76,8 @@ struct fg_ctx {
     DevBuf frame_io;          // frames from host memory: RGB in, offsets, 8-bit RGB out, planes out
     hipEvent_t scratch_done = nullptr;  // recorded after the last kernel that reads the scratch
     bool scratch_pending = false;
+    bool in_capture = false;   // the present call records into a graph of the caller's
+    std::vector<void *> kept;  // outgrown buffers that such graphs have the addresses of
     // optional kernel timing: start, generation done, test kernel start, end
     bool timing = false;
     bool timed = false;
@@ -114,11 +117,15 @@ int hip_error(fg_ctx *ctx, hipError_t e, const char *what)
     return set_error(ctx, FG_EHIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-void free_buf(DevBuf &b)
+// Gives a buffer back.  One that a graph of the caller's has recorded stays
+// until the context ends: the graph's replays still use it.
+void free_buf(fg_ctx *ctx, DevBuf &b)
 {
-    (void)hipFree(b.p);
-    b.p = nullptr;
-    b.cap = 0;
+    if (b.in_graph)
+        ctx->kept.push_back(b.p);
+    else
+        (void)hipFree(b.p);
+    b = DevBuf();
 }
 
 void free_buffers(fg_ctx *ctx)
@@ -128,34 +135,37 @@ void free_buffers(fg_ctx *ctx)
     (void)hipFree(ctx->d_out);
     ctx->d_lambda = ctx->d_offs = ctx->d_out = nullptr;
     ctx->cap_lambda = ctx->cap_offs = ctx->cap_out = 0;
-    free_buf(ctx->thresholds);
-    free_buf(ctx->bin_count);
-    free_buf(ctx->bin_start);
-    free_buf(ctx->scan_temp);
-    free_buf(ctx->grains);
-    free_buf(ctx->samples);
-    free_buf(ctx->bin_mask);
-    free_buf(ctx->plane_counts);
-    free_buf(ctx->pix_state);
-    free_buf(ctx->tiles);
-    free_buf(ctx->tile_temp);
-    free_buf(ctx->levels);
-    free_buf(ctx->frame);
-    free_buf(ctx->frame_io);
-    free_buf(ctx->cells);
-    free_buf(ctx->scale_state);
+    free_buf(ctx, ctx->thresholds);
+    free_buf(ctx, ctx->bin_count);
+    free_buf(ctx, ctx->bin_start);
+    free_buf(ctx, ctx->scan_temp);
+    free_buf(ctx, ctx->grains);
+    free_buf(ctx, ctx->samples);
+    free_buf(ctx, ctx->bin_mask);
+    free_buf(ctx, ctx->plane_counts);
+    free_buf(ctx, ctx->pix_state);
+    free_buf(ctx, ctx->tiles);
+    free_buf(ctx, ctx->tile_temp);
+    free_buf(ctx, ctx->levels);
+    free_buf(ctx, ctx->frame);
+    free_buf(ctx, ctx->frame_io);
+    free_buf(ctx, ctx->cells);
+    free_buf(ctx, ctx->scale_state);
 }
 
 int ensure_bytes(fg_ctx *ctx, DevBuf &b, size_t bytes, const char *what)
 {
-    if (b.cap >= bytes) return FG_OK;
+    if (b.cap >= bytes) {
+        b.in_graph |= ctx->in_capture;
+        return FG_OK;
+    }
     if (ctx->scratch_pending) {
         // the previous call's kernels may still read the buffer
         const hipError_t e = hipEventSynchronize(ctx->scratch_done);
         if (e != hipSuccess) return hip_error(ctx, e, what);
         ctx->scratch_pending = false;
     }
-    free_buf(b);
+    free_buf(ctx, b);
     const size_t want = std::max<size_t>(bytes + bytes / 8, 256);  // headroom for the next plane
     const hipError_t e = hipMalloc(&b.p, want);
     if (e != hipSuccess) {
@@ -165,24 +175,29 @@ int ensure_bytes(fg_ctx *ctx, DevBuf &b, size_t bytes, const char *what)
         return hip_error(ctx, e, what);
     }
     b.cap = want;
+    b.in_graph = ctx->in_capture;
     return FG_OK;
-}
-
-// The generation scratch is shared by every call on the context; a call waits
-// until the previous user's last kernel has finished before overwriting it.
-int scratch_acquire(fg_ctx *ctx, const char *what)
-{
-    if (!ctx->scratch_pending) return FG_OK;
-    const hipError_t e = hipEventSynchronize(ctx->scratch_done);
-    ctx->scratch_pending = false;
-    return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
 }
 
 // True while s records into a graph of the caller's.
 bool capturing(hipStream_t s)
 {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // s itself does not capture; the error is not the next launch's
+    return false;
+}
+
+// The generation scratch is shared by every call on the context; a call waits
+// until the previous user's last kernel has finished before overwriting it.
+// s: the call's stream (the buffers it takes are marked while s records).
+int scratch_acquire(fg_ctx *ctx, hipStream_t s, const char *what)
+{
+    ctx->in_capture = capturing(s);
+    if (!ctx->scratch_pending) return FG_OK;
+    const hipError_t e = hipEventSynchronize(ctx->scratch_done);
+    ctx->scratch_pending = false;
+    return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
 }
 
 // The same order without the host waiting: work enqueued on s from here on runs
@@ -191,8 +206,9 @@ bool capturing(hipStream_t s)
 // outside, so there the host waits.
 int scratch_acquire_on(fg_ctx *ctx, hipStream_t s, const char *what)
 {
+    ctx->in_capture = capturing(s);
     if (!ctx->scratch_pending) return FG_OK;
-    if (capturing(s)) return scratch_acquire(ctx, what);
+    if (ctx->in_capture) return scratch_acquire(ctx, s, what);
     const hipError_t e = hipStreamWaitEvent(s, ctx->scratch_done, 0);
     return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
 }
@@ -1547,7 +1563,7 @@ int frame_device(fg_ctx *ctx, const fg_frame_desc *fd, const float *d_rgb, const
     const bool joint = nr == 3 && fd->algo == FG_ALGO_PIXEL;
     const size_t bytes = (joint ? 6 : 4) * in_b + 256 + (d_planes ? 0 : (size_t)nr * out_b);
     // an earlier call's kernels may still read the scratch (on another stream)
-    int rc = scratch_acquire(ctx, what);
+    int rc = scratch_acquire(ctx, s, what);
     if (rc != FG_OK) return rc;
     if ((rc = ensure_bytes(ctx, ctx->frame, bytes, what)) != FG_OK) return rc;
     unsigned char *base = static_cast<unsigned char *>(ctx->frame.p);
@@ -1995,6 +2011,7 @@ void fg_ctx_destroy(fg_ctx *ctx)
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     free_buffers(ctx);
+    for (void *p : ctx->kept) (void)hipFree(p);
     (void)hipFree(ctx->d_status);
     (void)hipFree(ctx->d_stats);
     (void)hipFree(ctx->d_range);
@@ -2394,6 +2411,7 @@ int fg_render_frame(fg_ctx *ctx, const fg_frame_desc *fd, const float *rgb, cons
     const int nr = fd->color_mode == FG_COLOR_RGB ? 3 : 1;
     const size_t rgb_b = align256(nin * 12), offs_b = align256((size_t)d.n_samples * 8), out_b = align256(nout * 3);
     const size_t planes_b = planes ? align256((size_t)nr * nout * 4) : 0;
+    ctx->in_capture = false;  // the context's own stream
     if ((rc = ensure_bytes(ctx, ctx->frame_io, rgb_b + offs_b + out_b + planes_b, what)) != FG_OK) return rc;
     unsigned char *base = static_cast<unsigned char *>(ctx->frame_io.p);
     float *d_rgb = reinterpret_cast<float *>(base);
@@ -2432,11 +2450,11 @@ int fg_lambda_device(fg_ctx *ctx, const float *d_plane, uint32_t w, uint32_t h, 
     std::lock_guard<std::mutex> lock(ctx->mu);
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_error(ctx, e, "Lambda pre-pass");
-    int rc = scratch_acquire(ctx, "Lambda pre-pass");
+    const hipStream_t s = reinterpret_cast<hipStream_t>(hip_stream);
+    int rc = scratch_acquire(ctx, s, "Lambda pre-pass");
     if (rc != FG_OK) return rc;
     if ((rc = ensure_bytes(ctx, ctx->frame, 256, "Lambda pre-pass")) != FG_OK) return rc;
     // the max word: the first word of the frame scratch
-    const hipStream_t s = reinterpret_cast<hipStream_t>(hip_stream);
     e = fg::launch_lambda(d_plane, (long long)w * h, inv_e_pi_r2, static_cast<unsigned *>(ctx->frame.p), d_norm,
                           d_lambda, s);
     if (e != hipSuccess) return hip_error(ctx, e, "Lambda pre-pass");
@@ -2532,10 +2550,12 @@ int fg_budget_scale_device(fg_ctx *ctx, const float *d_pred_log_s, int64_t n, fl
     std::lock_guard<std::mutex> lock(ctx->mu);
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_error(ctx, e, what);
+    const hipStream_t s = reinterpret_cast<hipStream_t>(hip_stream);
+    ctx->in_capture = capturing(s);
     const int rc = ensure_bytes(ctx, ctx->scale_state, fg::budget_scale_state_bytes(), what);
     if (rc != FG_OK) return rc;
     e = fg::launch_budget_scale(d_pred_log_s, n, s_mult, target_mse, n_min, n_max, n_ref, 3, (long long)1 << 18,
-                                ctx->scale_state.p, d_scale, reinterpret_cast<hipStream_t>(hip_stream));
+                                ctx->scale_state.p, d_scale, s);
     return e == hipSuccess ? FG_OK : hip_error(ctx, e, what);
 }
 
@@ -2565,7 +2585,7 @@ int fg_pixelwise_grains(fg_ctx *ctx, const fg_plane_desc *desc, const float *d_l
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_error(ctx, e, what);
     hipStream_t s = ctx->stream;
-    if ((rc = scratch_acquire(ctx, what)) != FG_OK) return rc;
+    if ((rc = scratch_acquire(ctx, s, what)) != FG_OK) return rc;
     float4 range{};
     uint32_t seq = 0;
     e = enqueue_range(ctx, d_offsets_input_xy, (int)desc->n_samples, s, &seq);
@@ -2609,7 +2629,7 @@ int fg_grainwise_pixel_state(fg_ctx *ctx, const fg_plane_desc *desc, const float
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return hip_error(ctx, e, what);
     hipStream_t s = ctx->stream;
-    if ((rc = scratch_acquire(ctx, what)) != FG_OK) return rc;
+    if ((rc = scratch_acquire(ctx, s, what)) != FG_OK) return rc;
     const size_t npx = (size_t)desc->in_w * desc->in_h;
     if ((rc = ensure_bytes(ctx, ctx->pix_state, npx * 36 + 32, what)) != FG_OK) return rc;
     unsigned char *ps = static_cast<unsigned char *>(ctx->pix_state.p);

@@ -45,7 +45,8 @@ extern "C" {
 #define FG_OK 0
 #define FG_EINVAL 1         /* bad argument, e.g. offsets count != N (src/wgpu/mod.rs:353-358) -> Gpu(..) */
 #define FG_ENODEV 2         /* no HIP device ("no compatible GPU adapter found", src/wgpu/mod.rs:101) */
-#define FG_ENOMEM 3         /* device allocation failed (fatal; the context's buffers are dropped,
+#define FG_ENOMEM 3         /* device allocation failed (fatal; the context's buffers are dropped
+                               but for those in graphs, below;
                                src/wgpu/mod.rs:727-736) */
 #define FG_ECANCELLED 4     /* the cancel callback returned non-zero -> Cancelled */
 #define FG_EHIP 5           /* a HIP runtime call or launch failed -> Gpu(..) */
@@ -104,7 +105,18 @@ int fg_render_grainwise(fg_ctx *ctx, const fg_plane_desc *desc, const float *lam
  * for the default stream) and the call returns without waiting.  Errors found
  * on the device are reported by fg_stream_status.  No counterpart in the
  * reference (its GPU arm always copies through host memory); these are the
- * entry points for callers whose planes already live in HBM. */
+ * entry points for callers whose planes already live in HBM.
+ *
+ * Graphs.  Calls that read nothing back may be recorded into a graph of the
+ * caller's (grain-wise planes and frames, fg_lambda_device, fg_color_*, the
+ * error model's), after an eager call of the same sizes has grown the
+ * context's buffers; a pixel-wise render in the HBM formulation waits for its
+ * grain total and is refused (FG_EHIP) while its stream captures.  A recorded
+ * call works in the context's buffers, which later calls share: the context
+ * keeps every buffer that a graph has recorded until fg_ctx_destroy, also when
+ * later calls outgrow it or memory runs out, but it does not see the replays.
+ * The caller has to order each replay with every other call and replay on the
+ * context, on whatever streams they run, and with fg_ctx_destroy. */
 int fg_render_pixelwise_device(fg_ctx *ctx, const fg_plane_desc *desc, const float *d_lambda,
                                const float *d_offsets_input_xy, float *d_out, void *hip_stream);
 int fg_render_grainwise_device(fg_ctx *ctx, const fg_plane_desc *desc, const float *d_lambda,

@@ -170,3 +170,44 @@ def test_captured_grainwise_render(oracle):
         del graph
     ctx.stream_status()
     ctx.close()
+
+
+def test_graph_outlives_the_buffers_it_recorded(oracle):
+    """Grain-wise renders recorded while the context's buffers are small: later
+    calls outgrow every one of them, and the graphs, whose kernels still work in
+    the old ones, give their planes."""
+    import torch
+    jobs = _jobs(oracle)
+    want = _alone(jobs)
+    ctx = capi.Context(0)
+    recorded = []
+    for j in (1, 4):
+        algo, desc, lam, offs = jobs[j]
+        out = torch.zeros((desc.out_h, desc.out_w), device="cuda:0")
+        ctx.render_device(algo, desc, lam, offs, out)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            ctx.render_device(algo, desc, lam, offs, out, stream=torch.cuda.current_stream())
+        recorded.append((j, graph, out))
+    for size, n in ((300, 256), (700, 700)):
+        # more samples, pixels, tiles and classes than any plane before
+        c = fgcases.build_case(oracle, "large", synth.sinusoid_field(size, size - 40, size, n_waves=3), 0.25, 0.1,
+                               "lognorm", zoom=2.0, n_samples=n, seed=size)
+        lam, offs = torch.from_numpy(c.lam).to("cuda:0"), torch.from_numpy(c.offsets).to("cuda:0")
+        large = torch.empty((c.desc.out_h, c.desc.out_w), device="cuda:0")
+        ctx.render_device("grain", c.desc, lam, offs, large)
+        torch.cuda.synchronize()
+        before = large.clone()
+        for j, graph, out in recorded:
+            out.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(out.cpu().numpy(), want[j]), (size, j)
+        ctx.render_device("grain", c.desc, lam, offs, large)
+        torch.cuda.synchronize()
+        assert torch.equal(large, before)
+    del recorded
+    ctx.stream_status()
+    ctx.close()
