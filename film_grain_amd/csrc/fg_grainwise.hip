@@ -713,19 +713,15 @@ __global__ __launch_bounds__(BLOCK, grain_waves(MODE)) void grainwise_sorted(Gra
             gbx = bx;
             gby = by;
             gR = R;
-            const int rlen = listed ? 0 : len;
-            for (int it = 0; __any(it < rlen); ++it) {
-                // the cyclic run position (lanes past their run read a valid
-                // sample and queue nothing)
-                const int pr = p0 + it;
-                const int p = (int)min(min((uint32_t)pr, (uint32_t)(pr - N)), (uint32_t)(N - 1));
+            // one candidate a lane: sorted position p against the grain of
+            // lane g, target origin (ebx, eby) and output radius eR
+            auto visit = [&](bool ok, int p, int g, float ebx, float eby, float eR) {
                 const float4 r = srec[p];
-                const float txp = bx + r.x, typ = by + r.y;
+                const float txp = ebx + r.x, typ = eby + r.y;
                 float xl, xh, yl, yh;
-                bounds(txp, R, xl, xh);
-                bounds(typ, R, yl, yh);
-                const bool cand = (it < rlen) & (xl <= xh) & (yl <= yh) & (xl <= fx1) & (xh >= fx0) & (yl <= fy1) &
-                                  (yh >= fy0);
+                bounds(txp, eR, xl, xh);
+                bounds(typ, eR, yl, yh);
+                const bool cand = ok & (xl <= xh) & (yl <= yh) & (xl <= fx1) & (xh >= fx0) & (yl <= fy1) & (yh >= fy0);
                 // a candidate box of one pixel lies in the tile (it meets
                 // it); wider boxes queue their pixels inside the tile
                 const bool multi = cand & ((xh > xl) | (yh > yl));
@@ -734,10 +730,10 @@ __global__ __launch_bounds__(BLOCK, grain_waves(MODE)) void grainwise_sorted(Gra
                     // here in the lane (same f32 expression)
                     if (cand) {
                         const float dx = (xl + 0.5f) - txp, dy = (yl + 0.5f) - typ;
-                        if (dx * dx + dy * dy <= R * R) hit((int)(xl - fx0), (int)(yl - fy0), r);
+                        if (dx * dx + dy * dy <= eR * eR) hit((int)(xl - fx0), (int)(yl - fy0), r);
                     }
                 } else {
-                    const uint32_t base = (uint32_t)lane | ((uint32_t)p << 6);
+                    const uint32_t base = (uint32_t)g | ((uint32_t)p << 6);
                     const float cxl = fmaxf(xl, fx0), cxh = fminf(xh, fx1);
                     const float cyl = fmaxf(yl, fy0), cyh = fminf(yh, fy1);
                     const int tx = (int)(cxl - fx0), ty = (int)(cyl - fy0);
@@ -749,6 +745,31 @@ __global__ __launch_bounds__(BLOCK, grain_waves(MODE)) void grainwise_sorted(Gra
                         push(c, base | ((uint32_t)(tx + jx) << 17) | ((uint32_t)(ty + jy) << 24));
                     }
                 }
+            };
+            // the cyclic run position (lanes past their run read a valid
+            // sample and queue nothing)
+            auto position = [&](int pr) {
+                return (int)min(min((uint32_t)pr, (uint32_t)(pr - N)), (uint32_t)(N - 1));
+            };
+            if (LISTS) {
+                // The round's wide grains one after another, 64 samples of a
+                // grain's run a step.  In lockstep, a sample a step for every
+                // lane's grain, a few wide grains kept the wave for the
+                // longest run while the others' lanes idled, on top of the
+                // lists: 700x500 at zoom 3, N = 256, 4.6% wide grains: 25.0
+                // ms by runs alone, 30.1 with lists and lockstep, 4.7 now;
+                // 400x300 at zoom 2, N = 128, 42%: 2.77, 3.41 and 0.92; 96x64
+                // at zoom 4, N = 1024, all wide: 26.1, 26.5 and 3.2.
+                for (unsigned long long m = __ballot(!listed && len > 0); m; m &= m - 1ull) {
+                    const int g = __ffsll((long long)m) - 1;
+                    auto of_g = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), g)); };
+                    const float ubx = of_g(bx), uby = of_g(by), uR = of_g(R);
+                    const int up0 = __builtin_amdgcn_readlane(p0, g), ulen = __builtin_amdgcn_readlane(len, g);
+                    for (int i0 = 0; i0 < ulen; i0 += 64)
+                        visit(i0 + lane < ulen, position(up0 + i0 + lane), g, ubx, uby, uR);
+                }
+            } else {
+                for (int it = 0; __any(it < len); ++it) visit(it < len, position(p0 + it), lane, bx, by, R);
             }
             // the queue refers to the lanes' current grains
             if (qcount > 0) {

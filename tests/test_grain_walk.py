@@ -131,3 +131,26 @@ def test_counts_of_every_pixel(hip_ctx, oracle, w, h, r, sd):
     want = oracle.render_grainwise(c.plane, c.lam, c.offsets)
     got = hip_ctx.render_host("grain", c.desc, c.lam, c.offsets)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 16, 63, 64, 65, 127, 129, 1000, 2048])
+@pytest.mark.parametrize("r,sd,zoom", [(0.25, 0.1, 2.0),   # narrow and wide grains in one round
+                                       (0.15, 0.07, 2.0),  # a few wide ones
+                                       (0.45, 0.1, 3.0)])  # all wide, boxes of several pixels
+def test_wide_grains_among_narrow_ones(hip_ctx, oracle, n, r, sd, zoom):
+    """Lognormal radii on both sides of half an output pixel: the narrow grains
+    walk lists, each wide one its run of the sample order, 64 samples a step:
+    whole and broken steps, and runs past the end of the order."""
+    from film_grain_amd import synth
+    from tests import fgcases
+    c = fgcases.build_case(oracle, "wide", synth.sinusoid_field(13, 11, n, n_waves=3), r, sd, "lognorm", zoom=zoom,
+                           n_samples=n, seed=n + 7)
+    want = oracle.render_grainwise(c.plane, c.lam, c.offsets)
+    for block in (512, 256):
+        hip_ctx.set_launch_config(grain_variant=2, grain_block=block)
+        try:
+            got = hip_ctx.render_host("grain", c.desc, c.lam, c.offsets)
+        finally:
+            hip_ctx.reset_launch_config()
+        assert np.array_equal(got, want), block
