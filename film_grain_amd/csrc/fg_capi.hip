@@ -1359,9 +1359,10 @@ int do_grainwise(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lambda, con
             const int cq = lognorm ? fg::kGrainClassQ : fg::kGrainConstQ;
             const int classes =
                 lognorm ? std::max(1, std::min(cq, (int)std::ceil(std::min(a.r_out_max, 0.5f) * 2.0f * cq))) : 1;
+            const int ce = lognorm ? fg::kGrainClassE : cq;
             const size_t cells = (size_t)classes * cq * cq;
-            if ((rc = ensure_bytes(ctx, ctx->cells, 256 + cells * sizeof(uint2) + cells * a.n_samples * 2 + 256, what)) !=
-                FG_OK)
+            const size_t entries = fg::splat_lists_entries(cq, classes, ce, a.n_samples);
+            if ((rc = ensure_bytes(ctx, ctx->cells, 256 + cells * sizeof(uint2) + entries * 2 + 256, what)) != FG_OK)
                 return rc;
             unsigned char *cb = static_cast<unsigned char *>(ctx->cells.p);
             uint2 *cell = reinterpret_cast<uint2 *>(cb + 256);
@@ -1371,8 +1372,8 @@ int do_grainwise(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lambda, con
             set.classes = classes;
             if (e == hipSuccess) e = fg::launch_sample_levels(set, s);
             if (e == hipSuccess)
-                e = fg::launch_grain_lists(st, cq, classes, lognorm ? 0.0f : r_out, c_base, set.fill[0], cell, list,
-                                           a.status, s);
+                e = fg::launch_grain_lists(st, cq, classes, ce, lognorm ? 0.0f : r_out, c_base, set.fill[0], cell,
+                                           list, a.status, s);
             a.gl_cell = cell;
             a.gl_list = list;
             a.gl_classes = classes;

@@ -497,7 +497,8 @@ __global__ __launch_bounds__(BLOCK, grain_waves(MODE)) void grainwise_sorted(Gra
                                                          fmaxf(fabsf(ext.z), fabsf(ext.w))) + Rmax + 8.0f;
     const float eps = uniform_f(C * 9.5367431640625e-07f + 1.52587890625e-05f);  // C * 2^-20 + 2^-16
     // a grain below this radius covers pixels nearest its target alone
-    const float narrow_r = uniform_f(0.5f - (eps + eps));
+    // (0 where a lognormal law has no lists: their room is for a bounded eps)
+    const float narrow_r = uniform_f(MODE == kLognormal && !(eps <= kGrainWalkEps) ? 0.0f : 0.5f - (eps + eps));
     // within this of the radius a passing pixel's bounds() box is looked at
     const float edge = uniform_f(C * 4.76837158203125e-07f);  // C * 2^-21
     const float Qf = uniform_f((float)Q);

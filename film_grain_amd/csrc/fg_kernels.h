@@ -70,6 +70,14 @@ struct PixelArgs {
 
 // Cells per side of the grain-wise candidate lists.
 constexpr int kGrainConstQ = 64, kGrainClassQ = 32;
+// Room of the lognormal lists: for windows widened by at most kGrainClassE
+// cells in all, (2 eps + 2^-11) kGrainClassQ <= kGrainClassE, which holds up to
+// eps = 0.06225 (coordinates of 65000 output pixels and more).  Lists are built
+// up to kGrainBuildEps and walked up to kGrainWalkEps, below it by more than
+// the two kernels' roundings of eps can differ; beyond, grains walk their runs.
+// (Room for every sample in every cell took 134 MB at N = 2048, this 76 MB.)
+constexpr int kGrainClassE = 4;
+constexpr float kGrainBuildEps = 0.0622f, kGrainWalkEps = 0.062f;
 
 // Grain-wise integrator launch (src/grainwise.rs:12-124).
 struct GrainArgs {

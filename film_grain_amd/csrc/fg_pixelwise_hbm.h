@@ -141,11 +141,11 @@ hipError_t launch_grainwise_sorted(const GrainArgs &a, const SampleTable &st, in
 // Candidate lists of the sorted grain-wise kernel: for r_const > 0 one class of
 // that output radius, else `classes` classes of radius (k + 1) / (2 q); q x q
 // cells each.  cell: classes * q * q (start, length) pairs; list: room for
-// classes * q * q * n positions; fill: classes counters (cleared by the caller).
-// c_base = max(out_w, out_h) + the largest output radius + 8 (the kernel's
+// splat_lists_entries(q, classes, e, n) positions, e = q with r_const and
+// kGrainClassE without; fill: classes counters (cleared by the caller).  c_base = max(out_w, out_h) + the largest output radius + 8 (the kernel's
 // widening bound without the offsets).  Needs st.n <= 2048.
-hipError_t launch_grain_lists(const SampleTable &st, int q, int classes, float r_const, float c_base, uint32_t *fill,
-                              uint2 *cell, uint16_t *list, int *status, hipStream_t s);
+hipError_t launch_grain_lists(const SampleTable &st, int q, int classes, int e, float r_const, float c_base,
+                              uint32_t *fill, uint2 *cell, uint16_t *list, int *status, hipStream_t s);
 
 // Heaviest-first tile order: w[t] = the work of tile t (grains of the bins
 // covering its region), ids[t] = t; sort_tiles orders ids by w, descending

@@ -950,22 +950,22 @@ __global__ __launch_bounds__(256) void splat_lists_kernel(LevelSet set, int q, i
 // X + 1/2 with b = bx - 1/2, its bounds() box of the splat's form around b + X,
 // so the same windows around frac(-b) hold its samples; eps is that kernel's:
 // C * 2^-20 + 2^-16, which covers the box's five roundings of at most C * 2^-24.
-__global__ __launch_bounds__(256) void grain_lists_kernel(SampleTable st, int q, float r_const, float c_base,
+__global__ __launch_bounds__(256) void grain_lists_kernel(SampleTable st, int q, int e, float r_const, float c_base,
                                                           uint32_t *fill, uint2 *cell, uint16_t *list, int *status)
 {
     __shared__ ListsShared sh;
     const float4 ext = *st.ext;
     const float C = c_base + fmaxf(fmaxf(fabsf(ext.x), fabsf(ext.y)), fmaxf(fabsf(ext.z), fabsf(ext.w)));
     const float eps = C * 9.5367431640625e-07f + 1.52587890625e-05f;
-    // room for every sample in every cell: span q
-    splat_lists_body(st, q, q, eps, r_const, fill, cell, nullptr, list, status, blockIdx.x, sh);
+    if (r_const <= 0.0f && !(eps <= kGrainBuildEps)) return;  // not walked either (kGrainWalkEps)
+    splat_lists_body(st, q, e, eps, r_const, fill, cell, nullptr, list, status, blockIdx.x, sh);
 }
 
-hipError_t launch_grain_lists(const SampleTable &st, int q, int classes, float r_const, float c_base, uint32_t *fill,
-                              uint2 *cell, uint16_t *list, int *status, hipStream_t s)
+hipError_t launch_grain_lists(const SampleTable &st, int q, int classes, int e, float r_const, float c_base,
+                              uint32_t *fill, uint2 *cell, uint16_t *list, int *status, hipStream_t s)
 {
     if (q < 1 || q * q > 65536 || classes < 1 || st.n > 2048) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(grain_lists_kernel, dim3(classes * ((q * q + 63) / 64)), dim3(256), 0, s, st, q, r_const, c_base,
+    hipLaunchKernelGGL(grain_lists_kernel, dim3(classes * ((q * q + 63) / 64)), dim3(256), 0, s, st, q, e, r_const, c_base,
                        fill, cell, list, status);
     return hipGetLastError();
 }

@@ -154,3 +154,33 @@ def test_wide_grains_among_narrow_ones(hip_ctx, oracle, n, r, sd, zoom):
         finally:
             hip_ctx.reset_launch_config()
         assert np.array_equal(got, want), block
+
+
+def test_room_of_the_class_lists():
+    """No class of the lognormal lists holds more entries than its room,
+    N min(q, k + 4 + e)^2, up to the widest eps that lists are built for."""
+    q, e, N = 32, 4, 96
+    assert (2 * 0.0622 + 2.0 ** -11) * q <= e
+    rng = np.random.default_rng(3)
+    for fx, fy in (rng.random((2, N)).astype(f32), (rng.integers(0, q, (2, N)) / q).astype(f32)):
+        for eps in (f32(2.0 ** -16), f32(0.0622)):
+            for k in range(q):
+                R = f32(f32(k + 1) / f32(2 * q))
+                n = sum(int(members(fx, fy, qa, qb, q, R, eps).sum()) for qa in range(q) for qb in range(q))
+                assert n <= N * min(q, k + 4 + e) ** 2, (k, float(eps))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("far", [0.0, 30000.0, 64000.0, 65100.0, 70000.0, 300000.0])
+def test_far_offsets(hip_ctx, oracle, far):
+    """One sample's offset far outside the plane: the lists' widening grows to
+    its limit (about 65000) and the grains walk their runs beyond."""
+    from film_grain_amd import synth
+    from tests import fgcases
+    c = fgcases.build_case(oracle, "far", synth.sinusoid_field(24, 17, 3, n_waves=3), 0.1, 0.04, "lognorm", zoom=2.0,
+                           n_samples=70, seed=12)
+    offs = np.ascontiguousarray(c.offsets).copy()
+    offs[5, 0] += np.float32(far)
+    offs[6, 1] -= np.float32(far)
+    want = oracle.render_grainwise(c.plane, c.lam, offs)
+    assert np.array_equal(hip_ctx.render_host("grain", c.desc, c.lam, offs), want)
