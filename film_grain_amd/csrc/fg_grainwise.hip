@@ -420,8 +420,10 @@ constexpr int kGrainWaveWords = 256;
 static_assert(kGrainWaveWords >= kQueueCap, "the queue shares the records' room");
 
 // Waves per SIMD each mode's registers are held to (lognormal draws need f64
-// transcendentals; at eight waves they spilled 25 registers).
-constexpr int grain_waves(int mode) { return mode == kLognormal ? 5 : 8; }
+// transcendentals: at eight waves they spilled 25 registers; a CU holds two
+// workgroups of 512 at four waves and at five, 1021x767 at zoom 2, r = 0.1 /
+// 0.03, N = 128: 1.50 ms held to five, 1.40 to four).
+constexpr int grain_waves(int mode) { return mode == kLognormal ? 4 : 8; }
 
 // Per output tile: rounds of one grain per lane, each drawn from its input
 // pixel's stream and its samples found through its list or run.
