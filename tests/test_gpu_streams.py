@@ -126,8 +126,8 @@ def test_call_after_a_refused_one(oracle):
     (200, 200, 0.1, None),     # either side of 16384 bins: one workgroup, three launches
     (212, 212, 0.1, None),
     (64, 48, 0.1, 0.0),        # no grain at all
-    (2200, 2000, 1.0, 0.02),   # more than 2048 tiles: weights in their own launch
-    (3000, 2900, 1.0, 0.02),   # more than 8192: ordered by the radix sort
+    (2200, 2000, 1.0, 0.02),   # 8625 tiles and more: ordered by the radix sort
+    (3000, 2900, 1.0, 0.02),
 ])
 def test_bin_starts_and_tile_order(oracle, w, h, radius, grey):
     plane = (np.full((h, w), grey, dtype=np.float32) if grey is not None
@@ -138,6 +138,29 @@ def test_bin_starts_and_tile_order(oracle, w, h, radius, grey):
     got = ctx.render_host("pixel", c.desc, c.lam, c.offsets_input)
     ctx.close()
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("tiles,w,h", [
+    (2048, 1024, 1024),  # the most that one launch weighs and orders
+    (2080, 1024, 1033),  # weights in their own launch, then the counting sort
+    (8192, 2048, 2048),  # the most that it orders
+    (8256, 2048, 2049),  # ordered by the radix sort
+])
+@pytest.mark.parametrize("algo", ["pixel", "grain"])
+def test_tile_order(oracle, algo, tiles, w, h):
+    """Planes at the limits of the tile orders: every tile is in the order."""
+    c = fgcases.build_case(oracle, "order", np.full((h, w), 0.02, dtype=np.float32), 1.0, 0.0, "const", zoom=1.0,
+                           n_samples=4, seed=w + h)
+    ctx = capi.Context(0)
+    ctx.set_launch_config(pix_tile_w=32, pix_tile_h=16, grain_tile_w=32, grain_tile_h=16)
+    cfg = ctx.launch_config(c.desc, algo)
+    tw, th = (cfg[f"{'pix' if algo == 'pixel' else 'grain'}_tile_{s}"] for s in "wh")
+    assert -(-w // tw) * -(-h // th) == tiles
+    offs = c.offsets_input if algo == "pixel" else c.offsets
+    got = ctx.render_host(algo, c.desc, c.lam, offs)
+    ctx.close()
+    render = oracle.render_pixelwise if algo == "pixel" else oracle.render_grainwise
+    assert np.array_equal(got, render(c.plane, c.lam, offs))
 
 
 def test_captured_grainwise_render(oracle):
