@@ -222,7 +222,7 @@ __device__ __noinline__ uint32_t rejection_count(Xoshiro rng, double lambda)
 // once per cell and kept in an LDS record for the nonempty ones, and each
 // plane's count of a cell runs on the one uniform sequence against its own
 // threshold.  A bin of 2^32 or more grains saturates its count and sets
-// kStatusOverflow (the plane's 64-bit sum of the bin counts, sum_bins_u64,
+// kStatusOverflow (the plane's 64-bit total of the bin counts, launch_bin_scan,
 // then reaches 2^32 - 1 as well, and the host refuses the plane before any
 // kernel uses the u32 scan).
 // A nonempty cell's record in the count pass: its hash and seed words s0

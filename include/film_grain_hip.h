@@ -144,8 +144,9 @@ int fg_render_pixelwise_planes_device(fg_ctx *ctx, const fg_plane_desc *desc, in
  * device's array, across contexts: calls that overlap on one device race
  * (serialise them, e.g. on one stream with no other caller).  The array
  * keeps the last call's contents; the path clears what must start at zero.
- * Like the other device entry points it synchronises once with the stream
- * after its counting pass. */
+ * Like the other pixel-wise device entry points it waits for two values that
+ * its kernels publish, the offsets' range and, after its counting pass, the
+ * plane's grain total; the draws and the splat run after it has returned. */
 #define FG_NOALLOC_SCRATCH_BYTES (256u << 20)
 int fg_render_pixelwise_device_noalloc(fg_ctx *ctx, const fg_plane_desc *desc, const float *d_lambda,
                                        const float *d_offsets_input_xy, float *d_out, void *hip_stream);

@@ -74,9 +74,10 @@ def test_run_contains_every_candidate(N, z, sd):
 
 
 def cell_members(fx, fy, qa, qb, Q, R, eps):
-    """Membership of samples (fractions fx, fy) in the candidate list of
-    cell (qa, qb), in the f32 operation order of cell_lists_kernel in
-    fg_grainwise.hip."""
+    """Membership of samples (fractions fx, fy) in the window of cell
+    (qa, qb), both box sides of the cell's targets in f32: a square with
+    its corners.  (The lists keep those within the radius of the cell's own
+    square, corners rounded: tests/test_grain_walk.py.)"""
     m = f32(2.0 ** -12)
     w = f32(f32(f32(R + R) + f32(eps + eps)) + f32(f32(1) / f32(Q) + f32(m + m)))
     lx = f32(f32(f32(qa) / f32(Q) - f32(R + R)) - f32(eps + m))
@@ -91,9 +92,9 @@ def cell_members(fx, fy, qa, qb, Q, R, eps):
 @pytest.mark.parametrize("Q", [32, 64])
 @pytest.mark.parametrize("N,R,sd", [(1, 0.05, 0.8), (128, 0.05, 0.8), (513, 0.159, 1.5), (2048, 0.01, 0.4)])
 def test_cell_list_contains_every_candidate(N, R, sd, Q):
-    """The grain-wise kernel's per-cell candidate lists (constant radius):
-    every sample whose f32 bounds() box (src/grainwise.rs:126-142) has both
-    a column and a row is in the list of the cell of the grain's target
+    """The windows that the grain-wise candidate lists are cut from: every
+    sample whose f32 bounds() box (src/grainwise.rs:126-142) has both a
+    column and a row is in the window of the cell of the grain's target
     fractions (A, B), for grain centres anywhere in a 4096-pixel plane and
     at half-integers +- 1e-4."""
     rng = np.random.default_rng(N)
