@@ -233,6 +233,15 @@ hipError_t wait_published(const uint32_t *flag, uint32_t seq, hipStream_t s)
     return there() ? hipSuccess : hipErrorUnknown;
 }
 
+// Work that is only recorded publishes nothing that the host could wait for: a
+// call that waits is refused before it enqueues anything, and the caller's
+// capture stays valid (the wait for the stream would invalidate it).
+int refuse_capture(fg_ctx *ctx, const char *what)
+{
+    return set_error(ctx, FG_EHIP,
+                     std::string(what) + ": waits for its grain total and cannot be recorded into a graph");
+}
+
 // The offsets' range of a pixel-wise render: computed on s, published to the
 // host.  read_range waits for it.
 hipError_t enqueue_range(fg_ctx *ctx, const float *d_offs, int n, hipStream_t s, uint32_t *seq)
@@ -1025,6 +1034,7 @@ int do_pixelwise_budget(fg_ctx *ctx, const fg_plane_desc *d, const float *d_lamb
     // the context's buffers are shared by its calls
     int rc0 = scratch_acquire_on(ctx, s, what);
     if (rc0 != FG_OK) return rc0;
+    if (variant == 3 && ctx->in_capture) return refuse_capture(ctx, what);
     ScratchGuard guard{ctx, s};
     hipError_t e = enqueue_range(ctx, d_offs, (int)d->n_samples, s, &seq);
     if (e != hipSuccess) return hip_error(ctx, e, what);
@@ -1097,6 +1107,7 @@ int do_pixelwise_planes(fg_ctx *ctx, const fg_plane_desc *d, int n, const float 
     if (joint) {
         // the previous call's kernels may still read the context's buffers
         if ((rc = scratch_acquire_on(ctx, s, what)) != FG_OK) return rc;
+        if (ctx->in_capture) return refuse_capture(ctx, what);
         guard.armed = true;
         uint32_t seq = 0;
         hipError_t e = enqueue_range(ctx, d_offs, (int)d->n_samples, s, &seq);
@@ -2093,6 +2104,7 @@ int fg_render_pixelwise_device_noalloc(fg_ctx *ctx, const fg_plane_desc *desc, c
     if (e != hipSuccess) return hip_error(ctx, e, what);
     if (!ctx->noalloc_scratch) return set_error(ctx, FG_EHIP, std::string(what) + ": no scratch address");
     hipStream_t s = reinterpret_cast<hipStream_t>(hip_stream);
+    if (capturing(s)) return refuse_capture(ctx, what);
     ScratchSource src;
     src.arena = ctx->noalloc_scratch;
     src.cap = kNoAllocScratchBytes;

@@ -234,3 +234,42 @@ def test_graph_outlives_the_buffers_it_recorded(oracle):
     del recorded
     ctx.stream_status()
     ctx.close()
+
+
+def test_captured_pixelwise_render_is_refused(oracle):
+    """A pixel-wise render waits for its grain total: while its stream captures
+    it is refused before it enqueues anything, and the capture goes on."""
+    import torch
+    jobs = _jobs(oracle)
+    want = _alone(jobs)
+    ctx = capi.Context(0)
+    algo, desc, lam, offs = jobs[0]
+    out = torch.zeros((desc.out_h, desc.out_w), device="cuda:0")
+    ctx.render_device(algo, desc, lam, offs, out)
+    torch.cuda.synchronize()
+    x = torch.zeros(8, device="cuda:0")
+    graph = torch.cuda.CUDAGraph()
+    refused = []
+    with torch.cuda.graph(graph):
+        s = torch.cuda.current_stream()
+        for call in (lambda: ctx.render_device(algo, desc, lam, offs, out, stream=s),
+                     lambda: ctx.render_planes_device(desc, [lam, lam], offs, [out, out], stream=s),
+                     lambda: ctx.render_device_noalloc(desc, lam, offs, out, stream=s)):
+            try:
+                call()
+            except capi.FilmGrainError as err:
+                refused.append(err.code)
+        x += 1
+    assert refused == [capi.FG_EHIP] * 3
+    out.zero_()
+    for k in (1, 2):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.all(x == k) and torch.all(out == 0)
+    for j in (0, 1):
+        a, d, l, o = jobs[j]
+        out = torch.zeros((d.out_h, d.out_w), device="cuda:0")
+        ctx.render_device(a, d, l, o, out)
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), want[j])
+    ctx.close()
