@@ -431,7 +431,7 @@ constexpr int grain_waves(int mode) { return mode == kLognormal ? 4 : 8; }
 // holds the pixel) and about 28 VALU per list entry.  Before lognormal laws
 // had lists their lanes walked runs in lockstep, every candidate by its box
 // and the queue: 1021x767 at zoom 2, r = 0.1 / 0.03, N = 128 took 7.1 ms and
-// takes 1.6; a 1280x720 plane, r = 0.1 / 0.05, N = 64, 2.69 and 0.73.  The
+// takes 1.3; a 1280x720 plane, r = 0.1 / 0.05, N = 64, 2.69 and 0.71.  The
 // constant-radius plane of 4096x4096 (r = 0.05, N = 128; owners from a byte
 // map, boxes evaluated for every entry, 64x32 tiles): 16.7 and 14.6 ms.
 template <int MODE, int BLOCK>
@@ -760,9 +760,9 @@ __global__ __launch_bounds__(BLOCK, grain_waves(MODE)) void grainwise_sorted(Gra
                 // lane's grain, a few wide grains kept the wave for the
                 // longest run while the others' lanes idled, on top of the
                 // lists: 700x500 at zoom 3, N = 256, 4.6% wide grains: 25.0
-                // ms by runs alone, 30.1 with lists and lockstep, 4.7 now;
-                // 400x300 at zoom 2, N = 128, 42%: 2.77, 3.41 and 0.92; 96x64
-                // at zoom 4, N = 1024, all wide: 26.1, 26.5 and 3.2.
+                // ms by runs alone, 30.1 with lists and lockstep, 4.4 now;
+                // 400x300 at zoom 2, N = 128, 46%: 2.77, 3.41 and 0.90; 96x64
+                // at zoom 4, N = 1024, all wide: 26.1, 26.5 and 3.1.
                 for (unsigned long long m = __ballot(!listed && len > 0); m; m &= m - 1ull) {
                     const int g = __ffsll((long long)m) - 1;
                     auto of_g = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), g)); };
